@@ -9,7 +9,11 @@
 // y = p - kappa w. The reflector of hop h of sweep s occupies rows
 // [s+1+hb, min(s+(h+1)b, n-1)] and is stored for the back-transform.
 //
-// Our design (not the reference's):
+// Two kernels: the resident form (bc_chase_resident_kernel, described there) wherever its
+// workgroups, one per hop of the first sweep, fit on the GPU at once, and the windowed
+// form below for the larger n (b = 64 in FP64: n > 32768), where it still is the only one.
+//
+// Design of the windowed form (not the reference's):
 //  * Reflector convention: if the vector below the pivot is exactly zero the
 //    hop is the identity (w = 0), as LAPACK's dlarfg does; the reference's
 //    normalised reflector would flip the sign of the pivot instead.
@@ -500,6 +504,390 @@ __global__ __launch_bounds__(kBCThreads) void bc_chase_kernel(T *Bp, T *U, i64 l
     }
 }
 
+// ---------------------------------------------------------------------------
+// Resident form: the band stays in registers, only reflectors and rows travel.
+//
+// Workgroup h runs hop h of every sweep and holds the two b x b blocks that hop works
+// on for the whole chase: D = A[r0..r1, r0..r1] (full square) and L = A[r0..r1,
+// r0-b..r0-1], r0 = s + 1 + h b, r1 = r0 + b - 1 (h = 0: of L only column r0 - 1). Row i
+// and column j sit in slots i mod b and j mod b, so when the sweep number advances by
+// one nothing moves: row and column r0 leave their slot and row and column r1 + 1 = r0 +
+// b enter the same one. Thread = (row slot, group of CPT column slots), B lanes per row
+// vector, the CPT elements of each block in registers.
+//
+// Per sweep, workgroup h
+//   1. receives w' = w_{h-1}(s) from its left neighbour and the value beta that its
+//      right neighbour left in column r0 - 1 in sweep s - 1; the column r0 - 1 of D becomes
+//      a column of L, a zero row with beta in it enters L;
+//   2. y = 2 L w', x = column r0 - b of L - y w'^T, the reflector w and beta of x (every
+//      wave forms it from the same sums, so it is not sent through LDS), w to the right,
+//      beta to the left;
+//   3. L -= y w'^T, L -= w (2 w^T L); its row r0 goes to the left neighbour;
+//   4. receives row r1 of sweep s - 1 from the right (new last row and column of D);
+//      p = 2 D w, D -= w y^T + y w^T with y = p - (w^T p) w; D(r0, r0) goes to the left.
+// Workgroup 0 writes (d, e). Rows and columns from n on are zeros, which need no special
+// cases: a one-row hop finds a zero tail and makes the identity.
+//
+// A message word is 64 bits: 32 bits of payload and the sweep number + 1 as a tag, so the
+// receiver polls the data itself and one store-to-load latency covers the hand-off (a
+// flag behind the data costs a second one). Buffers are double: sweep s + 2 overwrites
+// sweep s's words only after an answer that was computed from them came back.
+//
+// Bound: the sweep-to-sweep lag, two hand-offs (w to the right, beta to the left; about
+// 1 us each) and two times steps 1-2. Measured alone, FP64: 3.9 us per sweep at b = 64 and
+// 3.2 at b = 32, against 16.4 and 9.1 for the windowed kernel, which moves 2 b columns
+// through memory per hop and pays two dependent global round trips per hop (n = 16384:
+// 276 -> 64 ms; n = 4096: 67 -> 16 ms; n = 1024, b = 32: 9.3 -> 3.3 ms). Beside Q_s^T's
+// products it shares every CU with them (n = 16384: 119 ms, and 183 ms for the products).
+// Neighbouring workgroups on one XCD gained nothing (3.9 us) and lost beside the products
+// (147 ms), a sleep between polls 0.1 us; three workgroups per CU (84 VGPRs) cost 1 us.
+// ---------------------------------------------------------------------------
+using u64 = unsigned long long;
+
+template <typename T> struct MsgWord;
+template <> struct MsgWord<double> {
+    static constexpr int N = 2; // words per value
+    __device__ static void put(u64 *p, double v, unsigned tag) {
+        const u64 b = (u64)__double_as_longlong(v), t = (u64)tag << 32;
+        st_agent(p, (b & 0xffffffffull) | t);
+        st_agent(p + 1, (b >> 32) | t);
+    }
+    __device__ static bool get(const u64 *p, double &v, unsigned tag) {
+        const u64 a = ld_agent(p), b = ld_agent(p + 1);
+        v = __longlong_as_double((long long)((a & 0xffffffffull) | (b << 32)));
+        return (unsigned)(a >> 32) == tag && (unsigned)(b >> 32) == tag;
+    }
+};
+template <> struct MsgWord<float> {
+    static constexpr int N = 1;
+    __device__ static void put(u64 *p, float v, unsigned tag) {
+        st_agent(p, (u64)__float_as_uint(v) | ((u64)tag << 32));
+    }
+    __device__ static bool get(const u64 *p, float &v, unsigned tag) {
+        const u64 a = ld_agent(p);
+        v = __uint_as_float((unsigned)a);
+        return (unsigned)(a >> 32) == tag;
+    }
+};
+
+// Message buffers of the link between workgroups h - 1 and h, one set per parity of s:
+// w (h - 1 -> h, b values), row (h -> h - 1, b values), beta (h -> h - 1, one value on a
+// line of its own).
+constexpr int kBetaPad = 16; // values
+template <typename T> __host__ __device__ constexpr i64 msg_words(int b) { return (2 * b + kBetaPad) * (i64)(sizeof(T) / 4); }
+
+// --- lane exchanges within a wave (DPP and permlane swaps: no LDS round trip)
+template <int CTRL> __device__ __forceinline__ float dpp_mov(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_mov(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kHalfMirror = 0x141, kRowRor8 = 0x128;
+// upper half of a <-> lower half of b, of the 64 lanes (32) or of each 32 lanes (16)
+template <int W> __device__ __forceinline__ void lane_swap(unsigned &a, unsigned &b) {
+    if constexpr (W == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    }
+}
+template <int W> __device__ __forceinline__ void lane_swap(float &a, float &b) {
+    unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+    lane_swap<W>(x, y);
+    a = __uint_as_float(x);
+    b = __uint_as_float(y);
+}
+template <int W> __device__ __forceinline__ void lane_swap(double &a, double &b) {
+    unsigned xl = (unsigned)__double2loint(a), xh = (unsigned)__double2hiint(a);
+    unsigned yl = (unsigned)__double2loint(b), yh = (unsigned)__double2hiint(b);
+    lane_swap<W>(xl, yl);
+    lane_swap<W>(xh, yh);
+    a = __hiloint2double((int)xh, (int)xl);
+    b = __hiloint2double((int)yh, (int)yl);
+}
+// sums over groups of 8 lanes, of B lanes: every lane gets its group's total
+template <typename V> __device__ __forceinline__ V sum8(V v) {
+    v += dpp_mov<kQuadXor1>(v);
+    v += dpp_mov<kQuadXor2>(v);
+    v += dpp_mov<kHalfMirror>(v);
+    return v;
+}
+template <int B, typename V> __device__ __forceinline__ V group_sum(V v) {
+    v = sum8(v);
+    v += dpp_mov<kRowRor8>(v);
+    if constexpr (B >= 32) {
+        V a = v, b = v;
+        lane_swap<16>(a, b);
+        v = a + b;
+    }
+    if constexpr (B >= 64) {
+        V a = v, b = v;
+        lane_swap<32>(a, b);
+        v = a + b;
+    }
+    return v;
+}
+__device__ __forceinline__ float read_lane(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double read_lane(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// v of row slot idx0 + j of the lane's column group: lane slots repeat every B lanes, so
+// lanes 0..B-1 hold them all. `first`: the first column slot of the wave (uniform).
+template <int B, int CPT, typename V>
+__device__ __forceinline__ V slot_value(V v, int first, int j, int lane) {
+    if constexpr (B == 64) return read_lane(v, first + j);
+    else if constexpr (B == 32) {
+        const V a = read_lane(v, first + j), b = read_lane(v, first + CPT + j);
+        return lane < 32 ? a : b;
+    } else return __shfl(v, first + CPT * (lane / B) + j, 64);
+}
+// totals over the B lanes of a group of CPT values per lane, all in every lane: halving
+// exchanges (each lane keeps half of the columns) instead of CPT butterflies
+template <int B, int CPT, typename V> __device__ __forceinline__ void column_sums(V (&v)[CPT], int lane) {
+    if constexpr (B == 16) {
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) v[j] = group_sum<16>(v[j]);
+    } else {
+        static_assert(CPT == B / 8, "eight lanes per column in the last step");
+        V t[4];
+        if constexpr (B == 64) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                V a = v[i], b = v[i + 4];
+                lane_swap<32>(a, b);
+                t[i] = a + b;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[i] = v[i];
+        }
+        V r[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            V a = t[i], b = t[i + 2];
+            lane_swap<16>(a, b);
+            r[i] = a + b;
+        }
+        const bool odd = (lane & 8) != 0;
+        const V keep = odd ? r[1] : r[0], give = odd ? r[0] : r[1];
+        const V q = sum8(keep + dpp_mov<kRowRor8>(give)); // column j of the group in its lanes 8 j ..
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) {
+            if constexpr (B == 64) v[j] = read_lane(q, 8 * j);
+            else {
+                const V a = read_lane(q, 8 * j), b = read_lane(q, 32 + 8 * j);
+                v[j] = lane < 32 ? a : b;
+            }
+        }
+    }
+}
+
+constexpr int chase_threads(int b) { return b == 64 ? 512 : 256; }
+
+template <typename T, int B>
+__global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(const T *Bp, T *U, i64 ldu, int n, T *dd,
+                                                                             T *ee, u64 *msg, int *err) {
+    constexpr int NT = chase_threads(B);
+    constexpr int NG = NT / B;   // column groups
+    constexpr int CPT = B / NG;  // columns per thread
+    constexpr int SPW = CPT * (64 / B); // column slots per wave
+    constexpr int NWD = MsgWord<T>::N;
+    constexpr int M = B - 1;
+    const int ldb = 2 * B;
+    __shared__ T s_wp[B], s_x[B], s_row[B], s_lrow[B];
+    __shared__ T s_part[NG][B], s_part2[NG][B];
+    __shared__ T s_beta;
+    __shared__ int s_go;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lam = tid & M, cg = tid / B;
+    const int c0 = cg * CPT;       // this thread's first column slot
+    const int cw = wave * SPW;     // this wave's first column slot
+    const int h = blockIdx.x;
+    // the chase is a chain of short latency-bound steps; products running beside it are not
+    __builtin_amdgcn_s_setprio(3);
+
+    const i64 mw = msg_words<T>(B);
+    u64 *left = msg + (i64)h * 2 * mw, *right = left + 2 * mw; // links to h - 1 and h + 1
+    constexpr int oRow = B * NWD, oBeta = 2 * B * NWD;
+
+    T L[CPT], D[CPT];
+    {
+        const int r0 = 1 + h * B;
+        const int gi = r0 + ((lam - r0) & M);
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) {
+            const int gc = r0 + ((c0 + j - r0) & M);
+            const int hi = max(gi, gc), lo = min(gi, gc);
+            D[j] = hi < n ? Bp[(hi - lo) + (i64)lo * ldb] : T(0);
+            const int gl = gc - B, diff = gi - gl;
+            L[j] = (gi < n && gl >= 0 && diff <= B) ? Bp[diff + (i64)gl * ldb] : T(0);
+        }
+    }
+    if (tid == 0) {
+        s_go = 1;
+        if (h == 0) {
+            dd[0] = Bp[0];
+            ee[n - 1] = T(0);
+        }
+    }
+    __syncthreads();
+
+    // one value per lane from p + lane * NWD, for the lanes that want one; false: the wait expired
+    auto poll = [&](const u64 *p, bool want, unsigned tag, T &v) -> bool {
+        bool ok = !want;
+        for (long long it = 0;; ++it) {
+            if (!ok) ok = MsgWord<T>::get(p + lane * NWD, v, tag);
+            if (__all(ok)) return true;
+            if (it > kSpinLimit) {
+                if (lane == 0)
+                    __hip_atomic_store(err, (int)DEV_WATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return false;
+            }
+        }
+    };
+
+    for (int s = 0;; ++s) {
+        const int r0 = s + 1 + h * B;
+        if (r0 > n - 1) break;
+        const int kap = r0 & M, kold = (r0 - 1) & M;
+        const bool right_row = s > 0 && r0 + B - 1 <= n - 1; // workgroup h + 1 ran sweep s - 1
+        const i64 cur = (s & 1) * mw, prev = mw - cur;       // this and the previous sweep's buffers
+        const unsigned tag = (unsigned)s + 1u;
+
+        // ---- 1. w' from the left, beta from the right
+        if (wave == 0 && h > 0) {
+            T v = T(0);
+            if (!poll(left + cur, lane < B, tag, v)) s_go = 0;
+            if (lane < B) s_wp[lane] = v;
+        }
+        if (wave == 1) {
+            T v = T(0);
+            if (right_row && !poll(right + prev + oBeta, lane == 0, tag - 1u, v)) s_go = 0;
+            if (lane == 0) s_beta = v;
+        }
+        __syncthreads();
+        if (!s_go) return;
+        T wp[CPT];
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) wp[j] = h > 0 ? s_wp[c0 + j] : T(0);
+        if (s > 0) {
+            const T beta = s_beta;
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) {
+                const bool col = c0 + j == kold;
+                L[j] = lam == kold ? (col ? beta : T(0)) : (col ? D[j] : L[j]);
+            }
+        }
+        // ---- 2. y = 2 L w', the reflector of column x
+        {
+            T acc = T(0);
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) acc += L[j] * wp[j];
+            s_part[cg][lam] = acc;
+            const int xs = h > 0 ? kap : kold; // slot of the column to eliminate
+#pragma unroll
+            for (int j = 0; j < CPT; ++j)
+                if (c0 + j == xs) s_x[lam] = L[j];
+        }
+        __syncthreads();
+        T y = T(0);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) y += s_part[g][lam];
+        y *= T(2);
+        const double x = (double)(s_x[lam] - (h > 0 ? y * s_wp[kap] : T(0)));
+        const double alpha = read_lane(x, kap);
+        const double tail = group_sum<B>(lam == kap ? 0.0 : x * x);
+        double wd = 0.0, beta = alpha;
+        if (tail != 0.0) {
+            const double nrm = sqrt(alpha * alpha + tail);
+            beta = (alpha >= 0.0) ? -nrm : nrm;
+            const double v0 = alpha - beta;
+            wd = (lam == kap ? v0 : x) * (1.0 / sqrt(v0 * v0 + tail));
+        }
+        const T w = (T)wd;
+        if (wave == 0) {
+            if (lane < B && r0 + B <= n - 1) MsgWord<T>::put(right + cur + lane * NWD, w, tag);
+        } else if (wave == 1) {
+            if (lane == 0) {
+                if (h > 0) MsgWord<T>::put(left + cur + oBeta, (T)beta, tag);
+                else ee[s] = (T)beta;
+            }
+        } else if (wave == 3) {
+            const int q = (lam - kap) & M;
+            if (lane < B && s <= n - 3 && r0 + q <= n - 1) U[(i64)h * B + q + (i64)s * ldu] = w;
+        }
+        // ---- 3. L -= y w'^T, L -= w (2 w^T L); row r0 of L
+        {
+            T u[CPT];
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) {
+                L[j] -= y * wp[j];
+                u[j] = w * L[j];
+            }
+            column_sums<B, CPT>(u, lane);
+            const T w2 = T(2) * w;
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) L[j] -= w2 * u[j];
+            if (lam == kap)
+#pragma unroll
+                for (int j = 0; j < CPT; ++j) s_lrow[c0 + j] = L[j];
+        }
+        if (wave == 2) {
+            T v = T(0);
+            if (right_row && !poll(right + prev + oRow, lane < B, tag - 1u, v)) s_go = 0;
+            if (lane < B) s_row[lane] = v;
+        }
+        __syncthreads();
+        if (!s_go) return;
+        if (wave == 3 && h > 0 && lane < B && lane != kap)
+            MsgWord<T>::put(left + cur + oRow + lane * NWD, s_lrow[lane], tag);
+        // ---- 4. D: its new row and column, then the two-sided update
+        if (s > 0) {
+            const T rl = s_row[lam];
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) {
+                const T rc = s_row[c0 + j];
+                D[j] = lam == kold ? rc : (c0 + j == kold ? rl : D[j]);
+            }
+        }
+        T wc[CPT];
+        {
+            T acc = T(0);
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) {
+                wc[j] = slot_value<B, CPT>(w, cw, j, lane);
+                acc += D[j] * wc[j];
+            }
+            s_part2[cg][lam] = acc;
+        }
+        __syncthreads();
+        T p = T(0);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) p += s_part2[g][lam];
+        p *= T(2);
+        const T yv = p - group_sum<B>(w * p) * w;
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) D[j] -= w * slot_value<B, CPT>(yv, cw, j, lane) + yv * wc[j];
+#pragma unroll
+        for (int j = 0; j < CPT; ++j)
+            if (lam == kap && c0 + j == kap) {
+                if (h > 0) MsgWord<T>::put(left + cur + oRow + kap * NWD, D[j], tag);
+                else dd[s + 1] = D[j];
+            }
+    }
+}
+
 template <typename T>
 __global__ void bc_extract_kernel(const T *Bp, T *d, T *e, int n, int b) {
     const i64 ldb = 2 * b;
@@ -514,7 +902,33 @@ template <typename T> size_t bc_lds_bytes(int b) {
     return sizeof(T) * ((size_t)2 * b * (2 * b + 1) + 2 * b + 3 * b + nseg * 3 * b);
 }
 
+// Resident form when its workgroups, one per hop of the first sweep, all fit on the GPU at
+// once (each waits for both neighbours); *done tells whether it was launched.
+template <typename T, int B> int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, bool *done) {
+    const int n = ws.n;
+    hipStream_t s = ws.stream;
+    *done = false;
+    const int hops = (n - 2) / B + 1;
+    int per_cu = 0;
+    CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bc_chase_resident_kernel<T, B>, chase_threads(B), 0));
+    if (hops > per_cu * device_cu_count()) return CUEV_STATUS_SUCCESS;
+    const i64 words = (i64)(hops + 1) * 2 * msg_words<T>(B);
+    CUEV_TRY(fill_int(s, reinterpret_cast<int *>(ws.chmsg), 2 * words, 0)); // no tag of an earlier chase
+    const double nhops = (double)n * n / (2.0 * B);
+    prof::Scope sc(s, "bc.chase", nhops * (6.0 * B * B + 16.0 * B * B), nhops * 4.0 * B * B * sizeof(T));
+    hipLaunchKernelGGL((bc_chase_resident_kernel<T, B>), dim3((unsigned)hops), dim3(chase_threads(B)), 0, s, Bp, ws.U,
+                       ws.ldu, n, d, e, reinterpret_cast<u64 *>(ws.chmsg), ws.err);
+    CUEV_LAUNCH_CHECK();
+    *done = true;
+    return CUEV_STATUS_SUCCESS;
+}
+
 } // namespace
+
+size_t bc_chase_msg_bytes(int n, int b) {
+    const i64 hops = n > 2 ? (n - 2) / b + 1 : 0;
+    return sizeof(u64) * (size_t)((hops + 1) * 2 * msg_words<double>(b));
+}
 
 template <typename T, int B> int launch_chase(Workspace<T> &ws, T *Bp) {
     const int n = ws.n;
@@ -562,6 +976,14 @@ template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e) {
     const int n = ws.n;
     hipStream_t s = ws.stream;
     if (n - 2 > 0) {
+        bool done = false;
+        switch (ws.b) {
+        case 16: CUEV_TRY((launch_chase_resident<T, 16>(ws, Bp, d, e, &done))); break;
+        case 32: CUEV_TRY((launch_chase_resident<T, 32>(ws, Bp, d, e, &done))); break;
+        case 64: CUEV_TRY((launch_chase_resident<T, 64>(ws, Bp, d, e, &done))); break;
+        default: CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "bc_chase: unsupported b=%d", ws.b);
+        }
+        if (done) return CUEV_STATUS_SUCCESS;
         switch (ws.b) {
         case 16: CUEV_TRY((launch_chase<T, 16>(ws, Bp))); break;
         case 32: CUEV_TRY((launch_chase<T, 32>(ws, Bp))); break;

@@ -9,4 +9,7 @@ namespace cuev {
 // reflectors stored in ws.U (shifted layout).
 template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e);
 
+// bytes of ws.chmsg, the message buffers of the resident chase (either precision)
+size_t bc_chase_msg_bytes(int n, int b);
+
 } // namespace cuev

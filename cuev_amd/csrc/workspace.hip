@@ -3,6 +3,7 @@
 
 #include <vector>
 
+#include "bulge.hpp"
 #include "gemm.hpp"
 #include "panel_qr.hpp"
 #include "util.hpp"
@@ -73,6 +74,8 @@ template <typename T> int workspace_alloc(Workspace<T> &ws, int n, int b, int k,
     off += al(64);
     const size_t op = off;
     off += al((size_t)n * sizeof(int));
+    const size_t ocm = off;
+    off += al(bc_chase_msg_bytes(n, b));
     const size_t oerr = off;
     off += al(64);
     // bc_back block reflectors: group g covers sweeps [16g, 16g+16) (sweeps 0..n-3), and
@@ -116,6 +119,7 @@ template <typename T> int workspace_alloc(Workspace<T> &ws, int n, int b, int k,
     ws.pqscratch = base + opq;
     ws.counter = reinterpret_cast<unsigned *>(base + oc);
     ws.prog = reinterpret_cast<int *>(base + op);
+    ws.chmsg = base + ocm;
     ws.err = reinterpret_cast<int *>(base + oerr);
     ws.BtT = reinterpret_cast<T *>(base + oBtT);
     ws.bt_off = reinterpret_cast<i64 *>(base + oBtO);
