@@ -615,7 +615,7 @@ int run_mixed(Context<float> &cf, MixedBuffers &mb, double *A, int n, double *ev
         if (!std::isfinite(mb.h_d[i]) || !std::isfinite(mb.h_e[i]))
             CUEV_FAIL(CUEV_STATUS_NOT_FINITE, "mixed: non-finite tridiagonal entry at %d", i);
     }
-    const int dc_mode = opt.dc_mode == CUEV_DC_AUTO ? (n >= 1024 ? CUEV_DC_DEVICE : CUEV_DC_HOST)
+    const int dc_mode = opt.dc_mode == CUEV_DC_AUTO ? (n >= kDeviceDcFrom ? CUEV_DC_DEVICE : CUEV_DC_HOST)
                                                    : opt.dc_mode;
     if (dc_mode == CUEV_DC_DEVICE) {
         if (!mb.dc) CUEV_TRY(dc_state_create<double>(mb.dc, n));

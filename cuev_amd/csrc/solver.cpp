@@ -61,6 +61,12 @@ float ev_ms(hipEvent_t a, hipEvent_t b) {
 // top three levels only, but bc_back alone varies there from 7.6 to 12 s between runs.
 int kDcGateFrom(int n) { return std::min(n / 4, 4096); }
 
+// The reordered order hides Q_s^T behind the chase and Q_b^T behind the D&C, also where
+// all of them are short: solves of n = 66, 130, 256, 512 and 1024 take 0.87, 1.84, 3.38,
+// 6.96 and 18.6 ms in the direct order and 0.84, 1.71, 2.97, 6.10 and 15.0 ms reordered
+// (FP64, b = 32). Below about 64 there is one panel and nothing to hide.
+constexpr int kReorderedFrom = 64;
+
 template <typename T>
 int tridi_dc(Context<T> &ctx, T *d, T *e, T *eval, T *evec, i64 ldv, double *dc_ms) {
     Workspace<T> &ws = ctx.ws;
@@ -116,9 +122,9 @@ int solve_native(Context<T> &ctx, T *A, T *eval, T *evec, cuev_solve_timer *time
     hipStream_t s = ws.stream;
     hipEvent_t *ev = ctx.ev;
     const auto wall0 = clk::now();
-    if (bt_mode == CUEV_BT_AUTO) bt_mode = (n >= 2048) ? CUEV_BT_REORDERED : CUEV_BT_DIRECT;
+    if (bt_mode == CUEV_BT_AUTO) bt_mode = (n >= kReorderedFrom) ? CUEV_BT_REORDERED : CUEV_BT_DIRECT;
     const bool reordered = bt_mode == CUEV_BT_REORDERED;
-    if (dc_mode == CUEV_DC_AUTO) dc_mode = (n >= 1024) ? CUEV_DC_DEVICE : CUEV_DC_HOST;
+    if (dc_mode == CUEV_DC_AUTO) dc_mode = (n >= kDeviceDcFrom) ? CUEV_DC_DEVICE : CUEV_DC_HOST;
     const bool dev_dc = dc_mode == CUEV_DC_DEVICE;
 
     if (reordered) CUEV_TRY(bt_ensure(ctx));

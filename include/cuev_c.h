@@ -100,13 +100,13 @@ typedef enum cuev_precision_t {
 } cuev_precision_t;
 
 typedef enum cuev_bt_mode_t {
-    CUEV_BT_AUTO = 0,      /* reordered for n >= 2048, direct otherwise */
+    CUEV_BT_AUTO = 0,      /* reordered for n >= 64, direct otherwise */
     CUEV_BT_DIRECT = 1,    /* evec <- Q_s (Q_b Q_d) after the D&C (reference order) */
     CUEV_BT_REORDERED = 2  /* build Q_b^T Q_s^T on the GPU beside the chase and the D&C, then one GEMM */
 } cuev_bt_mode_t;
 
 typedef enum cuev_dc_mode_t {
-    CUEV_DC_AUTO = 0,   /* device for n >= 1024, host otherwise */
+    CUEV_DC_AUTO = 0,   /* device for n >= 160, host otherwise */
     CUEV_DC_HOST = 1,   /* host LAPACK ?stedc, Q_d uploaded (the reference's north-star form) */
     CUEV_DC_DEVICE = 2  /* divide and conquer with Q resident on the GPU: host deflation
                            bookkeeping and leaves, device secular roots, vectors and GEMMs
@@ -114,7 +114,7 @@ typedef enum cuev_dc_mode_t {
 } cuev_dc_mode_t;
 
 typedef struct cuev_options {
-    int bandwidth;       /* b in {16, 32, 64}; 0 selects the default (64 for n >= 4096, else 32) */
+    int bandwidth;       /* b in {16, 32, 64}; 0 selects the default (64 for n >= 256, else 32) */
     int block;           /* k, a multiple of b; 0 selects 512 (clamped to n) */
     int precision;       /* cuev_precision_t */
     int refine_sweeps;   /* mixed form: maximum sweeps; 0 selects 3 */
