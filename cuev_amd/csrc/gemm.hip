@@ -799,9 +799,8 @@ int gemm_ex(hipStream_t s, i64 M, i64 N, i64 K, T alpha, const Operand<T> &A,
     };
     int cfg;
     const bool sym_panel = A.sym && N <= 64;
-    // a tall-skinny update (the band reduction's panel-wide products): 64 x 64 tiles
-    // for the row parallelism
-    const bool tall_skinny = !lower && !A.sym && N <= 64 && M >= 2048 && K < 1024;
+    // a panel-wide update (N <= 64, short K): 64 x 64 tiles for the row parallelism
+    const bool tall_skinny = !lower && !A.sym && N <= 64 && K < 1024;
     const bool tcat = A.split >= 0 && A.trans;
     if (tcat && (A.split % 64 != 0 || B.split >= 0 || B.trans || A.sym))
         CUEV_FAIL(CUEV_STATUS_NOT_SUPPORTED,
@@ -831,17 +830,21 @@ int gemm_ex(hipStream_t s, i64 M, i64 N, i64 K, T alpha, const Operand<T> &A,
 
     // split-K for products with few output tiles and a long K (from 1024, or from 256
     // for at most four tiles). The K chunks are short (64): a workgroup of these
-    // products waits on memory latency at every K step, so many short chunks keep more
-    // loads in flight than a few long ones. Tall-skinny updates (N <= 64, short K) are
-    // split four ways.
+    // products waits on memory latency at every K step (about 1.5 us per 16), so many
+    // short chunks keep more loads in flight than a few long ones. Panel-wide updates
+    // (N <= 64, K < 1024) of 2048 rows and more are split four ways, shorter ones until
+    // there is a workgroup per CU: 1200 x 64 with K = 800 took 100 us unsplit and takes
+    // 12 in 13 splits, and their sum 5. The symmetric panel product keeps chunks of 256
+    // while those fill the GPU and goes down to 64 below (1200 rows: 50 -> 13 us).
     int splits = 1;
     const i64 target = (sym_panel ? (cfg == C128x64W8 ? 8LL : 16LL) : 2LL) * cus;
-    const i64 kmin = sym_panel ? 256 : 64; // shortest K chunk per split
+    const i64 kmin = sym_panel ? std::min<i64>(256, std::max<i64>(64, K * ntiles / cus)) : 64;
     if (K == 0) {
         splits = 0;
     } else if (tall_skinny && K >= 128) {
         const i64 cap = (i64)(scratch.bytes / ((size_t)M * N * sizeof(T)));
-        const i64 want = std::min<i64>(std::min<i64>(4, K / 64), cap);
+        const i64 ways = M >= 2048 ? 4 : ceil_div(cus, ntiles);
+        const i64 want = std::min<i64>(std::min<i64>(ways, K / 64), cap);
         if (want > 1) splits = (int)want;
     } else if (ntiles < target / 2 && (K >= 1024 || (ntiles <= 4 && K >= 256))) {
         i64 want = std::min<i64>(ceil_div(target, ntiles), K / kmin);
