@@ -1,4 +1,5 @@
 // capi.cpp — the extern "C" boundary declared in include/cuev_c.h.
+#include <chrono>
 #include <cstring>
 
 #include "backtransform.hpp"
@@ -10,6 +11,7 @@
 #include "gemm.hpp"
 #include "lapack.hpp"
 #include "refine.hpp"
+#include "small.hpp"
 #include "solver.hpp"
 #include "tridi_values.hpp"
 #include "util.hpp"
@@ -37,6 +39,27 @@ template <> Context<double> *ctx_of<double>(cuev_handle_t h) {
     if (!ctx)                                                                                      \
         CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "%s: null handle or handle of the other precision", \
                   __func__);
+
+// Orders up to kSmallMaxN with no stage option set: one kernel of one workgroup instead of
+// the staged pipeline's launches and hand-offs (n = 48 and 128 in FP64: 0.50 and 1.67 ms staged,
+// 0.16 and 0.54 in one kernel). An option that names a stage keeps the pipeline, and so do
+// orders above 32 whose eigenvalues are too close for the kernel's fast path (*done = false,
+// A untouched): its QL takes 0.85 ms at n = 48 and 5.2 at 128.
+template <typename T>
+int small_entry(const T *A, int n, T *eval, T *evec, int il, int iu, hipStream_t s, cuev_solve_timer *timer,
+                bool *done) {
+    const auto t0 = std::chrono::steady_clock::now();
+    int failed = 0, bad = 0, ql = 0;
+    CUEV_TRY(small_eig<T>(s, A, n, 1, eval, evec, il, iu, &failed, &bad, n > 32 ? &ql : nullptr));
+    *done = ql == 0;
+    if (bad) CUEV_FAIL(CUEV_STATUS_NOT_FINITE, "the matrix has a non-finite entry");
+    if (failed) CUEV_FAIL(CUEV_STATUS_LAPACK_ERROR, "the tridiagonal QL iteration did not converge (n=%d)", n);
+    if (timer) {
+        std::memset(timer, 0, sizeof(*timer));
+        timer->total_ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    }
+    return CUEV_STATUS_SUCCESS;
+}
 
 template <typename T>
 int solve_entry(T *A, int n, T *eval, T *evec, hipStream_t s, cuev_solve_timer *timer,
@@ -67,6 +90,11 @@ int solve_entry(T *A, int n, T *eval, T *evec, hipStream_t s, cuev_solve_timer *
     }
     if (o.precision != CUEV_PRECISION_NATIVE)
         CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "symm_eig_solve: bad precision %d", o.precision);
+    if (n <= kSmallMaxN && !o.bandwidth && !o.block && o.bt_mode == CUEV_BT_AUTO && o.dc_mode == CUEV_DC_AUTO) {
+        bool done = false;
+        CUEV_TRY(small_entry<T>(A, n, eval, evec, 0, n - 1, s, timer, &done));
+        if (done) return CUEV_STATUS_SUCCESS;
+    }
     Context<T> *ctx = nullptr;
     CUEV_TRY(context_acquire<T>(ctx, n, b, k, s));
     const int st = solve_native<T>(*ctx, A, eval, evec, timer, o.bt_mode, o.dc_mode, o.dc_leaf);
@@ -96,6 +124,10 @@ int values_entry(T *A, int n, int il, int iu, T *eval, hipStream_t s, cuev_solve
     int b = o.bandwidth, k = o.block;
     CUEV_TRY(resolve_blocking(n, b, k));
     if (k > n) k = (int)round_up(n, b);
+    if (n <= kSmallMaxN && !o.bandwidth && !o.block) {
+        bool done = false;
+        return small_entry<T>(A, n, eval, static_cast<T *>(nullptr), il, iu, s, timer, &done);
+    }
     Context<T> *ctx = nullptr;
     CUEV_TRY(context_acquire<T>(ctx, n, b, k, s));
     const int st = solve_values<T>(*ctx, A, il, iu, eval, timer);
@@ -269,6 +301,7 @@ int cuev_cache_release(void) {
     context_release_all<double>();
     mixed_release_all();
     backward_release_all();
+    small_release_all();
     return CUEV_STATUS_SUCCESS;
 }
 

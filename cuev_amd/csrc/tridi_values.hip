@@ -37,39 +37,14 @@
 
 #include <cfloat>
 
+#include "sturm.hpp"
+
 namespace cuev {
 namespace {
 
 constexpr int kTvThreads = 256;
 constexpr int kTvRows = 4080; // (d, e^2) pairs per LDS stage, a multiple of 8 (64 KiB with the 8 more)
 inline int tv_stage_rows(int n) { return n < kTvRows ? (n + 7) / 8 * 8 : kTvRows; }
-
-// Sign changes of p over the rows of one stage: pp = p_{i-2}, p = p_{i-1} on entry. The
-// next 8 rows are read from LDS while 8 are computed (de holds 8 rows more than `rows`).
-__device__ __forceinline__ int sturm_rows(const double2 *de, int rows, double x, double &pp, double &p) {
-    int cnt = 0;
-    double2 v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = de[u];
-    for (int i = 0; i < rows; i += 8) {
-        double2 nx[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) nx[u] = de[i + 8 + u];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const double q = fma(v[u].x - x, p, -(v[u].y * pp));
-            cnt += (int)((unsigned)(__double2hiint(q) ^ __double2hiint(p)) >> 31);
-            pp = p;
-            p = q;
-        }
-        const int ex = __builtin_amdgcn_frexp_exp(fmax(fabs(pp), fabs(p)));
-        pp = ldexp(pp, -ex);
-        p = ldexp(p, -ex);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = nx[u];
-    }
-    return cnt;
-}
 
 template <typename T, int L>
 __global__ __launch_bounds__(kTvThreads) void sturm_multisect_kernel(const T *__restrict__ d,

@@ -137,7 +137,8 @@ void cuev_options_init(cuev_options *opt);
 
 /* ------------------------------------------------------------------------ */
 /* Full eigensolve (drop-in for cuev::symm_eig_solve<T>, include/cuev.h:31)  */
-/* Blocking: returns after all results are in eval/evec.                     */
+/* Blocking: returns after all results are in eval/evec. Up to n = 128 with   */
+/* no stage option set the stages are one kernel: only total_ms is filled.   */
 /* ------------------------------------------------------------------------ */
 int cuev_ssymm_eig_solve(float *A, int n, float *eval, float *evec, hipStream_t stream,
                          cuev_solve_timer *timer);
@@ -176,9 +177,9 @@ int cuev_dtridi_values(const double *d, const double *e, int n, int il, int iu, 
 /* Batched small eigenproblems (no reference counterpart: the reference      */
 /* solves one matrix per call, include/cuev.h:31-33). batch matrices of order */
 /* n <= 256, stored one after another (each n x n column-major, ld n; lower   */
-/* triangle read; A is overwritten); eval receives batch x n eigenvalues      */
+/* triangle read; A may be overwritten); eval receives batch x n eigenvalues      */
 /* (ascending per matrix), evec batch eigenvector matrices (columns). One      */
-/* workgroup per matrix, cyclic Jacobi. Blocking. Returns NOT_CONVERGED if a   */
+/* workgroup per matrix: tridiagonalization up to n = 128, cyclic Jacobi above. Blocking. Returns NOT_CONVERGED if a   */
 /* matrix did not converge (count in *n_not_converged when not NULL).          */
 /* ------------------------------------------------------------------------ */
 int cuev_ssymm_eig_batched(float *A, int n, int batch, float *eval, float *evec, hipStream_t stream,
