@@ -88,14 +88,7 @@ int check_args(const void *V, const void *lam, const void *Abar, int n) {
     return CUEV_STATUS_SUCCESS;
 }
 
-// ---- cached work buffer of the allocating entry point (one idle buffer per device)
-struct BwdBuf {
-    void *p = nullptr;
-    size_t bytes = 0;
-    int device = -1;
-};
-std::mutex g_bwd_mu;
-BwdBuf g_bwd_idle[64];
+IdleBuffers g_bwd; // work buffers of the allocating entry point
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -134,23 +127,8 @@ int eig_backward(const T *V, const T *lam, const T *Vbar, const T *lambar, int n
     const size_t mat = align256((size_t)n * n * sizeof(T));
     const size_t gsb = gemm_scratch_bytes(n, n, sizeof(T));
     const size_t need = 2 * mat + 256 + gsb;
-    int dev = 0;
-    CUEV_HIP(hipGetDevice(&dev));
-    BwdBuf buf;
-    {
-        std::lock_guard<std::mutex> lk(g_bwd_mu);
-        BwdBuf &slot = g_bwd_idle[dev & 63];
-        if (slot.p && slot.device == dev && slot.bytes >= need) {
-            buf = slot;
-            slot = BwdBuf{};
-        }
-    }
-    if (!buf.p) {
-        buf.device = dev;
-        buf.bytes = need;
-        if (hipMalloc(&buf.p, need) != hipSuccess)
-            CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "eig_backward: device allocation of %zu bytes failed (n=%d)", need, n);
-    }
+    IdleBuffers::Buffer buf;
+    CUEV_TRY(g_bwd.take(buf, need));
     auto *base = static_cast<unsigned char *>(buf.p);
     T *C = reinterpret_cast<T *>(base);
     T *Tm = reinterpret_cast<T *>(base + mat);
@@ -159,40 +137,11 @@ int eig_backward(const T *V, const T *lam, const T *Vbar, const T *lambar, int n
     const int st =
         backward_core<T>(V, lam, Vbar, lambar, n, Abar, gap_tol, n_masked_host, s, C, Tm, dmask, gs, true);
     (void)hipStreamSynchronize(s);
-    BwdBuf victim;
-    {
-        std::lock_guard<std::mutex> lk(g_bwd_mu);
-        BwdBuf &slot = g_bwd_idle[dev & 63];
-        if (slot.p && slot.bytes >= buf.bytes) {
-            victim = buf; // keep the larger of the two
-        } else {
-            victim = slot;
-            slot = buf;
-        }
-    }
-    if (victim.p) (void)hipFree(victim.p);
+    g_bwd.give(buf);
     return st;
 }
 
-void backward_release_all() {
-    BwdBuf victims[64];
-    {
-        std::lock_guard<std::mutex> lk(g_bwd_mu);
-        for (int i = 0; i < 64; ++i) {
-            victims[i] = g_bwd_idle[i];
-            g_bwd_idle[i] = BwdBuf{};
-        }
-    }
-    int cur = 0;
-    (void)hipGetDevice(&cur);
-    for (BwdBuf &v : victims)
-        if (v.p) {
-            (void)hipSetDevice(v.device);
-            (void)hipDeviceSynchronize();
-            (void)hipFree(v.p);
-        }
-    (void)hipSetDevice(cur);
-}
+void backward_release_all() { g_bwd.release_all(); }
 
 template <typename T>
 int eig_backward_noalloc(const T *V, const T *lam, const T *Vbar, const T *lambar, int n, T *Abar,

@@ -146,6 +146,10 @@ int tridi_values_entry(const T *d, const T *e, int n, int il, int iu, T *w, hipS
     return tridi_values<T>(s, d, e, n, il, iu, w);
 }
 
+// split-K partials of the product entry points (allocating and freeing 100 to 200 MB took
+// 0.27 ms per call: an FP32 product of order 1000 took 0.37 ms and takes 0.11)
+IdleBuffers g_product_scratch;
+
 template <typename T>
 int gemm_entry(hipStream_t s, int ta, int tb, i64 m, i64 n, i64 k, T alpha, const T *A, i64 lda,
                const T *B, i64 ldb, T beta, T *C, i64 ldc) {
@@ -154,12 +158,11 @@ int gemm_entry(hipStream_t s, int ta, int tb, i64 m, i64 n, i64 k, T alpha, cons
     if ((ta != 0 && ta != 1) || (tb != 0 && tb != 1))
         CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "gemm: trans must be 0 or 1");
     const size_t bytes = gemm_scratch_bytes(m, n, sizeof(T));
-    void *scr = nullptr;
-    if (hipMalloc(&scr, bytes) != hipSuccess)
-        CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "gemm: scratch allocation failed");
-    int st = gemm<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, Scratch{scr, bytes});
+    IdleBuffers::Buffer scr;
+    CUEV_TRY(g_product_scratch.take(scr, bytes));
+    int st = gemm<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, Scratch{scr.p, bytes});
     (void)hipStreamSynchronize(s);
-    (void)hipFree(scr);
+    g_product_scratch.give(scr);
     return st;
 }
 
@@ -168,12 +171,11 @@ int symm_entry(hipStream_t s, i64 m, i64 n, T alpha, const T *A, i64 lda, const 
                T beta, T *C, i64 ldc) {
     detail::clear_error();
     const size_t bytes = gemm_scratch_bytes(m, n, sizeof(T));
-    void *scr = nullptr;
-    if (hipMalloc(&scr, bytes) != hipSuccess)
-        CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "symm: scratch allocation failed");
-    int st = symm_lower<T>(s, m, n, alpha, A, lda, B, ldb, beta, C, ldc, Scratch{scr, bytes});
+    IdleBuffers::Buffer scr;
+    CUEV_TRY(g_product_scratch.take(scr, bytes));
+    int st = symm_lower<T>(s, m, n, alpha, A, lda, B, ldb, beta, C, ldc, Scratch{scr.p, bytes});
     (void)hipStreamSynchronize(s);
-    (void)hipFree(scr);
+    g_product_scratch.give(scr);
     return st;
 }
 
@@ -182,12 +184,11 @@ int syr2k_entry(hipStream_t s, i64 n, i64 k, T alpha, const T *A, i64 lda, const
                 T beta, T *C, i64 ldc) {
     detail::clear_error();
     const size_t bytes = gemm_scratch_bytes(n, n, sizeof(T));
-    void *scr = nullptr;
-    if (hipMalloc(&scr, bytes) != hipSuccess)
-        CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "syr2k: scratch allocation failed");
-    int st = syr2k_lower<T>(s, n, k, alpha, A, lda, B, ldb, beta, C, ldc, Scratch{scr, bytes});
+    IdleBuffers::Buffer scr;
+    CUEV_TRY(g_product_scratch.take(scr, bytes));
+    int st = syr2k_lower<T>(s, n, k, alpha, A, lda, B, ldb, beta, C, ldc, Scratch{scr.p, bytes});
     (void)hipStreamSynchronize(s);
-    (void)hipFree(scr);
+    g_product_scratch.give(scr);
     return st;
 }
 
@@ -302,6 +303,7 @@ int cuev_cache_release(void) {
     mixed_release_all();
     backward_release_all();
     small_release_all();
+    g_product_scratch.release_all();
     return CUEV_STATUS_SUCCESS;
 }
 
