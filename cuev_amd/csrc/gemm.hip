@@ -380,8 +380,8 @@ __device__ __forceinline__ void gemm_body_regs(const KParams<T> &p) {
 //     one DMA instruction fills 1 KB of consecutive LDS);
 //   RC operand (rows contiguous): [k][row] with a row stride of R + 8 doubles, which
 //     puts the k and k+2 reads of one fragment read in different bank halves.
-// Edge tiles, K tails and unaligned operands are loaded per element (bounds-checked)
-// into the same layouts.
+// K tails, row-contiguous edges of odd sizes and symmetric tiles across the diagonal are
+// loaded per element (bounds-checked) into the same layouts.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int kc_swz(int r) { return (r ^ (r >> 3)) & 7; }
 
@@ -391,9 +391,12 @@ template <int R> struct DmaTile {
     template <bool KC> static constexpr int bytes() { return KC ? R * BK * 8 : BK * RSTR * 8; }
 };
 
-// DMA of one interior R x 16 tile; the LDS destination of each instruction is wave-uniform.
+// DMA of one R x 16 tile; the LDS destination of each instruction is wave-uniform. Rows past
+// the operand's last one (rlim) are read from it again: what they give is never stored. A
+// row-contiguous tile moves pairs of rows, so there rlim has to be even (dma_rows).
+__device__ __forceinline__ bool dma_rows(bool kc, bool inside, i64 rlim) { return inside || kc || !(rlim & 1); }
 template <int R, int NT>
-__device__ __forceinline__ void dma_tile(bool kc, const double *p, i64 ld, i64 r0, i64 k0, char *s, int tid) {
+__device__ __forceinline__ void dma_tile(bool kc, const double *p, i64 ld, i64 r0, i64 k0, i64 rlim, char *s, int tid) {
     const int lane = tid & 63, wave = tid >> 6;
     constexpr int NW = NT / 64;
     if (kc) {
@@ -403,7 +406,7 @@ __device__ __forceinline__ void dma_tile(bool kc, const double *p, i64 ld, i64 r
             const int inst = wave * NI + i;
             const int pos = inst * 64 + lane;
             const int row = pos >> 3, c = (pos & 7) ^ kc_swz(row);
-            const double *g = p + (r0 + row) * ld + k0 + 2 * c;
+            const double *g = p + min(r0 + row, rlim - 1) * ld + k0 + 2 * c;
             __builtin_amdgcn_global_load_lds((gvoid_t *)g, (lvoid_t *)(s + inst * 1024), 16, 0, 0);
         }
     } else if constexpr (R >= 128) {
@@ -415,7 +418,7 @@ __device__ __forceinline__ void dma_tile(bool kc, const double *p, i64 ld, i64 r
         for (int i = 0; i < NI; ++i) {
             const int inst = wave * NI + i;
             const int kk = inst / PER_K, part = inst % PER_K;
-            const double *g = p + (k0 + kk) * ld + r0 + part * 128 + 2 * lane;
+            const double *g = p + (k0 + kk) * ld + min(r0 + part * 128 + 2 * lane, rlim - 2);
             __builtin_amdgcn_global_load_lds((gvoid_t *)g,
                                              (lvoid_t *)(s + ((size_t)kk * DmaTile<R>::RSTR + part * 128) * 8), 16,
                                              0, 0);
@@ -424,7 +427,7 @@ __device__ __forceinline__ void dma_tile(bool kc, const double *p, i64 ld, i64 r
 }
 
 // Per-element load of an R x 16 tile (rows < rlim, k < klim; zero elsewhere) into the
-// DMA layouts (synchronous: used for edge tiles, K tails and unaligned operands).
+// DMA layouts (synchronous).
 // sym: p holds the lower triangle of a symmetric matrix, (r, k) read at p[r + k*ld]
 // if r >= k, else p[k + r*ld], into either layout.
 template <int R, int NT>
@@ -432,23 +435,27 @@ __device__ __forceinline__ void scalar_tile(bool kc, const double *p, i64 ld, i6
                                             char *s, int tid, bool sym = false) {
     double *d = reinterpret_cast<double *>(s);
     constexpr int PER = R * 16 / NT;
-    // one element at a time (edge tiles only): few live registers beside the accumulators
+    // four loads in flight per thread (their round trip is what such a tile costs; more
+    // take registers from the accumulators)
+    constexpr int U = PER < 4 ? PER : 4;
 #pragma unroll 1
-    for (int q = 0; q < PER; ++q) {
-        const int idx = tid + q * NT;
-        int row, kk;
-        if (kc) {
-            row = idx >> 4;
-            kk = idx & 15;
-        } else {
-            row = idx % R;
-            kk = idx / R;
+    for (int q = 0; q < PER; q += U) {
+        double v[U];
+        int row[U], kk[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int idx = tid + (q + u) * NT;
+            row[u] = kc ? idx >> 4 : idx % R;
+            kk[u] = kc ? idx & 15 : idx / R;
+            const i64 r = r0 + row[u], k = k0 + kk[u];
+            const i64 off = sym ? ((r >= k) ? r + k * ld : k + r * ld) : (kc ? k + r * ld : r + k * ld);
+            v[u] = (r < rlim && k < klim) ? p[off] : 0.0;
         }
-        const i64 r = r0 + row, k = k0 + kk;
-        const i64 off = sym ? ((r >= k) ? r + k * ld : k + r * ld) : (kc ? k + r * ld : r + k * ld);
-        const double v = (r < rlim && k < klim) ? p[off] : 0.0;
-        if (kc) d[(row * 8 + ((kk >> 1) ^ kc_swz(row))) * 2 + (kk & 1)] = v;
-        else d[kk * DmaTile<R>::RSTR + row] = v;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (kc) d[(row[u] * 8 + ((kk[u] >> 1) ^ kc_swz(row[u]))) * 2 + (kk[u] & 1)] = v[u];
+            else d[kk[u] * DmaTile<R>::RSTR + row[u]] = v[u];
+        }
     }
 }
 
@@ -525,10 +532,11 @@ __device__ __forceinline__ void gemm_body_dma(const KParams<double> &p) {
             }
             if constexpr (ASYM) {
                 const bool above = m0 + BM - 1 <= k0, below = m0 >= k0 + BK - 1;
-                if ((above || below) && m_in && k_in && p.avec) dma_tile<BM, NT>(above, pa, lda, m0, k0, st, tid);
+                if ((above || below) && k_in && p.avec && dma_rows(above, m_in, p.M))
+                    dma_tile<BM, NT>(above, pa, lda, m0, k0, p.M, st, tid);
                 else scalar_tile<BM, NT>(above, pa, lda, m0, k0, p.M, kend, st, tid, true);
             } else {
-                if (m_in && k_in && p.avec) dma_tile<BM, NT>(AKC, pa, lda, m0, k0 - ko, st, tid);
+                if (k_in && p.avec && dma_rows(AKC, m_in, p.M)) dma_tile<BM, NT>(AKC, pa, lda, m0, k0 - ko, p.M, st, tid);
                 else scalar_tile<BM, NT>(AKC, pa, lda, m0, k0 - ko, p.M, kend - ko, st, tid);
             }
         }
@@ -542,7 +550,8 @@ __device__ __forceinline__ void gemm_body_dma(const KParams<double> &p) {
                     ko = p.bsplit;
                 }
             }
-            if (n_in && k_in && p.bvec) dma_tile<BN, NT>(BKC, pb, ldb, n0, k0 - ko, st + ABYTES, tid);
+            if (k_in && p.bvec && dma_rows(BKC, n_in, p.N))
+                dma_tile<BN, NT>(BKC, pb, ldb, n0, k0 - ko, p.N, st + ABYTES, tid);
             else scalar_tile<BN, NT>(BKC, pb, ldb, n0, k0 - ko, p.N, kend - ko, st + ABYTES, tid);
         }
     };
