@@ -11,7 +11,7 @@
 //
 // Two kernels: the resident form (bc_chase_resident_kernel, described there) wherever its
 // workgroups, one per hop of the first sweep, fit on the GPU at once, and the windowed
-// form below for the larger n (b = 64 in FP64: n > 32768), where it still is the only one.
+// form below for the larger n (b = 64 in FP64: n > 49152), where it still is the only one.
 //
 // Design of the windowed form (not the reference's):
 //  * Reflector convention: if the vector below the pivot is exactly zero the
@@ -517,31 +517,39 @@ __global__ __launch_bounds__(kBCThreads) void bc_chase_kernel(T *Bp, T *U, i64 l
 // vector, the CPT elements of each block in registers.
 //
 // Per sweep, workgroup h
-//   1. receives w' = w_{h-1}(s) from its left neighbour and the value beta that its
-//      right neighbour left in column r0 - 1 in sweep s - 1; the column r0 - 1 of D becomes
-//      a column of L, a zero row with beta in it enters L;
+//   1. receives w' = w_{h-1}(s) from its left neighbour; column r0 - 1 of D becomes a column
+//      of L, a zero row enters L;
 //   2. y = 2 L w', x = column r0 - b of L - y w'^T, the reflector w and beta of x (every
 //      wave forms it from the same sums, so it is not sent through LDS), w to the right,
-//      beta to the left;
+//      beta to the left. The value beta that the right neighbour left in the entering row
+//      in sweep s - 1 (its only entry, in column r0 - 1) joins after the partial sums;
 //   3. L -= y w'^T, L -= w (2 w^T L); its row r0 goes to the left neighbour;
 //   4. receives row r1 of sweep s - 1 from the right (new last row and column of D);
 //      p = 2 D w, D -= w y^T + y w^T with y = p - (w^T p) w; D(r0, r0) goes to the left.
+//      The right's D(r1, r1), the last value it forms, joins after the partial sums.
 // Workgroup 0 writes (d, e). Rows and columns from n on are zeros, which need no special
-// cases: a one-row hop finds a zero tail and makes the identity.
+// cases: a one-row hop finds a zero tail and makes the identity. A ninth wave (fifth, for
+// b <= 32) does the receiving, each message between the two barriers before its first use,
+// so that no round trip of 0.4 us stands in the others' way.
 //
 // A message word is 64 bits: 32 bits of payload and the sweep number + 1 as a tag, so the
 // receiver polls the data itself and one store-to-load latency covers the hand-off (a
 // flag behind the data costs a second one). Buffers are double: sweep s + 2 overwrites
 // sweep s's words only after an answer that was computed from them came back.
 //
-// Bound: the sweep-to-sweep lag, two hand-offs (w to the right, beta to the left; about
-// 1 us each) and two times steps 1-2. Measured alone, FP64: 3.9 us per sweep at b = 64 and
-// 3.2 at b = 32, against 16.4 and 9.1 for the windowed kernel, which moves 2 b columns
-// through memory per hop and pays two dependent global round trips per hop (n = 16384:
-// 276 -> 64 ms; n = 4096: 67 -> 16 ms; n = 1024, b = 32: 9.3 -> 3.3 ms). Beside Q_s^T's
-// products it shares every CU with them (n = 16384: 119 ms, and 183 ms for the products).
-// Neighbouring workgroups on one XCD gained nothing (3.9 us) and lost beside the products
-// (147 ms), a sleep between polls 0.1 us; three workgroups per CU (84 VGPRs) cost 1 us.
+// Bound: the sweep-to-sweep lag. Its cycles: a hand-off to the right, steps 1-2 there, beta
+// back, the end of step 2; the same with D(r1, r1); and a workgroup's own steps 1-4. All
+// three take about 3.1 us at b = 64 (of which a hand-off 0.5, step 2 1.0, step 4 1.2).
+// Measured alone, FP64: 3.1 us per sweep at b = 64 and 2.75 at b = 32, against 16.4 and 9.1
+// for the windowed kernel, which moves 2 b columns through memory per hop and pays two
+// dependent global round trips per hop (n = 16384: 276 -> 52 ms; n = 4096: 67 -> 13 ms;
+// n = 1024, b = 32: 9.3 -> 2.7 ms). Beside Q_s^T's products it shares every CU with them
+// (n = 16384: 99 ms, and 145 ms for the products). With compute waves polling and both late
+// values awaited at the start it took 3.9 us (the form without the ninth wave still does);
+// neighbouring workgroups on one XCD, a sleep between polls or two to four polls in flight
+// gained nothing; four or sixteen compute waves took 4.9 and 3.8 us against 3.9 for eight.
+// The ninth wave's own loop keeps it from holding a block it never uses: 74 VGPRs instead
+// of 104, so that two workgroups fit on a CU, and 3.1 us instead of 3.3.
 // ---------------------------------------------------------------------------
 using u64 = unsigned long long;
 
@@ -572,10 +580,10 @@ template <> struct MsgWord<float> {
 };
 
 // Message buffers of the link between workgroups h - 1 and h, one set per parity of s:
-// w (h - 1 -> h, b values), row (h -> h - 1, b values), beta (h -> h - 1, one value on a
-// line of its own).
+// w (h - 1 -> h, b values), row (h -> h - 1, b values), beta and the row's diagonal entry
+// (h -> h - 1, one value each on a line of its own).
 constexpr int kBetaPad = 16; // values
-template <typename T> __host__ __device__ constexpr i64 msg_words(int b) { return (2 * b + kBetaPad) * (i64)(sizeof(T) / 4); }
+template <typename T> __host__ __device__ constexpr i64 msg_words(int b) { return (2 * b + 2 * kBetaPad) * (i64)(sizeof(T) / 4); }
 
 // v of row slot idx0 + j of the lane's column group: lane slots repeat every B lanes, so
 // lanes 0..B-1 hold them all. `first`: the first column slot of the wave (uniform).
@@ -593,21 +601,15 @@ template <int B, int CPT, typename V> __device__ __forceinline__ void column_sum
     if constexpr (B == 16) {
 #pragma unroll
         for (int j = 0; j < CPT; ++j) v[j] = group_sum<16>(v[j]);
-    } else {
-        static_assert(CPT == B / 8, "eight lanes per column in the last step");
-        V t[4];
-        if constexpr (B == 64) {
+    } else if constexpr (B == 64) {
+        static_assert(CPT == 8, "eight lanes per column at the end");
+        V t[4], r[2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                V a = v[i], b = v[i + 4];
-                lane_swap<32>(a, b);
-                t[i] = a + b;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) t[i] = v[i];
+        for (int i = 0; i < 4; ++i) {
+            V a = v[i], b = v[i + 4];
+            lane_swap<32>(a, b);
+            t[i] = a + b;
         }
-        V r[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             V a = t[i], b = t[i + 2];
@@ -615,39 +617,62 @@ template <int B, int CPT, typename V> __device__ __forceinline__ void column_sum
             r[i] = a + b;
         }
         const bool odd = (lane & 8) != 0;
-        const V keep = odd ? r[1] : r[0], give = odd ? r[0] : r[1];
-        const V q = sum8(keep + dpp_mov<kRowRor8>(give)); // column j of the group in its lanes 8 j ..
+        const V q = sum8((odd ? r[1] : r[0]) + dpp_mov<kRowRor8>(odd ? r[0] : r[1]));
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) {
-            if constexpr (B == 64) v[j] = read_lane(q, 8 * j);
-            else {
-                const V a = read_lane(q, 8 * j), b = read_lane(q, 32 + 8 * j);
-                v[j] = lane < 32 ? a : b;
-            }
+        for (int j = 0; j < CPT; ++j) v[j] = read_lane(q, 8 * j);
+    } else if constexpr (B == 32) {
+        static_assert(CPT == 4, "eight lanes per column at the end");
+        V r[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            V a = v[i], b = v[i + 2];
+            lane_swap<16>(a, b);
+            r[i] = a + b;
+        }
+        const bool odd = (lane & 8) != 0;
+        const V q = sum8((odd ? r[1] : r[0]) + dpp_mov<kRowRor8>(odd ? r[0] : r[1]));
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) { // column j of the group in its lanes 8 j ..
+            const V a = read_lane(q, 8 * j), b = read_lane(q, 32 + 8 * j);
+            v[j] = lane < 32 ? a : b;
         }
     }
 }
 
-constexpr int chase_threads(int b) { return b == 64 ? 512 : 256; }
+// f(0) + ... + f(N - 1) pairwise (N a power of two): a short chain
+template <int N, typename F> __device__ __forceinline__ auto tree_sum(F &&f) {
+    decltype(f(0)) v[N];
+#pragma unroll
+    for (int g = 0; g < N; ++g) v[g] = f(g);
+#pragma unroll
+    for (int d = N / 2; d > 0; d /= 2)
+#pragma unroll
+        for (int g = 0; g < d; ++g) v[g] += v[g + d];
+    return v[0];
+}
 
-template <typename T, int B>
-__global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(const T *Bp, T *U, i64 ldu, int n, T *dd,
-                                                                             T *ee, u64 *msg, int *err) {
-    constexpr int NT = chase_threads(B);
-    constexpr int NG = NT / B;   // column groups
-    constexpr int CPT = B / NG;  // columns per thread
-    constexpr int SPW = CPT * (64 / B); // column slots per wave
+// compute threads (column groups of b rows), and with RECV one wave more that only receives
+constexpr int chase_compute(int b) { return b == 64 ? 512 : 256; }
+constexpr int chase_threads(int b, bool recv) { return chase_compute(b) + (recv ? 64 : 0); }
+
+template <typename T, int B, bool RECV>
+__global__ __launch_bounds__(chase_threads(B, RECV)) void bc_chase_resident_kernel(const T *Bp, T *U, i64 ldu, int n,
+                                                                                   T *dd, T *ee, u64 *msg, int *err) {
+    constexpr int NG = chase_compute(B) / B; // column groups
+    constexpr int CPT = B / NG;              // columns per thread
+    constexpr int SPW = CPT * (64 / B);      // column slots per wave
     constexpr int NWD = MsgWord<T>::N;
     constexpr int M = B - 1;
     const int ldb = 2 * B;
     __shared__ T s_wp[B], s_x[B], s_row[B], s_lrow[B];
     __shared__ T s_part[NG][B], s_part2[NG][B];
-    __shared__ T s_beta;
+    __shared__ T s_beta, s_diag;
     __shared__ int s_go;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lam = tid & M, cg = tid / B;
+    const bool receiver = RECV && wave == NG * B / 64;
+    const int lam = tid & M, cg = B == 64 ? wave : tid / B; // b = 64: uniform in the wave
     const int c0 = cg * CPT;       // this thread's first column slot
     const int cw = wave * SPW;     // this wave's first column slot
     const int h = blockIdx.x;
@@ -656,21 +681,8 @@ __global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(con
 
     const i64 mw = msg_words<T>(B);
     u64 *left = msg + (i64)h * 2 * mw, *right = left + 2 * mw; // links to h - 1 and h + 1
-    constexpr int oRow = B * NWD, oBeta = 2 * B * NWD;
+    constexpr int oRow = B * NWD, oBeta = 2 * B * NWD, oDiag = (2 * B + kBetaPad) * NWD;
 
-    T L[CPT], D[CPT];
-    {
-        const int r0 = 1 + h * B;
-        const int gi = r0 + ((lam - r0) & M);
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) {
-            const int gc = r0 + ((c0 + j - r0) & M);
-            const int hi = max(gi, gc), lo = min(gi, gc);
-            D[j] = hi < n ? Bp[(hi - lo) + (i64)lo * ldb] : T(0);
-            const int gl = gc - B, diff = gi - gl;
-            L[j] = (gi < n && gl >= 0 && diff <= B) ? Bp[diff + (i64)gl * ldb] : T(0);
-        }
-    }
     if (tid == 0) {
         s_go = 1;
         if (h == 0) {
@@ -694,63 +706,110 @@ __global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(con
         }
     };
 
-    for (int s = 0;; ++s) {
+    // the four messages of sweep s, each to be received before its barrier (A to D below)
+    auto right_ran = [&](int s) { return s > 0 && s + (h + 1) * B <= n - 1; }; // h + 1 had sweep s - 1
+    auto receive_w = [&](int s) { // A
+        T v = T(0);
+        if (h > 0 && !poll(left + (s & 1) * mw, lane < B, (unsigned)s + 1u, v)) s_go = 0;
+        if (lane < B) s_wp[lane] = v; // h = 0: zero
+    };
+    auto receive_one = [&](int s, int at, T *to) { // B: beta, D: the diagonal entry
+        T v = T(0);
+        if (right_ran(s) && !poll(right + ((s & 1) ^ 1) * mw + at, lane == 0, (unsigned)s, v)) s_go = 0;
+        if (lane == 0) *to = v;
+    };
+    auto receive_row = [&](int s) { // C; the diagonal slot stays zero
+        T v = T(0);
+        const bool want = lane < B && lane != ((s + h * B) & M);
+        if (right_ran(s) && !poll(right + ((s & 1) ^ 1) * mw + oRow, want, (unsigned)s, v)) s_go = 0;
+        if (lane < B) s_row[lane] = v;
+    };
+    if (receiver) {
+        for (int s = 0; s + 1 + h * B <= n - 1; ++s) {
+            receive_w(s);
+            __syncthreads(); // A
+            if (!s_go) return;
+            receive_one(s, oBeta, &s_beta);
+            __syncthreads(); // B
+            receive_row(s);
+            __syncthreads(); // C
+            receive_one(s, oDiag, &s_diag);
+            __syncthreads(); // D
+        }
+        return;
+    }
+
+    T L[CPT], D[CPT];
+    {
+        const int r0 = 1 + h * B;
+        const int gi = r0 + ((lam - r0) & M);
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) {
+            const int gc = r0 + ((c0 + j - r0) & M);
+            const int hi = max(gi, gc), lo = min(gi, gc);
+            D[j] = hi < n ? Bp[(hi - lo) + (i64)lo * ldb] : T(0);
+            const int gl = gc - B, diff = gi - gl;
+            L[j] = (gi < n && gl >= 0 && diff <= B) ? Bp[diff + (i64)gl * ldb] : T(0);
+        }
+    }
+    for (int s = 0; s + 1 + h * B <= n - 1; ++s) {
         const int r0 = s + 1 + h * B;
-        if (r0 > n - 1) break;
         const int kap = r0 & M, kold = (r0 - 1) & M;
-        const bool right_row = s > 0 && r0 + B - 1 <= n - 1; // workgroup h + 1 ran sweep s - 1
-        const i64 cur = (s & 1) * mw, prev = mw - cur;       // this and the previous sweep's buffers
+        const i64 cur = (s & 1) * mw; // this sweep's buffers
         const unsigned tag = (unsigned)s + 1u;
 
-        // ---- 1. w' from the left, beta from the right
-        if (wave == 0 && h > 0) {
-            T v = T(0);
-            if (!poll(left + cur, lane < B, tag, v)) s_go = 0;
-            if (lane < B) s_wp[lane] = v;
-        }
-        if (wave == 1) {
-            T v = T(0);
-            if (right_row && !poll(right + prev + oBeta, lane == 0, tag - 1u, v)) s_go = 0;
-            if (lane == 0) s_beta = v;
-        }
-        __syncthreads();
+        if (!RECV && wave == 0) receive_w(s);
+        __syncthreads(); // A: w' is here
         if (!s_go) return;
-        T wp[CPT];
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) wp[j] = h > 0 ? s_wp[c0 + j] : T(0);
+        // column indexes of this thread's group (outside 0 .. CPT - 1: another group's)
+        const int jo = kold - c0, jk = kap - c0, jx = h > 0 ? jk : jo; // jx: the column to eliminate
+        // ---- 1. the entering column and (zero) row of L; beta, its only entry there, joins below
         if (s > 0) {
-            const T beta = s_beta;
 #pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                const bool col = c0 + j == kold;
-                L[j] = lam == kold ? (col ? beta : T(0)) : (col ? D[j] : L[j]);
-            }
+            for (int j = 0; j < CPT; ++j) L[j] = lam == kold ? T(0) : (j == jo ? D[j] : L[j]);
         }
         // ---- 2. y = 2 L w', the reflector of column x
         {
-            T acc = T(0);
+            T acc[2] = {T(0), T(0)};
 #pragma unroll
-            for (int j = 0; j < CPT; ++j) acc += L[j] * wp[j];
-            s_part[cg][lam] = acc;
-            const int xs = h > 0 ? kap : kold; // slot of the column to eliminate
+            for (int j = 0; j < CPT; ++j) acc[j & 1] += L[j] * s_wp[c0 + j];
+            s_part[cg][lam] = acc[0] + acc[1];
 #pragma unroll
             for (int j = 0; j < CPT; ++j)
-                if (c0 + j == xs) s_x[lam] = L[j];
+                if (j == jx) s_x[lam] = L[j];
         }
-        __syncthreads();
-        T y = T(0);
-#pragma unroll
-        for (int g = 0; g < NG; ++g) y += s_part[g][lam];
+        if (!RECV && wave == 1) receive_one(s, oBeta, &s_beta);
+        __syncthreads(); // B: the partial sums, and beta
+        const T bold = s_beta, wpk = s_wp[kap], wpo = s_wp[kold];
+        T y = tree_sum<NG>([&](int g) { return s_part[g][lam]; });
+        T xt = s_x[lam];
+        if (s > 0 && lam == kold) { // the entering row is beta in column slot kold
+            y = bold * wpo;
+            if (h == 0) xt = bold;
+        }
         y *= T(2);
-        const double x = (double)(s_x[lam] - (h > 0 ? y * s_wp[kap] : T(0)));
-        const double alpha = read_lane(x, kap);
-        const double tail = group_sum<B>(lam == kap ? 0.0 : x * x);
+        double x = (double)(xt - y * wpk);
+        double alpha = read_lane(x, kap);
+        double tail = group_sum<B>(lam == kap ? 0.0 : x * x);
         double wd = 0.0, beta = alpha;
         if (tail != 0.0) {
-            const double nrm = sqrt(alpha * alpha + tail);
-            beta = (alpha >= 0.0) ? -nrm : nrm;
-            const double v0 = alpha - beta;
-            wd = (lam == kap ? v0 : x) * (1.0 / sqrt(v0 * v0 + tail));
+            double back = 1.0;
+            if (!(tail + alpha * alpha > 0x1p-900 && tail + alpha * alpha < 0x1p900)) {
+                // into the short square roots' range
+                const bool up = fabs(alpha) < 1.0 && tail < 1.0;
+                const double sc = up ? 0x1p500 : 0x1p-500;
+                back = up ? 0x1p-500 : 0x1p500;
+                x *= sc;
+                alpha *= sc;
+                tail = group_sum<B>(lam == kap ? 0.0 : x * x);
+            }
+            double nrm, inv, r;
+            fast_sqrt(alpha * alpha + tail, nrm, r);
+            if (alpha >= 0.0) nrm = -nrm;
+            beta = nrm * back;
+            alpha -= nrm;
+            fast_sqrt(alpha * alpha + tail, r, inv);
+            wd = (lam == kap ? alpha : x) * inv;
         }
         const T w = (T)wd;
         if (wave == 0) {
@@ -769,7 +828,8 @@ __global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(con
             T u[CPT];
 #pragma unroll
             for (int j = 0; j < CPT; ++j) {
-                L[j] -= y * wp[j];
+                if (s > 0 && lam == kold && j == jo) L[j] = bold;
+                L[j] -= y * s_wp[c0 + j]; // read again: held, it would cost the registers of a wave
                 u[j] = w * L[j];
             }
             column_sums<B, CPT>(u, lane);
@@ -780,13 +840,8 @@ __global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(con
 #pragma unroll
                 for (int j = 0; j < CPT; ++j) s_lrow[c0 + j] = L[j];
         }
-        if (wave == 2) {
-            T v = T(0);
-            if (right_row && !poll(right + prev + oRow, lane < B, tag - 1u, v)) s_go = 0;
-            if (lane < B) s_row[lane] = v;
-        }
-        __syncthreads();
-        if (!s_go) return;
+        if (!RECV && wave == 2) receive_row(s);
+        __syncthreads(); // C: row r0 of L, and the right's last row but for its diagonal entry
         if (wave == 3 && h > 0 && lane < B && lane != kap)
             MsgWord<T>::put(left + cur + oRow + lane * NWD, s_lrow[lane], tag);
         // ---- 4. D: its new row and column, then the two-sided update
@@ -795,31 +850,39 @@ __global__ __launch_bounds__(chase_threads(B)) void bc_chase_resident_kernel(con
 #pragma unroll
             for (int j = 0; j < CPT; ++j) {
                 const T rc = s_row[c0 + j];
-                D[j] = lam == kold ? rc : (c0 + j == kold ? rl : D[j]);
+                D[j] = lam == kold ? rc : (j == jo ? rl : D[j]);
             }
         }
         T wc[CPT];
         {
-            T acc = T(0);
+            T acc[2] = {T(0), T(0)};
 #pragma unroll
             for (int j = 0; j < CPT; ++j) {
                 wc[j] = slot_value<B, CPT>(w, cw, j, lane);
-                acc += D[j] * wc[j];
+                acc[j & 1] += D[j] * wc[j];
             }
-            s_part2[cg][lam] = acc;
+            s_part2[cg][lam] = acc[0] + acc[1];
         }
-        __syncthreads();
-        T p = T(0);
+        if (!RECV && wave == 3) receive_one(s, oDiag, &s_diag);
+        __syncthreads(); // D: the partial sums, and the diagonal entry
+        T p = tree_sum<NG>([&](int g) { return s_part2[g][lam]; });
+        if (s > 0) {
+            const T dg = s_diag;
+            if (lam == kold) {
+                p += dg * w;
 #pragma unroll
-        for (int g = 0; g < NG; ++g) p += s_part2[g][lam];
+                for (int j = 0; j < CPT; ++j)
+                    if (j == jo) D[j] = dg;
+            }
+        }
         p *= T(2);
         const T yv = p - group_sum<B>(w * p) * w;
 #pragma unroll
         for (int j = 0; j < CPT; ++j) D[j] -= w * slot_value<B, CPT>(yv, cw, j, lane) + yv * wc[j];
 #pragma unroll
         for (int j = 0; j < CPT; ++j)
-            if (lam == kap && c0 + j == kap) {
-                if (h > 0) MsgWord<T>::put(left + cur + oRow + kap * NWD, D[j], tag);
+            if (lam == kap && j == jk) {
+                if (h > 0) MsgWord<T>::put(left + cur + oDiag, D[j], tag);
                 else dd[s + 1] = D[j];
             }
     }
@@ -839,24 +902,51 @@ template <typename T> size_t bc_lds_bytes(int b) {
     return sizeof(T) * ((size_t)2 * b * (2 * b + 1) + 2 * b + 3 * b + nseg * 3 * b);
 }
 
-// Resident form when its workgroups, one per hop of the first sweep, all fit on the GPU at
-// once (each waits for both neighbours); *done tells whether it was launched.
-template <typename T, int B> int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, bool *done) {
+// Workgroups of the resident kernel that fit on the GPU together wherever the hardware puts
+// their waves: the occupancy query divides a CU's wave slots by a workgroup's waves, but a
+// workgroup of nine may take three of one SIMD's slots every time.
+template <typename T, int B, bool RECV> int chase_capacity(i64 *out) {
+    const void *k = reinterpret_cast<const void *>(bc_chase_resident_kernel<T, B, RECV>);
+    hipFuncAttributes fa;
+    CUEV_HIP(hipFuncGetAttributes(&fa, k));
+    int per_cu = 0;
+    CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bc_chase_resident_kernel<T, B, RECV>,
+                                                          chase_threads(B, RECV), 0));
+    const int simd_waves = std::min(8, 512 / std::max(8, (fa.numRegs + 7) / 8 * 8));
+    const int wg_waves = (chase_threads(B, RECV) / 64 + 3) / 4; // of one SIMD
+    *out = (i64)std::min(per_cu, simd_waves / wg_waves) * device_cu_count();
+    return CUEV_STATUS_SUCCESS;
+}
+
+template <typename T, int B, bool RECV>
+int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, int hops) {
     const int n = ws.n;
     hipStream_t s = ws.stream;
-    *done = false;
-    const int hops = (n - 2) / B + 1;
-    int per_cu = 0;
-    CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bc_chase_resident_kernel<T, B>, chase_threads(B), 0));
-    if (hops > per_cu * device_cu_count()) return CUEV_STATUS_SUCCESS;
     const i64 words = (i64)(hops + 1) * 2 * msg_words<T>(B);
     CUEV_TRY(fill_int(s, reinterpret_cast<int *>(ws.chmsg), 2 * words, 0)); // no tag of an earlier chase
     const double nhops = (double)n * n / (2.0 * B);
-    prof::Scope sc(s, "bc.chase", nhops * (6.0 * B * B + 16.0 * B * B), nhops * 4.0 * B * B * sizeof(T));
-    hipLaunchKernelGGL((bc_chase_resident_kernel<T, B>), dim3((unsigned)hops), dim3(chase_threads(B)), 0, s, Bp, ws.U,
-                       ws.ldu, n, d, e, reinterpret_cast<u64 *>(ws.chmsg), ws.err);
+    // each hop writes and reads two messages of b tagged values and writes b values of U
+    prof::Scope sc(s, "bc.chase", nhops * (6.0 * B * B + 16.0 * B * B), nhops * 9.0 * B * sizeof(T));
+    hipLaunchKernelGGL((bc_chase_resident_kernel<T, B, RECV>), dim3((unsigned)hops), dim3(chase_threads(B, RECV)), 0, s,
+                       Bp, ws.U, ws.ldu, n, d, e, reinterpret_cast<u64 *>(ws.chmsg), ws.err);
     CUEV_LAUNCH_CHECK();
+    return CUEV_STATUS_SUCCESS;
+}
+
+// Resident form when its workgroups, one per hop of the first sweep, all fit on the GPU at
+// once (each waits for both neighbours); *done tells whether it was launched. The form with
+// a receiving wave is taken where two such chases fit at once (b = 64 in FP64: n <= 16384;
+// two solves may share the GPU, as with the windowed form), the one without it, which has
+// more room, where one does (n <= 49152; at n = 16384 3.9 us per sweep, windowed 16.4).
+template <typename T, int B> int try_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, bool *done) {
+    const int hops = (ws.n - 2) / B + 1;
+    i64 with = 0, without = 0;
+    CUEV_TRY((chase_capacity<T, B, true>(&with)));
+    CUEV_TRY((chase_capacity<T, B, false>(&without)));
     *done = true;
+    if (2 * hops <= with) return launch_chase_resident<T, B, true>(ws, Bp, d, e, hops);
+    if (hops <= without) return launch_chase_resident<T, B, false>(ws, Bp, d, e, hops);
+    *done = false;
     return CUEV_STATUS_SUCCESS;
 }
 
@@ -915,9 +1005,9 @@ template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e) {
     if (n - 2 > 0) {
         bool done = false;
         switch (ws.b) {
-        case 16: CUEV_TRY((launch_chase_resident<T, 16>(ws, Bp, d, e, &done))); break;
-        case 32: CUEV_TRY((launch_chase_resident<T, 32>(ws, Bp, d, e, &done))); break;
-        case 64: CUEV_TRY((launch_chase_resident<T, 64>(ws, Bp, d, e, &done))); break;
+        case 16: CUEV_TRY((try_chase_resident<T, 16>(ws, Bp, d, e, &done))); break;
+        case 32: CUEV_TRY((try_chase_resident<T, 32>(ws, Bp, d, e, &done))); break;
+        case 64: CUEV_TRY((try_chase_resident<T, 64>(ws, Bp, d, e, &done))); break;
         default: CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "bc_chase: unsupported b=%d", ws.b);
         }
         if (done) return CUEV_STATUS_SUCCESS;

@@ -85,14 +85,6 @@ __device__ __forceinline__ double fast_rcp(double q) {
     r = fma(fma(-q, r, 1.0), r, r);
     return fma(fma(-q, r, 1.0), r, r);
 }
-// sqrt(h) and 1 / sqrt(h), h in [2^-1000, 2^1000]: v_rsq_f64, two Newton steps
-__device__ __forceinline__ void fast_sqrt(double h, double &r, double &ri) {
-    double y = __builtin_amdgcn_rsq(h);
-    y = fma(0.5 * y, fma(-h * y, y, 1.0), y);
-    const double t = h * y;
-    r = fma(0.5 * y, fma(-t, t, h), t);
-    ri = fma(y, fma(-r, y, 1.0), y);
-}
 __device__ __forceinline__ double guarded(double q) { return fabs(q) < 0x1p-200 ? -0x1p-200 : q; }
 
 // One QL sweep's bookkeeping on (d, e) of order n by one wave (every lane alike): the next

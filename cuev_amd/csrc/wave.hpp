@@ -73,5 +73,14 @@ __device__ __forceinline__ double read_lane(double v, int l) {
                             __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
+// sqrt(h) and 1 / sqrt(h), h in [2^-1000, 2^1000]: v_rsq_f64, two Newton steps
+__device__ __forceinline__ void fast_sqrt(double h, double &r, double &ri) {
+    double y = __builtin_amdgcn_rsq(h);
+    y = fma(0.5 * y, fma(-h * y, y, 1.0), y);
+    const double t = h * y;
+    r = fma(0.5 * y, fma(-t, t, h), t);
+    ri = fma(y, fma(-r, y, 1.0), y);
+}
+
 } // namespace cuev
 #endif
