@@ -25,6 +25,9 @@
 #include "panel_qr.hpp"
 
 #include <algorithm>
+#include <type_traits>
+
+#include "wave.hpp"
 
 namespace cuev {
 namespace {
@@ -88,12 +91,9 @@ __device__ __forceinline__ double ld_wt(const double *p) {
 __device__ __forceinline__ void st_wt(double *p, double v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool grid_barrier_wt(unsigned *counter, unsigned target, int *err) {
-    vm_drain();
-    __syncthreads();
+__device__ __forceinline__ bool grid_wait_wt(unsigned *counter, unsigned target, int *err) {
     __shared__ int s_ok;
     if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         long long it = 0;
         int ok = 1;
         while (counter_load_relaxed(counter) < target) {
@@ -109,6 +109,13 @@ __device__ __forceinline__ bool grid_barrier_wt(unsigned *counter, unsigned targ
     }
     __syncthreads();
     return s_ok != 0;
+}
+__device__ __forceinline__ bool grid_barrier_wt(unsigned *counter, unsigned target, int *err) {
+    vm_drain();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return grid_wait_wt(counter, target, err);
 }
 
 template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_kernel(PQArgs<T> a) {
@@ -355,13 +362,25 @@ template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_ker
 // Per pass: partial Gram -> global, grid barrier, each workgroup sums a slice of
 // the entries over all partials in a fixed order, grid barrier, then every
 // workgroup factors the same b x b Gram matrix redundantly (bit-identical
-// results everywhere), with X = L'^-1 alongside for P <- P R_p^-1. Workgroup 0 then
-// factors Q_1 and publishes U and Mw = -S L^-T (fifth barrier): every workgroup forms
-// its rows of W = Y T = (Q - [S; 0]) Mw and of Y = Q_2 U^-1 (by substitution along
-// its rows, four lanes per row), and workgroup 0 forms T = U Mw. The b x b factorizations keep the matrix in registers as 4x4 blocks
-// per thread and broadcast the pivot column/row through LDS: one LDS barrier per
-// elimination step. All arithmetic is FP64.
-constexpr int kCQThreads = 256;
+// results everywhere), its rows of P stacked under it: the column operations that
+// turn G into its Cholesky factor turn P into P R_p^-1, so no inverse is formed.
+// Workgroup 0 then factors Q_1 and publishes U^-1 and Mw = -S L^-T: every workgroup
+// forms its rows of W = Y T = (Q - [S; 0]) Mw and Y = Q_2 U^-1, workgroup 0 also
+// T = U Mw and R = R_2 R_1. All arithmetic is FP64.
+//
+// Bound: latency, of the two eliminations (b dependent pivots each) and of the grid
+// barriers. An elimination holds its matrix in registers, a row in each lane and the
+// columns in groups of four dealt out to the waves: the wave that owns the next group
+// brings it up to date, eliminates its four columns by itself (pivots and multipliers by
+// lane reads) and passes them on through LDS, so there is one barrier for four columns;
+// what the columns further right still miss is made up beside the next group. The products
+// run on the FP64 matrix cores. Measured at b = 64: 150 -> 60 us per panel, of which
+// the first elimination 14, Q_1's 20, both Gram matrices 3.7 and their sums 8, the second pass 3.2
+// and W, Y and the top rows 8 (with a barrier for every column, 4 x 4 blocks per thread, vector
+// products and explicit inverses: elimination and P R_1^-1 41, Q_1 33, Gram 9, second pass 16,
+// W and Y 25); at b = 32 80 -> 28.
+constexpr int kCQThreads = 512;
+constexpr int kCQWaves = kCQThreads / 64;
 constexpr int kCQMaxCH = 96;
 
 template <typename T> struct CQArgs {
@@ -374,185 +393,327 @@ template <typename T> struct CQArgs {
     T *Tm;
     T *tau;
     int rows, CH, G;
-    double *part; // [G][b*b] partial Gram matrices
-    double *gsum; // [b*b]
-    double *bc;   // [2*b*b]: U, then Mw = -S L^-T (column-major)
+    double *part; // [G][tiles * 256] partial Gram matrices
+    double *gsum; // [tiles * 256]
+    double *bc;   // [2*b*b]: U^-1 (column-major), then Mw = -S L^-T (row-major)
     int *gate;
     unsigned *counter;
     unsigned *reset; // the Householder kernel's barrier counter, zeroed for the launch after this one
     int *err;
 };
 
-// Packed lower-triangle index of (i, j), i >= j, of a B x B symmetric matrix.
-template <int B> __device__ __forceinline__ int cq_lo(int i, int j) { return i + j * B - (j * (j + 1)) / 2; }
+typedef double cq_v4 __attribute__((ext_vector_type(4)));
+// D += A B, 16 x 16 x 4: lane l holds A(l % 16, l / 16), B(l / 16, l % 16), D(l / 16 + 4 r, l % 16)
+__device__ __forceinline__ cq_v4 cq_mma(double a, double b, cq_v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
 
-// out (packed lower) = P^T P over the first nr rows (P column-major, ld CHp).
-// Thread = strided 4x4 block, rows ti + NB u and columns tj + NB v, so the 16
-// lanes with different ti read 16 different banks.
-template <int B>
-__device__ __forceinline__ void cq_gram(const double *P, int CHp, int nr, double *out, int tid) {
-    constexpr int NB = B / 4;
-    if (tid >= NB * NB) return;
-    const int ti = tid % NB, tj = tid / NB;
-    double acc[4][4];
+// Panel slice in LDS: element (r, c) at c * ld + r. A half wave's fragment read is 16 rows of two
+// columns, or two rows of 16 columns (P^T P): a leading dimension of 18 modulo 32 spreads both
+// over the banks (16 would put the second on four of 64). The b x b matrices, read two rows of 16
+// columns at a time, have b + 2.
+__host__ __device__ constexpr int cq_ldp(int CH) { return CH + (50 - CH % 32) % 32; }
+
+// lower 16 x 16 tile q of a Gram matrix, row by row
+__device__ __forceinline__ void cq_tile(int q, int &I, int &J) {
+    I = q >= 6 ? 3 : (q >= 3 ? 2 : (q >= 1 ? 1 : 0));
+    J = q - I * (I + 1) / 2;
+}
+
+// out (lower tiles, each as the accumulator's four registers x 64 lanes) = P^T P
+template <int B> __device__ __forceinline__ void cq_gram(const double *P, int ldp, int CH, double *out, int wave, int lane) {
+    constexpr int NT = (B / 16) * (B / 16 + 1) / 2;
+    const int lr = lane & 15, lk = lane >> 4;
+    for (int q = wave; q < NT; q += kCQWaves) {
+        int I, J;
+        cq_tile(q, I, J);
+        const double *x = P + (size_t)(16 * I + lr) * ldp + lk, *y = P + (size_t)(16 * J + lr) * ldp + lk;
+        cq_v4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+        for (int r = 0; r < CH; r += 16) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-    for (int r = 0; r < nr; ++r) {
-        double x[4], y[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            x[u] = P[(size_t)(ti + NB * u) * CHp + r];
-            y[u] = P[(size_t)(tj + NB * u) * CHp + r];
+            for (int u = 0; u < 4; ++u) acc[u & 1] = cq_mma(x[r + 4 * u], y[r + 4 * u], acc[u & 1]);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[u][v] += x[u] * y[v];
+        for (int u = 0; u < 4; ++u) st_wt(out + q * 256 + u * 64 + lane, acc[0][u] + acc[1][u]);
     }
+}
+
+// 1 / sqrt(h), h in [1e-290, 1e290], and 1 / p, |p| in [1, 2^1000]: one step of third order from
+// the instruction's 24 bits or more
+__device__ __forceinline__ double cq_rsqrt(double h) {
+    const double y = __builtin_amdgcn_rsq(h), e = fma(-h * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double cq_rcp(double p) {
+    const double r = __builtin_amdgcn_rcp(p), e = fma(-p, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+
+// Columns of a b-column matrix held by the waves: group c (columns 4 c .. 4 c + 3) in wave
+// c % kCQWaves, as its local group c / kCQWaves.
+template <int B> struct CQCols {
+    static constexpr int NCH = B / 4;                                        // groups
+    static constexpr int LC = NCH <= kCQWaves ? 1 : NCH / kCQWaves;          // local groups
+    static constexpr int NC = 4 * LC;                                        // local columns
+};
+
+// Drives an elimination over the groups. factor(lc, c): the wave eliminates its local group
+// lc = group c and writes it to buffer c % 3; load(c): reads group c from its buffer; apply(lc,
+// c): brings local group lc up to date with the group read; rest(lc, c): other work on group
+// c for local group lc that nothing waits for (the group's own columns included). A wave that
+// has just eliminated group c + 1 leaves its other columns until the next step, beside the next
+// wave's elimination.
+template <int LC, typename F> __device__ __forceinline__ void cq_each(F &&f) {
+    static_assert(LC <= 2, "local groups");
+    f(std::integral_constant<int, 0>{});
+    if constexpr (LC > 1) f(std::integral_constant<int, 1>{});
+}
+template <int B, typename Fa, typename Lo, typename Ap, typename Re>
+__device__ __forceinline__ void cq_eliminate(int wave, Fa &&factor, Lo &&load, Ap &&apply, Re &&rest) {
+    using C = CQCols<B>;
+    if (wave == 0) factor(std::integral_constant<int, 0>{}, 0);
+    int done = 0; // groups whose other work is done
+#pragma unroll 1
+    for (int c = 0; c < C::NCH; ++c) {
+        __syncthreads(); // group c is in its buffer
+        if (c + 1 < C::NCH && (c + 1) % kCQWaves == wave) {
+            __builtin_amdgcn_s_setprio(3); // before the other wave of this SIMD
+            load(c);
+            cq_each<C::LC>([&](auto lc) {
+                if (kCQWaves * lc() + wave == c + 1) {
+                    apply(lc, c);
+                    factor(lc, c + 1);
+                }
+            });
+            __builtin_amdgcn_s_setprio(0);
+            continue;
+        }
+#pragma unroll 1
+        for (; done <= c; ++done) {
+            load(done);
+            cq_each<C::LC>([&](auto lc) {
+                const int own = kCQWaves * lc() + wave;
+                if (own > done + 1 && own < C::NCH) apply(lc, done);
+                if (own < C::NCH) rest(lc, done);
+            });
+        }
+    }
+    __syncthreads(); // the buffers are free
+}
+
+// Cholesky factor of the b x b Gram matrix Gm (LDS, full, ld b + 2) with the panel rows below
+// it: P <- P R^-1 in place; R (upper, column-major, ld b + 2) into Rout if it is set. False in
+// every thread if a pivot falls below tol of its diagonal entry or is not finite.
+template <int B, int NSET>
+__device__ __forceinline__ bool cq_chol(double *P, int ldp, int CH, const double *Gm, double *buf, double *Rout,
+                                        double tol, int *s_bad, int wave, int lane) {
+    using C = CQCols<B>;
+    constexpr int LD = B + 2, NR = 64 * NSET;
+    double g[NSET][C::NC];
+    // row q = 64 t + lane of [G; P]
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int lc = 0; lc < C::LC; ++lc)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * (kCQWaves * lc + wave) + u;
+#pragma unroll
+            for (int t = 0; t < NSET; ++t) {
+                const int q = 64 * t + lane;
+                double v = 0.0;
+                if (j < B && q < B) v = Gm[q + j * LD];
+                else if (j < B && q < B + CH) v = P[(size_t)j * ldp + q - B];
+                g[t][4 * lc + u] = v;
+            }
+        }
+    const double diag = lane < B ? Gm[lane + lane * LD] : 0.0;
+    double piv[C::NC], l[4][NSET];
+    auto factor = [&](auto lcc, int c) {
+        constexpr int lc = decltype(lcc)::value;
+        double *dst = buf + (size_t)(c % 3) * 4 * NR + lane;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int i = ti + NB * u, j = tj + NB * v;
-            if (i >= j) st_wt(out + cq_lo<B>(i, j), acc[u][v]);
+            const int k = 4 * c + v;
+            const double dk = read_lane(g[0][4 * lc + v], k), rs = cq_rsqrt(dk);
+            piv[4 * lc + v] = dk; // looked at afterwards
+            double w[NSET]; // in G's rows above k: what rounding left of zero, read by no one
+#pragma unroll
+            for (int t = 0; t < NSET; ++t) w[t] = g[t][4 * lc + v] *= rs;
+#pragma unroll
+            for (int u = v + 1; u < 4; ++u) {
+                const double m = read_lane(w[0], 4 * c + u);
+#pragma unroll
+                for (int t = 0; t < NSET; ++t) g[t][4 * lc + u] -= w[t] * m;
+            }
+#pragma unroll
+            for (int t = 0; t < NSET; ++t) dst[v * NR + 64 * t] = w[t];
         }
-}
-
-// acc = X Y for B x B LDS matrices (column-major, ld B + 1; XT: X transposed),
-// thread = strided 4x4 block (ti + NB u, tj + NB v).
-template <int B, bool XT>
-__device__ __forceinline__ void cq_mm(double (&acc)[4][4], const double *X, const double *Y, int ti, int tj) {
-    constexpr int NB = B / 4, LD = B + 1;
+    };
+    auto load = [&](int c) {
+        const double *src = buf + (size_t)(c % 3) * 4 * NR + lane;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+        for (int v = 0; v < 4; ++v)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-    for (int k = 0; k < B; ++k) {
-        double x[4], y[4];
+            for (int t = 0; t < NSET; ++t) l[v][t] = src[v * NR + 64 * t];
+    };
+    auto apply = [&](auto lcc, int) {
+        constexpr int lc = decltype(lcc)::value;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int i = ti + NB * u;
-            x[u] = XT ? X[k + i * LD] : X[i + k * LD];
-            y[u] = Y[k + (tj + NB * u) * LD];
-        }
+            const int j = 4 * (kCQWaves * lc + wave) + u;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+            for (int v = 0; v < 4; ++v) {
+                const double m = read_lane(l[v][0], j);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[u][v] += x[u] * y[v];
-    }
-}
-
-// P[rows r0..r1) <- P U for an upper-triangular U (LDS, column-major, ld B + 1), in
-// place: rounds of whole 4-row blocks, all column blocks of a row block in the
-// same round (a row's new values depend on that row only). Columns are strided
-// over threads (tj + NB v) so the U reads of a wave spread over the banks.
-template <int B>
-__device__ __forceinline__ void cq_trmm(double *P, int CHp, int r0, int r1, const double *U, int tid) {
-    constexpr int NB = B / 4, LD = B + 1;
-    constexpr int RB_PER_ROUND = kCQThreads / NB;
-    const int nrb = (r1 - r0 + 3) / 4;
-    for (int rb0 = 0; rb0 < nrb; rb0 += RB_PER_ROUND) {
-        const int rb = rb0 + tid / NB, tj = tid % NB;
-        const bool act = rb < nrb;
-        double acc[4][4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-        const int rr = r0 + 4 * rb;
-        if (act) {
-            const int imax = tj + NB * 3; // U(i, j) = 0 for i > j
-            for (int i = 0; i <= imax; ++i) {
-                double x[4], w[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) x[u] = P[(size_t)i * CHp + rr + u];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) w[v] = U[i + (tj + NB * v) * LD];
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[u][v] += x[u] * w[v];
+                for (int t = 0; t < NSET; ++t) g[t][4 * lc + u] -= l[v][t] * m;
             }
         }
-        __syncthreads();
-        if (act)
+    };
+    cq_eliminate<B>(wave, factor, load, apply, [](auto, int) {});
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+    for (int lc = 0; lc < C::LC; ++lc)
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (rr + u < r1) P[(size_t)(tj + NB * v) * CHp + rr + u] = acc[u][v];
-        __syncthreads();
-    }
-}
-
-// P[r, :] <- P[r, :] U^-1 for the rows r0 <= r < r1, in place: forward substitution along
-// each row, four lanes per row (a quad of one wave) and 64 rows per round. The columns go
-// in blocks of 16, lane q of a quad holding columns 16J + 4q .. 16J + 4q + 3 of block J:
-// the block's columns first take the contributions of the finished blocks (read back from
-// P), then are finished one by one, each broadcast within the quad by a lane shuffle. U is
-// upper triangular in LDS (column-major, ld B + 1) and rd[j] = 1 / U(j, j). A row's values
-// are written and read back by its own quad only, so no workgroup barrier is needed until
-// the end.
-template <int B>
-__device__ __forceinline__ void cq_rsolve(double *P, int CHp, int r0, int r1, const double *U, const double *rd,
-                                          int tid) {
-    static_assert(B % 16 == 0 && kCQThreads == 256, "row solve layout");
-    constexpr int LD = B + 1;
-    const int q = tid & 3, lane = tid & 63;
-    for (int rb = r0; rb < r1; rb += kCQThreads / 4) {
-        const int r = rb + (tid >> 2);
-        const bool act = r < r1;
-#pragma unroll 1
-        for (int J = 0; J < B / 16; ++J) {
-            const int jb = 16 * J + 4 * q; // this lane's first column of the block
-            double acc[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[c] = act ? P[(size_t)(jb + c) * CHp + r] : 0.0;
-            for (int k = 0; k < 16 * J; ++k) {
-                const double y = act ? P[(size_t)k * CHp + r] : 0.0;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[c] -= y * U[k + (jb + c) * LD];
-            }
-#pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const int qt = t >> 2, ct = t & 3, kt = 16 * J + t;
-                const double mine = (q == qt) ? acc[ct] * rd[kt] : 0.0;
-                const double y = __shfl(mine, (lane & ~3) + qt, 64);
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if (4 * q + c > t) acc[c] -= y * U[kt + (jb + c) * LD];
-                if (q == qt && act) P[(size_t)kt * CHp + r] = y;
-            }
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * (kCQWaves * lc + wave) + u;
+            const double d = piv[4 * lc + u];
+            if (j < B && !(d > tol * read_lane(diag, j) && d > 1e-290 && d < 1e290)) *s_bad = 1;
         }
-    }
     __syncthreads();
+    if (*s_bad) return false;
+#pragma unroll
+    for (int lc = 0; lc < C::LC; ++lc)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * (kCQWaves * lc + wave) + u;
+#pragma unroll
+            for (int t = 0; t < NSET; ++t) {
+                const int q = 64 * t + lane;
+                if (j < B && q < B) {
+                    if (Rout) Rout[j + q * LD] = q < j ? 0.0 : g[t][4 * lc + u];
+                } else if (j < B && q < B + CH) P[(size_t)j * ldp + q - B] = g[t][4 * lc + u];
+            }
+        }
+    __syncthreads();
+    return true;
 }
 
-template <typename T, int B> __global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
+// Workgroup 0: Q_1 - S = L U for the top b rows of P, with L^-1 (row operations on I) and U^-1
+// (column operations on I) alongside. L and U into LU (packed, ld b + 2; its memory, buf, is
+// free before), U^-1 and Mw to bc, S to sv and into P's diagonal (Q_1 - S).
+template <int B>
+__device__ __forceinline__ void cq_lu(double *P, int ldp, double *LU, double *buf, double *bc, double *sv, int wave,
+                                      int lane) {
+    using C = CQCols<B>;
+    constexpr int LD = B + 2;
+    double m[C::NC], x[C::NC], z[C::NC], sg[C::NC];
+#pragma unroll
+    for (int lc = 0; lc < C::LC; ++lc)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * (kCQWaves * lc + wave) + u, q = 4 * lc + u;
+            m[q] = (j < B && lane < B) ? P[(size_t)j * ldp + lane] : 0.0;
+            x[q] = z[q] = lane == j ? 1.0 : 0.0;
+            sg[q] = 1.0;
+        }
+    double l[4], xk[4];
+    auto factor = [&](auto lcc, int c) {
+        constexpr int lc = decltype(lcc)::value;
+        double *dst = buf + (size_t)(c % 3) * 512 + lane;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int k = 4 * c + v, q = 4 * lc + v;
+            const double mkk = read_lane(m[q], k);
+            const double s = (mkk >= 0.0) ? -1.0 : 1.0;
+            const double piv = mkk - s, rp = cq_rcp(piv);
+            const double w = lane > k ? m[q] * rp : 0.0;
+            sg[q] = s;
+            m[q] = lane > k ? w : m[q];
+            x[q] *= rp;
+#pragma unroll
+            for (int u = v + 1; u < 4; ++u) {
+                const double mu = read_lane(m[4 * lc + u], k);
+                m[4 * lc + u] -= w * mu;
+                x[4 * lc + u] -= x[q] * mu;
+            }
+            dst[v * 64] = w;
+            dst[256 + v * 64] = x[q];
+        }
+    };
+    auto load = [&](int c) {
+        const double *src = buf + (size_t)(c % 3) * 512 + lane;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            l[v] = src[v * 64];
+            xk[v] = src[256 + v * 64];
+        }
+    };
+    auto apply = [&](auto lcc, int c) {
+        constexpr int lc = decltype(lcc)::value;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double mu = read_lane(m[4 * lc + u], 4 * c + v);
+                m[4 * lc + u] -= l[v] * mu;
+                x[4 * lc + u] -= xk[v] * mu;
+            }
+    };
+    auto rest = [&](auto lcc, int c) {
+        constexpr int lc = decltype(lcc)::value;
+        if (kCQWaves * lc + wave > c) return; // columns of L^-1 that are still those of I
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) z[4 * lc + u] -= l[v] * read_lane(z[4 * lc + u], 4 * c + v);
+    };
+    cq_eliminate<B>(wave, factor, load, apply, rest);
+#pragma unroll
+    for (int lc = 0; lc < C::LC; ++lc)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * (kCQWaves * lc + wave) + u, q = 4 * lc + u;
+            if (j < B && lane < B) {
+                st_wt(bc + lane + j * B, x[q]);
+                st_wt(bc + B * B + lane + j * B, -sg[q] * z[q]); // Mw(j, lane) = -s_j L^-1(lane, j)
+                LU[lane + j * LD] = lane == j ? m[q] - sg[q] : m[q];
+                if (lane == j) {
+                    sv[j] = sg[q];
+                    P[(size_t)j * ldp + j] -= sg[q];
+                }
+            }
+        }
+}
+
+// acc = tile (I, J), I <= J, of X Y for upper triangular X and Y (column-major, ld b + 2;
+// entries of X below its diagonal are not read as zeros but masked)
+template <int B> __device__ __forceinline__ cq_v4 cq_upper_mm(const double *X, const double *Y, int I, int J, cq_v4 acc, int lane) {
+    constexpr int LD = B + 2;
+    const int lr = lane & 15, lk = lane >> 4, i = 16 * I + lr;
+    for (int k0 = 16 * I; k0 < 16 * (J + 1); k0 += 4) {
+        const int k = k0 + lk;
+        acc = cq_mma(k >= i ? X[i + k * LD] : 0.0, Y[k + (16 * J + lr) * LD], acc);
+    }
+    return acc;
+}
+
+template <typename T, int B, int NSET>
+__global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    constexpr int NB = B / 4, LD = B + 1, BB = B * B, BL = B * (B + 1) / 2;
-    const int CH = a.CH, CHp = CH + 1;
-    const int tid = threadIdx.x, g = blockIdx.x;
-    const bool own = tid < NB * NB;
-    // contiguous 4x4 blocks (4 ti + u, 4 tj + v) for the factorizations, strided
-    // (si + NB u, sj + NB v) for the products
-    const int ti = own ? tid % NB : 0, tj = own ? tid / NB : 0;
-    const int si = ti, sj = tj;
-    double *P = reinterpret_cast<double *>(smem_raw); // [B][CHp]: panel(r, c) at P[c*CHp + r]
-    double *M1 = P + (size_t)B * CHp;                 // [B][LD] column-major
-    double *M2 = M1 + B * LD;
-    double *M3 = M2 + B * LD;
-    double *cb = M3 + B * LD; // [2][B] broadcast: pivot column
-    double *rb = cb + 2 * B;  // [2][B] broadcast: pivot row
-    double *xb = rb + 2 * B;  // [2][B] broadcast: row of the inverse
-    double *dv = xb + 2 * B;  // [B] pivots
-    double *gd = dv + B;      // [B] Gram diagonal before the factorization
-    double *sv = gd + B;      // [B] signs S
-    double *red = sv + B;     // [kCQThreads]
+    constexpr int LD = B + 2, BB = B * B, NTB = B / 16, NT = NTB * (NTB + 1) / 2, NE = 256 * NT;
+    constexpr int NP = NTB > 2 ? NTB / 2 : 1; // pairs of column tiles {p, NTB - 1 - p}: equal work for triangular factors
+    constexpr int KC = (B * LD > 768 * NSET) ? B * LD : 768 * NSET;
+    const int CH = a.CH, ldp = cq_ldp(CH);
+    const int tid = threadIdx.x, lane = tid & 63, g = blockIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    double *P = reinterpret_cast<double *>(smem_raw); // [B][ldp]: panel(r, c) at P[c * ldp + r]
+    double *MA = P + (size_t)B * ldp;                 // [B][LD]: Gram matrix; F or R_2; U^-1
+    double *MB = MA + B * LD;                         // [B][LD]: R_1; Mw
+    double *MC = MB + B * LD;                         // [KC]: column groups of the eliminations; L and U
+    double *sv = MC + KC;                             // [B] signs S
+    int *s_bad = reinterpret_cast<int *>(sv + B);     // [2]
 
     if (g == 0 && tid == 0) __hip_atomic_store(a.reset, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid < 2) s_bad[tid] = 0;
     const int r0g = g * CH;
     const int chl = max(0, min(CH, a.rows - r0g));
     {
@@ -570,20 +731,24 @@ template <typename T, int B> __global__ __launch_bounds__(kCQThreads) void panel
             for (int q = 0; q < LB; ++q) {
                 const int idx = base + q * kCQThreads + tid;
                 const int j = idx / CH, rl = idx - j * CH;
-                if (idx < B * CH) P[(size_t)j * CHp + rl] = v[q];
+                if (idx < B * CH) P[(size_t)j * ldp + rl] = v[q];
             }
         }
     }
     __syncthreads();
 
+    // tasks of the products with a panel slice: (row tile, pair of column tiles), round robin
+    const int ntask = (CH / 16) * NP;
+    bool tiny = false;
     unsigned nbar = 0;
+#pragma unroll 1
     for (int pass = 0; pass < 2; ++pass) {
         // ---- Gram matrix of the panel: partials, then fixed-order slice sums
-        cq_gram<B>(P, CHp, chl, a.part + (size_t)g * BL, tid);
+        cq_gram<B>(P, ldp, CH, a.part + (size_t)g * NE, wave, lane);
         if (!grid_barrier_wt(a.counter, (unsigned)a.G * ++nbar, a.err)) return;
         {
-            const int S = (BL + a.G - 1) / a.G;
-            const int e0 = g * S, ne = max(0, min(BL, e0 + S) - e0);
+            const int S = (NE + a.G - 1) / a.G;
+            const int e0 = g * S, ne = max(0, min(NE, e0 + S) - e0);
             int tpe = 1; // threads per entry (power of two)
             while (tpe < 64 && tpe * 2 * max(ne, 1) <= kCQThreads) tpe *= 2;
             const int per_round = kCQThreads / tpe;
@@ -597,389 +762,210 @@ template <typename T, int B> __global__ __launch_bounds__(kCQThreads) void panel
 #pragma unroll
                         for (int u = 0; u < 16; ++u) {
                             const int gg = g0 + u * tpe;
-                            v[u] = (gg < a.G) ? ld_wt(src + (size_t)gg * BL) : 0.0;
+                            v[u] = (gg < a.G) ? ld_wt(src + (size_t)gg * NE) : 0.0;
                         }
 #pragma unroll
                         for (int u = 0; u < 16; ++u) s += v[u];
                     }
                 }
-                red[tid] = s;
-                __syncthreads();
-                if (el < ne && pt == 0) {
-                    double t = 0.0;
-                    for (int q = 0; q < tpe; ++q) t += red[tid + q];
-                    st_wt(a.gsum + e0 + el, t);
-                }
-                __syncthreads();
+                for (int d = tpe / 2; d > 0; d /= 2) s += __shfl_xor(s, d, 64);
+                if (el < ne && pt == 0) st_wt(a.gsum + e0 + el, s);
             }
         }
         if (!grid_barrier_wt(a.counter, (unsigned)a.G * ++nbar, a.err)) return;
 
-        // ---- second pass, G = I + E with E tiny (the usual case): R_2 = I + F,
-        // F = up(E - up(E)^T up(E)) with up(M) = strict upper of M + diag(M)/2,
-        // leaves R_2^T R_2 - G = O(|E|^3); R_2^-1 = I - F + F^2 + O(|F|^3)
-        if (pass == 1) {
-            double e[4][4];
-            double emax = 0.0;
+        {
+            double v[(NE + kCQThreads - 1) / kCQThreads];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int i = si + NB * u, j = sj + NB * v;
-                    const double gij = own ? ld_wt(a.gsum + ((i >= j) ? cq_lo<B>(i, j) : cq_lo<B>(j, i))) : 0.0;
-                    e[u][v] = own ? gij - (i == j ? 1.0 : 0.0) : 0.0;
-                    emax = fmax(emax, fabs(e[u][v]));
-                    if (own) M2[i + j * LD] = (i < j) ? e[u][v] : (i == j ? 0.5 * e[u][v] : 0.0);
-                }
-            red[tid] = (emax == emax) ? emax : 1.0; // NaN -> not small
-            __syncthreads();
-            for (int s2 = kCQThreads / 2; s2 > 0; s2 >>= 1) {
-                if (tid < s2) red[tid] = fmax(red[tid], red[tid + s2]);
-                __syncthreads();
+            for (int q = 0; q < (NE + kCQThreads - 1) / kCQThreads; ++q) {
+                const int idx = q * kCQThreads + tid;
+                v[q] = idx < NE ? ld_wt(a.gsum + idx) : 0.0;
             }
-            // |E| <= 1e-10 entrywise (the usual case): up(E)^T up(E) and F^2 have entries
-            // below B 1e-20, under half an ulp of R_2's unit diagonal, so F = up(E) and
-            // R_2^-1 = I - F, and only F R_1 is formed
-            const bool small = red[0] <= 1e-6, tiny = red[0] <= 1e-10;
-            __syncthreads();
-            if (small) {
-                if (!tiny) {
-                    double c[4][4];
-                    cq_mm<B, true>(c, M2, M2, si, sj); // up(E)^T up(E)
-                    __syncthreads();
-                    if (own)
+            auto place = [&](bool second) {
+#pragma unroll
+                for (int q = 0; q < (NE + kCQThreads - 1) / kCQThreads; ++q) {
+                    const int idx = q * kCQThreads + tid;
+                    if (idx >= NE) continue;
+                    int I, J;
+                    cq_tile(idx >> 8, I, J);
+                    const int i = 16 * I + 4 * ((idx >> 6) & 3) + ((idx & 63) >> 4), j = 16 * J + (idx & 15);
+                    if (!second) { // G
+                        MA[i + j * LD] = v[q];
+                        if (I != J) MA[j + i * LD] = v[q];
+                        continue;
+                    }
+                    // second pass: G = I + E with E tiny (the usual case): R_2 = I + F, R_2^-1 = I - F,
+                    // F = up(E) = strict upper of E + diag(E) / 2. |E| <= 1e-10 entrywise: up(E)^T
+                    // up(E) and F^2 have entries below b 1e-20, under half an ulp of the diagonal
+                    const double e = v[q] - (i == j ? 1.0 : 0.0);
+                    if (!(fabs(e) <= 1e-10)) s_bad[1] = 1;
+                    MA[i + j * LD] = I != J || i > j ? 0.0 : (i < j ? e : 0.5 * e);
+                    if (I != J) MA[j + i * LD] = e;
+                }
+                __syncthreads();
+            };
+            place(pass == 1);
+            tiny = pass == 1 && s_bad[1] == 0;
+            if (pass == 1 && !tiny) {
+                __syncthreads();
+                place(false);
+            }
+        }
+        if (tiny) {
+            // P <- P - P F, transposed (16 rows of one column in 16 lanes)
+            for (int t0 = 0; t0 < ntask; t0 += kCQWaves) {
+                const int t = t0 + wave, I = t / NP, pr = t % NP;
+                cq_v4 acc[2];
+                if (t < ntask) {
+                    const int Jt[2] = {pr, NTB - 1 - pr};
+#pragma unroll
+                    for (int c = 0; c < (NTB > 1 ? 2 : 1); ++c)
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
+                            acc[c][u] = P[(size_t)(16 * Jt[c] + 4 * u + lk) * ldp + 16 * I + lr];
+                    for (int k0 = 0; k0 < 16 * (Jt[1] + 1); k0 += 4) {
+                        const double x = P[(size_t)(k0 + lk) * ldp + 16 * I + lr];
 #pragma unroll
-                            for (int v = 0; v < 4; ++v) {
-                                const int i = si + NB * u, j = sj + NB * v;
-                                const double f = e[u][v] - c[u][v];
-                                M2[i + j * LD] = (i < j) ? f : (i == j ? 0.5 * f : 0.0);
-                            }
-                    __syncthreads();
-                }
-                double f2[4][4], fr[4][4];
-                if (!tiny) {
-                    cq_mm<B, false>(f2, M2, M2, si, sj); // F^2
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) f2[u][v] = 0.0;
-                }
-                cq_mm<B, false>(fr, M2, M1, si, sj); // F R_1
-                double fo[4][4], r1[4][4];
-                if (own)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const int i = si + NB * u, j = sj + NB * v;
-                            fo[u][v] = M2[i + j * LD];
-                            r1[u][v] = M1[i + j * LD];
-                        }
-                __syncthreads();
-                if (own)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const int i = si + NB * u, j = sj + NB * v;
-                            M2[i + j * LD] = (i == j ? 1.0 : 0.0) - fo[u][v] + f2[u][v]; // R_2^-1
-                            M1[i + j * LD] = r1[u][v] + fr[u][v];                         // R_2 R_1
-                        }
-                __syncthreads();
-                cq_trmm<B>(P, CHp, 0, CH, M2, tid);
-                continue;
-            }
-        }
-
-        // ---- G = L' D L'^T with X = L'^-1 (registers), R_p = D^1/2 L'^T. Each step
-        // applies masked multiplier vectors to all 16 entries of a thread's block.
-        double gr[4][4], xr[4][4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = 4 * ti + u, j = 4 * tj + v;
-                gr[u][v] = own ? ld_wt(a.gsum + ((i >= j) ? cq_lo<B>(i, j) : cq_lo<B>(j, i))) : 0.0;
-                xr[u][v] = (i == j) ? 1.0 : 0.0;
-            }
-        double *Rout = (pass == 0) ? M1 : M3;
-        if (tid < B) gd[tid] = ld_wt(a.gsum + cq_lo<B>(tid, tid));
-        if (own && tj == 0)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) cb[4 * ti + u] = gr[u][0];
-        if (own && ti == 0)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) xb[4 * tj + v] = xr[0][v];
-        const double tol = (pass == 0) ? 1e-10 : 1e-3;
-        bool ok = true;
-        for (int kb = 0; kb < NB && ok; ++kb) {
-#pragma unroll
-            for (int v0 = 0; v0 < 4; ++v0) {
-                const int k = 4 * kb + v0, p = k & 1;
-                __syncthreads();
-                const double dk = cb[p * B + k];
-                if (!(dk > tol * gd[k]) || !(dk < 1e300)) {
-                    ok = false;
-                    break;
-                }
-                const double rk = 1.0 / dk, sq = sqrt(dk), rs = 1.0 / sq;
-                double ci[4], cim[4], cjm[4], xk[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    ci[u] = cb[p * B + 4 * ti + u];
-                    cim[u] = (4 * ti + u > k) ? ci[u] : 0.0;
-                    const double cj = cb[p * B + 4 * tj + u];
-                    cjm[u] = (4 * tj + u > k) ? cj * rk : 0.0;
-                    xk[u] = xb[p * B + 4 * tj + u];
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const double lx = cim[u] * rk;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        gr[u][v] -= cim[u] * cjm[v];
-                        xr[u][v] -= lx * xk[v];
+                        for (int c = 0; c < (NTB > 1 ? 2 : 1); ++c)
+                            if (k0 < 16 * (Jt[c] + 1))
+                                acc[c] = cq_mma(-MA[k0 + lk + (16 * Jt[c] + lr) * LD], x, acc[c]);
                     }
                 }
-                if (tid == 0) dv[k] = dk;
-                if (own && tj == 0)
+                __syncthreads();
+                if (t < ntask) {
+                    const int Jt[2] = {pr, NTB - 1 - pr};
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int i = 4 * ti + u;
-                        Rout[k + i * LD] = (i > k) ? ci[u] * rs : (i == k ? sq : 0.0);
-                    }
-                const int kn = k + 1, vn = (v0 + 1) & 3, bn = kn >> 2;
-                if (kn < B) {
-                    if (own && tj == bn)
+                    for (int c = 0; c < (NTB > 1 ? 2 : 1); ++c)
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) cb[(kn & 1) * B + 4 * ti + u] = gr[u][vn];
-                    if (own && ti == bn)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) xb[(kn & 1) * B + 4 * tj + v] = xr[vn][v];
+                        for (int u = 0; u < 4; ++u)
+                            P[(size_t)(16 * Jt[c] + 4 * u + lk) * ldp + 16 * I + lr] = acc[c][u];
                 }
             }
-        }
-        if (!ok) {
+            __syncthreads();
+        } else if (!cq_chol<B, NSET>(P, ldp, CH, MA, MC, g == 0 ? (pass == 0 ? MB : MA) : nullptr, pass == 0 ? 1e-10 : 1e-3,
+                                     s_bad, wave, lane)) {
             if (g == 0 && tid == 0) *a.gate = 1;
             return; // every workgroup takes the same decision
         }
-        // R_p^-1 (i, j) = X(j, i) / sqrt(d_j) into M2
-        __syncthreads();
-        if (own)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    M2[(4 * tj + v) + (4 * ti + u) * LD] = xr[u][v] / sqrt(dv[4 * ti + u]);
-        __syncthreads();
-        cq_trmm<B>(P, CHp, 0, CH, M2, tid);
-        if (pass == 1) {
-            // R = R_2 R_1 into M1
-            double acc[4][4];
-            cq_mm<B, false>(acc, M3, M1, si, sj);
-            __syncthreads();
-            if (own)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) M1[(si + NB * u) + (sj + NB * v) * LD] = acc[u][v];
-            __syncthreads();
-        }
     }
 
-    // ---- workgroup 0: Q_1 - S = L U (signs chosen on the way), L^-1, T, U^-1
     if (g == 0) {
-        double mr[4][4], xr[4][4];
+        cq_lu<B>(P, ldp, MC, MC, a.bc, sv, wave, lane);
+        if (tid == 0) *a.gate = 0;
+        vm_drain();
+        __syncthreads();
+        if (tid == 0) __hip_atomic_fetch_add(a.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // R = R_2 R_1, or R_1 + F R_1, into MA
+        cq_v4 acc[(NT + kCQWaves - 1) / kCQWaves];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int q = 0; q < (NT + kCQWaves - 1) / kCQWaves; ++q) {
+            const int t = wave + kCQWaves * q;
+            if (t >= NT) continue;
+            int I, J;
+            cq_tile(t, J, I); // upper tiles
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                mr[u][v] = own ? P[(size_t)(4 * tj + v) * CHp + 4 * ti + u] : 0.0;
-                xr[u][v] = (4 * ti + u == 4 * tj + v) ? 1.0 : 0.0;
-            }
-        if (own && tj == 0)
+            for (int u = 0; u < 4; ++u) acc[q][u] = tiny ? MB[16 * I + 4 * u + lk + (16 * J + lr) * LD] : 0.0;
+            acc[q] = cq_upper_mm<B>(MA, MB, I, J, acc[q], lane);
+        }
+        __syncthreads();
 #pragma unroll
-            for (int u = 0; u < 4; ++u) cb[4 * ti + u] = mr[u][0];
-        if (own && ti == 0)
+        for (int q = 0; q < (NT + kCQWaves - 1) / kCQWaves; ++q) {
+            const int t = wave + kCQWaves * q;
+            if (t >= NT) continue;
+            int I, J;
+            cq_tile(t, J, I);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                rb[4 * tj + v] = mr[0][v];
-                xb[4 * tj + v] = xr[0][v];
-            }
-        double *Lm = M2, *Um = M3; // unit-lower L, upper U (column-major)
-        for (int kb = 0; kb < NB; ++kb) {
-#pragma unroll
-            for (int v0 = 0; v0 < 4; ++v0) {
-                const int k = 4 * kb + v0, p = k & 1;
-                __syncthreads();
-                const double mkk = cb[p * B + k];
-                const double s = (mkk >= 0.0) ? -1.0 : 1.0;
-                const double piv = mkk - s, rp = 1.0 / piv;
-                double li[4], lim[4], rj[4], rjm[4], xk[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    li[u] = cb[p * B + 4 * ti + u] * rp;
-                    lim[u] = (4 * ti + u > k) ? li[u] : 0.0;
-                    rj[u] = rb[p * B + 4 * tj + u];
-                    rjm[u] = (4 * tj + u > k) ? rj[u] : 0.0;
-                    xk[u] = xb[p * B + 4 * tj + u]; // X(k, j) = 0 for j > k
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        mr[u][v] -= lim[u] * rjm[v];
-                        xr[u][v] -= lim[u] * xk[v];
-                    }
-                if (tid == 0) {
-                    sv[k] = s;
-                    dv[k] = piv;
-                }
-                if (own && tj == 0)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int i = 4 * ti + u;
-                        Lm[i + k * LD] = (i > k) ? li[u] : (i == k ? 1.0 : 0.0);
-                    }
-                if (own && ti == 0)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int j = 4 * tj + v;
-                        Um[k + j * LD] = (j > k) ? rj[v] : (j == k ? piv : 0.0);
-                    }
-                const int kn = k + 1, vn = (v0 + 1) & 3, bn = kn >> 2;
-                if (kn < B) {
-                    if (own && tj == bn)
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) cb[(kn & 1) * B + 4 * ti + u] = mr[u][vn];
-                    if (own && ti == bn)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            rb[(kn & 1) * B + 4 * tj + v] = mr[vn][v];
-                            xb[(kn & 1) * B + 4 * tj + v] = xr[vn][v];
-                        }
-                }
-            }
+            for (int u = 0; u < 4; ++u) MA[16 * I + 4 * u + lk + (16 * J + lr) * LD] = acc[q][u];
         }
         __syncthreads();
         // panel rows 0..b-1 of A: R_house = S R on and above the diagonal, L below
         for (int idx = tid; idx < BB; idx += kCQThreads) {
             const int r = idx % B, j = idx / B;
-            const double v = (j >= r) ? sv[r] * M1[r + j * LD] : Lm[r + j * LD];
-            a.A[(i64)r + (i64)j * a.lda] = (T)v;
-            if (a.Y) a.Y[(i64)r + (i64)j * a.ldy] = (T)((j < r) ? Lm[r + j * LD] : (j == r ? 1.0 : 0.0));
-        }
-        // Mw = -S L^-T (upper triangular: Mw(k, j) = -s_k L^-1(j, k)) into M1 and, with U,
-        // into bc for the other workgroups. Every workgroup then forms its rows of
-        // W = Y T = (Q - [S; 0]) Mw from its rows of Q (T = -U S L^-T gives
-        // Q_2 U^-1 T = -Q_2 S L^-T below the first b rows, and L T = -(Q_1 - S) S L^-T on
-        // them) and Y = Q_2 U^-1 by substitution along its rows; workgroup 0 also forms
-        // T = U Mw for the output, after the barrier.
-        __syncthreads(); // R in M1 and L in M2 read above
-        if (own)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int j = 4 * ti + u, k = 4 * tj + v; // xr[u][v] = L^-1(j, k)
-                    const double m = -sv[k] * xr[u][v];
-                    M1[k + j * LD] = m;
-                    st_wt(a.bc + BB + k + (size_t)j * B, m);
-                }
-        for (int idx = tid; idx < BB; idx += kCQThreads) st_wt(a.bc + idx, Um[(idx % B) + (idx / B) * LD]);
-        if (tid < B) P[(size_t)tid * CHp + tid] -= sv[tid]; // Q - [S; 0] on the top block
-        if (tid == 0) *a.gate = 0;
-    }
-    if (!grid_barrier_wt(a.counter, (unsigned)a.G * ++nbar, a.err)) return;
-    if (g != 0) {
-        // U and Mw: rounds of 2 x LB loads per thread, all issued before their LDS stores
-        constexpr int LB = 8;
-        for (int base = 0; base < BB; base += LB * kCQThreads) {
-            double u[LB], t[LB];
-#pragma unroll
-            for (int q = 0; q < LB; ++q) {
-                const int idx = base + q * kCQThreads + tid;
-                u[q] = (idx < BB) ? ld_wt(a.bc + idx) : 0.0;
-                t[q] = (idx < BB) ? ld_wt(a.bc + BB + idx) : 0.0;
-            }
-#pragma unroll
-            for (int q = 0; q < LB; ++q) {
-                const int idx = base + q * kCQThreads + tid;
-                const int i = idx % B, j = idx / B;
-                if (idx < BB) {
-                    M3[i + j * LD] = u[q];
-                    M1[i + j * LD] = t[q];
-                }
-            }
+            const double l = MC[r + j * LD];
+            a.A[(i64)r + (i64)j * a.lda] = (T)((j >= r) ? sv[r] * MA[r + j * LD] : l);
+            if (a.Y) a.Y[(i64)r + (i64)j * a.ldy] = (T)((j < r) ? l : (j == r ? 1.0 : 0.0));
         }
         __syncthreads();
+    } else {
+        // workgroup 0's arrival alone
+        if (!grid_wait_wt(a.counter, (unsigned)a.G * nbar + 1u, a.err)) return;
     }
-    if (tid < B) gd[tid] = 1.0 / M3[tid + tid * LD]; // 1 / U(j, j)
+    {
+        // U^-1 and Mw: rounds of 2 x LB loads per thread, all issued before their LDS stores
+        constexpr int LB = (BB + kCQThreads - 1) / kCQThreads;
+        double u[LB], t[LB];
+#pragma unroll
+        for (int q = 0; q < LB; ++q) {
+            const int idx = q * kCQThreads + tid;
+            u[q] = (idx < BB) ? ld_wt(a.bc + idx) : 0.0;
+            t[q] = (idx < BB) ? ld_wt(a.bc + BB + idx) : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < LB; ++q) {
+            const int idx = q * kCQThreads + tid;
+            const int i = idx % B, j = idx / B;
+            if (idx < BB) {
+                MA[i + j * LD] = u[q];
+                MB[j + i * LD] = t[q];
+            }
+        }
+    }
     __syncthreads();
-    // W = (Q - [S; 0]) Mw for every row of this workgroup, before Y replaces Q
-    if (a.W) {
-        const int nrb = (chl + 3) / 4;
-        for (int blk = tid; blk < nrb * NB; blk += kCQThreads) {
-            const int rbk = blk / NB, cj = blk % NB;
-            const int rr = 4 * rbk;
-            double acc[4][4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-            for (int i = 0; i <= cj + NB * 3; ++i) { // Mw(i, j) = 0 for i > j
-                double x[4], w[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) x[u] = P[(size_t)i * CHp + rr + u];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) w[v] = M1[i + (cj + NB * v) * LD];
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[u][v] += x[u] * w[v];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (rr + u < chl)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        a.W[(i64)(r0g + rr + u) + (i64)(cj + NB * v) * a.ldw] = (T)acc[u][v];
-        }
-        __syncthreads();
-    }
-    // Y = Q U^-1 for the rows below the first b (workgroup 0 wrote its top rows, L)
+    // W = Y T = (Q - [S; 0]) Mw (T = -U S L^-T gives Q_2 U^-1 T = -Q_2 S L^-T below the first b
+    // rows, and L T = -(Q_1 - S) S L^-T on them), and Y = Q U^-1 for the rows below the
+    // first b (workgroup 0 wrote its top rows, L), also the reflector tails in A
     const int ylo = (g == 0) ? B : 0;
-    cq_rsolve<B>(P, CHp, ylo, chl, M3, gd, tid);
-    // outputs: Y and the reflector tails in A
-    for (int idx = tid; idx < B * chl; idx += kCQThreads) {
-        const int j = idx / chl, rl = idx - j * chl;
-        if (rl < ylo) continue;
-        const T y = (T)P[(size_t)j * CHp + rl];
+    for (int t = wave; t < ntask; t += kCQWaves) {
+        const int I = t / NP, pr = t % NP;
+        const int Jt[2] = {pr, NTB - 1 - pr};
+        cq_v4 w[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, y[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+        for (int k0 = 0; k0 < 16 * (Jt[1] + 1); k0 += 4) {
+            const double x = P[(size_t)(k0 + lk) * ldp + 16 * I + lr];
+#pragma unroll
+            for (int c = 0; c < (NTB > 1 ? 2 : 1); ++c)
+                if (k0 < 16 * (Jt[c] + 1)) {
+                    const int at = k0 + lk + (16 * Jt[c] + lr) * LD;
+                    if (a.W) w[c] = cq_mma(MB[at], x, w[c]);
+                    if (16 * I >= ylo) y[c] = cq_mma(MA[at], x, y[c]);
+                }
+        }
+        const int rl = 16 * I + lr;
         const i64 r = r0g + rl;
-        a.A[r + (i64)j * a.lda] = y;
-        if (a.Y) a.Y[r + (i64)j * a.ldy] = y;
+        if (rl < chl)
+#pragma unroll
+            for (int c = 0; c < (NTB > 1 ? 2 : 1); ++c)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const i64 j = 16 * Jt[c] + 4 * u + lk;
+                    if (a.W) a.W[r + j * a.ldw] = (T)w[c][u];
+                    if (16 * I >= ylo) {
+                        a.A[r + j * a.lda] = (T)y[c][u];
+                        if (a.Y) a.Y[r + j * a.ldy] = (T)y[c][u];
+                    }
+                }
     }
     if (g == 0) {
         // T = U Mw (upper triangular), and tau = diag(T)
-        double acc[4][4];
-        cq_mm<B, false>(acc, M3, M1, si, sj);
-        if (own)
+        for (int t = wave; t < NTB * NTB; t += kCQWaves) {
+            const int I = t / NTB, J = t % NTB;
+            cq_v4 acc = {0, 0, 0, 0};
+            if (I <= J) acc = cq_upper_mm<B>(MC, MB, I, J, acc, lane);
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int i = si + NB * u, j = sj + NB * v;
-                    a.Tm[i + (size_t)j * B] = (T)acc[u][v];
-                    if (i == j) a.tau[j] = (T)acc[u][v];
-                }
+            for (int u = 0; u < 4; ++u) {
+                const int i = 16 * I + 4 * u + lk, j = 16 * J + lr;
+                a.Tm[i + (size_t)j * B] = (T)acc[u];
+                if (i == j) a.tau[j] = (T)acc[u];
+            }
+        }
     }
 }
 
+// sets of 64 lanes that hold the rows of [G; P]
+constexpr int cq_sets(int b, int CH) { return (b + CH + 63) / 64; }
+
 template <int B> size_t cq_lds_bytes(int CH) {
-    return sizeof(double) * ((size_t)B * (CH + 1) + 3 * (size_t)B * (B + 1) + 9 * (size_t)B + kCQThreads);
+    const size_t groups = std::max((size_t)B * (B + 2), (size_t)768 * cq_sets(B, CH));
+    return sizeof(double) * ((size_t)B * cq_ldp(CH) + 2 * (size_t)B * (B + 2) + groups + B + 1);
 }
 
 __global__ void zero_u32_kernel(unsigned *p, int n) {
@@ -1023,11 +1009,13 @@ int launch_cholqr(hipStream_t s, T *A, i64 lda, T *Y, i64 ldy, T *W, i64 ldw, T 
     const int CH = std::max(64, (int)round_up(ceil_div(rows, ncu), 16));
     if (CH > kCQMaxCH) return CUEV_STATUS_SUCCESS;
     const int G = (int)ceil_div(rows, CH);
+    // [G; P] takes two sets of 64 lanes, for b = 64 and more than 64 rows three
+    static_assert(cq_sets(16, kCQMaxCH) <= 2 && cq_sets(32, kCQMaxCH) <= 2 && cq_sets(64, kCQMaxCH) <= 3, "");
+    const auto kernel = cq_sets(B, CH) <= 2 ? panel_cholqr_kernel<T, B, 2> : panel_cholqr_kernel<T, B, B == 64 ? 3 : 2>;
     const size_t lds = cq_lds_bytes<B>(CH);
-    CUEV_HIP(hipFuncSetAttribute((const void *)panel_cholqr_kernel<T, B>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    CUEV_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int per_cu = 0;
-    CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, panel_cholqr_kernel<T, B>, kCQThreads, lds));
+    CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kCQThreads, lds));
     if (G > per_cu * ncu) return CUEV_STATUS_SUCCESS;
     const size_t need = kPQGateBytes + sizeof(double) * ((size_t)(G + 3) * B * B);
     if (need > scratch_bytes) return CUEV_STATUS_SUCCESS;
@@ -1050,7 +1038,7 @@ int launch_cholqr(hipStream_t s, T *A, i64 lda, T *Y, i64 ldy, T *W, i64 ldw, T 
     a.counter = counter;
     a.reset = counter + 1;
     a.err = err;
-    hipLaunchKernelGGL((panel_cholqr_kernel<T, B>), dim3(G), dim3(kCQThreads), lds, s, a);
+    hipLaunchKernelGGL(kernel, dim3(G), dim3(kCQThreads), lds, s, a);
     CUEV_LAUNCH_CHECK();
     *launched = true;
     return CUEV_STATUS_SUCCESS;
