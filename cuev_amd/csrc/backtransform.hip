@@ -9,7 +9,7 @@
 // their row ranges overlap, and then the one of the later sweep goes first.
 // Overlaps occur only between (s, h) and (s', h) with |s - s'| < b, and between
 // (s, h+1) and (s', h) with s' > s. Hence this order is valid:
-//   passes of G = 128/b hop indices, in increasing order;
+//   passes of 4 or 8 hop indices, in increasing order;
 //   inside a pass, groups of 16 consecutive sweeps, in decreasing order;
 //   inside a group, its hops in increasing order; for one hop the 16
 //   reflectors (sweeps s0..s0+15) are one block H_s0 ... H_s0+15 = I - V T V^T
@@ -17,13 +17,11 @@
 //   T = (I/2 + striu(V^T V))^-1 for reflectors H = I - 2 w w^T).
 // Each block is three small MFMA products on 16 columns of M:
 //   X = V^T M_J, Y = T X, M_J -= V Y.
-// One wave64 owns 16 columns of M and walks every block; waves never share
-// data, so the kernel has no barriers. With v_mfma_*_16x16x4, the
-// accumulator register r of lane l holds row kidx(r, l/16) of its 16x16 tile;
-// the K index of every product is ordered by the same kidx, so the registers of
-// X and Y are directly the B operand of the next product and the rows of M_J
-// kept in registers are at once the B operand of X and the accumulator of the
-// update.
+// A workgroup owns 16 or 32 columns of M, each of its waves one hop of a pass (see
+// bc_back_kernel). With v_mfma_*_16x16x4, the accumulator register r of lane l holds row
+// kidx(r, l/16) of its 16x16 tile; the K index of every product is ordered by the same kidx, so
+// the registers of X and Y are directly the B operand of the next product and the rows of M_J
+// kept in registers are at once the B operand of X and the accumulator of the update.
 //
 // sbr_back (M <- Q_s M): the reference applies the DBBR panels last-first,
 // M_b -= W_j (Y_j^T M_b) (backtransform.cu:210-230), one rank-b update of M per
@@ -32,6 +30,7 @@
 #include "backtransform.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -43,8 +42,13 @@ namespace cuev {
 namespace {
 
 constexpr int kBTThreads = 256; // T-factor kernel: one wave per block reflector
-constexpr int kBBThreads = 128; // apply kernel: independent waves, 2 per workgroup (LDS <= 64 KB)
-// blocks per launch of the paired apply kernel (a quarter of the stream at n = 16384)
+// apply kernel: hops per pass, one wave each. Transposed it runs beside the tridiagonal solver, to
+// whose kernels the registers of one wave per SIMD leave room; otherwise nothing runs beside it, and
+// two waves hide each other's waits (FP64: n = 8192 26.7 -> 23.0 ms, n = 16384 205 -> 174; beside
+// the solver both together take 38 ms at n = 8192 with four waves and 41 with eight).
+constexpr int bt_waves(bool tr) { return tr ? 4 : 8; }
+// blocks per launch of the apply kernel (a quarter of the stream at n = 16384; 8000 makes no
+// difference there)
 constexpr i64 kBtSegBlocks = 33000;
 
 template <typename T> struct MfmaBt;
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(kBTThreads, 2) void bt_pack_kernel(const T *__restr
     }
     __syncthreads();
     if (!act) {
-        if (id == nblocks) // an all-zero block after the last (the identity, for the paired kernel)
+        if (id == nblocks) // an all-zero block after the last (the identity, for waves without one)
             for (int c = 0; c < NOP; ++c) ops[id * (i64)(NOP * 64) + c * 64 + lane] = T(0);
         return;
     }
@@ -171,536 +175,223 @@ __global__ __launch_bounds__(kBTThreads, 2) void bt_pack_kernel(const T *__restr
         }
 }
 
-// Position of a block in the application order (wave-uniform), with the block's
-// index in the packed operands, toff[g] + h.
-struct BtPos {
-    int h0, g, h; // pass start hop, sweep group, hop
-    i64 id;
-};
-
-// Blocks (hops) of sweep group g: toff[g + 1] - toff[g].
-template <int B> __device__ __forceinline__ int bt_hops(int g, int n) { return (n - 2 - g * kBtGroup) / B + 1; }
-
-// Advance to the next block: hops of the group, then the group below, then the
-// next pass. Returns false after the last block. The index follows from the
-// previous one except at a pass start (toff read once per pass).
-template <int B> __device__ __forceinline__ bool bt_next(BtPos &p, int n, const i64 *__restrict__ toff) {
-    constexpr int G = 128 / B;
-    if (p.h + 1 < p.h0 + G && p.g * kBtGroup + 1 + (p.h + 1) * B <= n - 1) {
-        ++p.h;
-        ++p.id;
-        return true;
-    }
-    if (p.g > 0) {
-        --p.g;
-        p.id += p.h0 - p.h - bt_hops<B>(p.g, n); // toff[g-1] = toff[g] - hops(g-1)
-        p.h = p.h0;
-        return true;
-    }
-    p.h0 += G;
-    const int smax = min(n - 3, n - 2 - p.h0 * B);
-    if (smax < 0) return false;
-    p.g = smax / kBtGroup;
-    p.h = p.h0;
-    p.id = toff[p.g] + p.h;
-    return true;
-}
-
-// Step back to the previous block of that order (the order of Q_b^T M, whose blocks
-// are the same reflectors in reverse, each transposed). Returns false before the first.
-template <int B> __device__ __forceinline__ bool bt_prev(BtPos &p, int n) {
-    constexpr int G = 128 / B;
-    if (p.h > p.h0) {
-        --p.h;
-        --p.id;
-        return true;
-    }
-    if (p.g < min(n - 3, n - 2 - p.h0 * B) / kBtGroup) {
-        const i64 t = p.id - p.h + bt_hops<B>(p.g, n); // toff[g+1] = toff[g] + hops(g)
-        ++p.g;
-        p.h = min(p.h0 + G - 1, (n - 2 - p.g * kBtGroup) / B);
-        p.id = t + p.h;
-        return true;
-    }
-    if (p.h0 == 0) return false;
-    p.h0 -= G;
-    p.g = 0;
-    p.h = min(p.h0 + G - 1, (n - 2) / B);
-    p.id = p.h; // toff[0] = 0
-    return true;
-}
-
-// One block's packed operands (see bt_pack_kernel), as NOP/2 pairs.
-template <typename T, int NP>
-__device__ __forceinline__ void bt_load_ops(T (&o)[2 * NP], const T *__restrict__ ops, i64 id, int lane) {
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    const T2 *p = reinterpret_cast<const T2 *>(ops + id * (i64)(2 * NP * 64)) + lane;
-#pragma unroll
-    for (int c = 0; c < NP; ++c) {
-        const T2 v = p[c * 64];
-        o[2 * c] = v.x;
-        o[2 * c + 1] = v.y;
-    }
-}
-
-// M <- Q_b M (TR: M <- Q_b^T M, the blocks in reverse order, each transposed) for
-// columns [0, ncols): one wave per 16 columns (see the header). Each wave keeps the
-// rows of the current pass's window, WS = G*b + 16 rows of its 16 columns, in a
-// private LDS buffer of RS = WS + 64 rows: row r of the matrix sits in buffer row
-// r - org. The window slides 16 rows per sweep group (a group costs 16 rows in and
-// 16 out); when it reaches the end of the buffer, its rows move back to the other
-// end in one copy (every 4 groups), so a block's 16 NKB rows are always contiguous
-// and every LDS access of a block is one base address plus a constant. The next
-// block's operands are loaded into the other of two register sets at the start of
-// each block, and the rows entering at a group change are loaded at the previous
-// change, so neither load is waited for inside the block that issues it. Rows past
-// n are read from zp (zeros) and not written.
-template <typename T, int B, bool TR>
-__global__ __launch_bounds__(kBBThreads) void bc_back_kernel(const T *__restrict__ ops,
-                                                             const i64 *__restrict__ toff,
-                                                             const T *__restrict__ zp, T *M,
-                                                             i64 ldm, int n, int ncols) {
-    using MB = MfmaBt<T>;
-    using V4 = typename MB::v4;
-    constexpr int NG = kBtGroup;
-    constexpr int NKB = B / 16 + 1; // 16-row tiles covering a block's b + 15 rows
-    constexpr int NC = 4 * NKB;     // 4-row K chunks
-    constexpr int NOP = 2 * NC;     // operand values per lane per block
-    constexpr int G = 128 / B;      // hops per pass
-    constexpr int WS = G * B + 16;  // window rows
-    constexpr int RS = WS + 64;     // buffer rows
-    constexpr int LDW = 17;         // LDS row stride: rows and 16-column reads both conflict-free
-    __shared__ T win[(kBBThreads / 64) * RS * LDW];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, q = lane >> 4, li = lane & 15;
-    const int wcol = (blockIdx.x * (kBBThreads / 64) + wave) * 16;
-    if (wcol >= ncols) return; // whole wave
-    const int wb = wave * (RS * LDW); // this wave's buffer
-    const int last = n - 3;           // last sweep
-    for (int e = lane; e < RS * LDW; e += 64) win[wb + e] = T(0);
-
-// matrix rows [r0, r0+16) of the wave's 16 columns: lane = (row li, columns q + 4i)
-#define BT_LOAD16(r0, v)                                                                           \
-    do {                                                                                           \
-        const int r_ = (r0) + li;                                                                  \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                         \
-            const int col_ = wcol + q + 4 * i_;                                                    \
-            const bool ok_ = r_ >= 0 && r_ < n && col_ < ncols;                                    \
-            (v)[i_] = *(ok_ ? M + r_ + (i64)col_ * ldm : zp);                                      \
-        }                                                                                          \
-    } while (0)
-// buffer rows [b0, b0+16)
-#define BT_PUT16(b0, v)                                                                            \
-    do {                                                                                           \
-        const int o_ = wb + ((b0) + li) * LDW + q;                                                 \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) win[o_ + 4 * i_] = (v)[i_];               \
-    } while (0)
-// matrix rows [r0, r0+16) from buffer rows [b0, b0+16)
-#define BT_STORE16(r0, b0)                                                                         \
-    do {                                                                                           \
-        const int r_ = (r0) + li;                                                                  \
-        const int o_ = wb + ((b0) + li) * LDW + q;                                                 \
-        T v_[4];                                                                                   \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) v_[i_] = win[o_ + 4 * i_];                \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                         \
-            const int col_ = wcol + q + 4 * i_;                                                    \
-            if (r_ < n && col_ < ncols) M[r_ + (i64)col_ * ldm] = v_[i_];                          \
-        }                                                                                          \
-    } while (0)
-// buffer rows [s0, s0 + WS - 16) -> [d0, d0 + WS - 16): all read, then all written
-// (so the two ranges may overlap)
-#define BT_MOVE(s0, d0)                                                                            \
-    do {                                                                                           \
-        constexpr int NM_ = (WS - 16) / 16;                                                        \
-        T v_[NM_][4];                                                                              \
-        const int os_ = wb + ((s0) + li) * LDW + q, od_ = wb + ((d0) + li) * LDW + q;              \
-        _Pragma("unroll") for (int c_ = 0; c_ < NM_; ++c_)                                         \
-            _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) v_[c_][i_] = win[os_ + 16 * c_ * LDW + 4 * i_]; \
-        _Pragma("unroll") for (int c_ = 0; c_ < NM_; ++c_)                                         \
-            _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) win[od_ + 16 * c_ * LDW + 4 * i_] = v_[c_][i_]; \
-    } while (0)
-
-    BtPos p;
-    if (TR) {
-        p.h0 = ((n - 2) / B) / G * G; // last pass
-        p.g = 0;
-        p.h = min(p.h0 + G - 1, (n - 2) / B);
-    } else {
-        p.h0 = 0;
-        p.g = min(last, n - 2) / NG;
-        p.h = 0;
-    }
-    p.id = toff[p.g] + p.h;
-    // the window moves down the buffer going up the groups (TR), up it going down
-    int top = p.g * NG + 1 + p.h0 * B; // first window row
-    int org = TR ? top : top - (RS - WS);
-    BtPos pn = p;
-    bool more = TR ? bt_prev<B>(pn, n) : bt_next<B>(pn, n, toff);
-    T opa[NOP], opb[NOP];
-    bt_load_ops<T, NC>(opa, ops, p.id, lane);
-    for (int c = 0; c < WS; c += 16) {
-        T v[4];
-        BT_LOAD16(top + c, v);
-        BT_PUT16(top + c - org, v);
-    }
-    // this lane's first element of a block tile: row kidx(0, q), column li; the
-    // others are at constant offsets (kidx(r, q) = kidx(0, q) + kidx(r, 0))
-    const int lofs = wb + MB::kidx(0, q) * LDW + li;
-    // rows entering at the next group change (below the window going up the groups
-    // (TR), above it going down), loaded as soon as the window's position is known so
-    // that their latency is spread over the group's blocks
-    T ent[4];
-    BT_LOAD16(TR ? top + WS : top - 16, ent);
-
-    // One block with operands cur; the next block's operands are loaded into nxt
-    // first (a repeat of this block when nothing follows: no branch). Returns false
-    // after the last block. Called alternately with the two register sets, so no
-    // operand is copied and the loads have a whole block to arrive.
-    auto step = [&](T(&cur)[NOP], T(&nxt)[NOP]) -> bool {
-        bt_load_ops<T, NC>(nxt, ops, more ? pn.id : p.id, lane);
-        __builtin_amdgcn_sched_barrier(0);
-
-        // ---- block (g, h): rows [base, base + 16 NKB) of the window
-        const int base = p.g * NG + 1 + p.h * B;
-        const int wr = lofs + (base - org) * LDW;
-        T m[NC];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) m[c] = win[wr + (16 * (c >> 2) + MB::kidx(c & 3, 0)) * LDW];
-        // X = V^T M_J in two independent chains (even and odd chunks)
-        V4 x = {T(0), T(0), T(0), T(0)}, x1 = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-        for (int c = 0; c < NC; c += 2) {
-            x = MB::mma(cur[c], m[c], x);
-            x1 = MB::mma(cur[c + 1], m[c + 1], x1);
-        }
-        x += x1;
-        // M_J += W X, W = -V T (or -V T^T): the registers of X are the B operand
-#pragma unroll
-        for (int t = 0; t < NKB; ++t) {
-            V4 acc = {m[4 * t], m[4 * t + 1], m[4 * t + 2], m[4 * t + 3]};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc = MB::mma(cur[NC + 4 * t + r], x[r], acc);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) win[wr + (16 * t + MB::kidx(r, 0)) * LDW] = acc[r];
-        }
-
-        // ---- window bookkeeping for the next block
-        if (!more || pn.h0 != p.h0) {
-            // pass done: write the window back
-            for (int c = 0; c < WS; c += 16) BT_STORE16(top + c, top + c - org);
-            if (!more) return false;
-            wave_stores_done(); // the next pass reads these rows back through other lanes
-            top = pn.g * NG + 1 + pn.h0 * B;
-            org = TR ? top : top - (RS - WS);
-            for (int c = 0; c < WS; c += 16) {
-                T v[4];
-                BT_LOAD16(top + c, v);
-                BT_PUT16(top + c - org, v);
-            }
-            BT_LOAD16(TR ? top + WS : top - 16, ent);
-        } else if (pn.g != p.g) {
-            if (TR) {
-                // group g -> g+1: 16 rows leave at the top, 16 enter at the bottom
-                BT_STORE16(top, top - org);
-                top += 16;
-                if (top + WS - org > RS) {
-                    // rows [top, top + WS - 16) back to the start of the buffer
-                    BT_MOVE(top - org, 0);
-                    org = top;
-                }
-                BT_PUT16(top + WS - 16 - org, ent);
-                BT_LOAD16(top + WS, ent);
-            } else {
-                // group g -> g-1: 16 rows leave at the bottom, 16 enter at the top
-                BT_STORE16(top + WS - 16, top + WS - 16 - org);
-                top -= 16;
-                if (top < org) {
-                    // rows [top + 16, top + WS) to the end of the buffer
-                    const int norg = top - (RS - WS);
-                    BT_MOVE(top + 16 - org, top + 16 - norg);
-                    org = norg;
-                }
-                BT_PUT16(top - org, ent);
-                BT_LOAD16(top - 16, ent);
-            }
-        }
-        p = pn;
-        more = more && (TR ? bt_prev<B>(pn, n) : bt_next<B>(pn, n, toff));
-        return true;
-    };
-    for (;;) {
-        if (!step(opa, opb)) break;
-        if (!step(opb, opa)) break;
-    }
-#undef BT_LOAD16
-#undef BT_PUT16
-#undef BT_STORE16
-#undef BT_MOVE
-}
-
-// Passes of two hops for the paired kernel below. The blocks of a pass, in the
-// order of bc_back_kernel (groups down, hops up), taken two at a time as steps
-// {(g, h0+1), (g-1, h0)}: the two blocks of a step cover disjoint rows (the first
-// ends where the second starts), so they are independent and the step is the same
-// sequence of blocks. In the order of Q_b^T M (TR: groups up, hops down) the steps
-// are {(g, h0), (g+1, h0+1)}. Either way one step covers the rows of a window of
-// 2 NKB 16-row tiles: its lower block the first NKB, its upper block the others.
-struct BtStep {
-    int h0, g;  // pass start hop, step group (see bt_step_blocks)
-    int gA, gB; // last group with hop h0, with hop h0 + 1 (-1: none)
-    i64 tg;     // forward: toff[g]; TR: toff[g + 1]
-};
-
-template <int B> __device__ __forceinline__ int bt_gmax(int n, int h) {
-    const int m = min(n - 3, n - 2 - h * B);
+// last group with hop h (-1: none)
+template <int B> __host__ __device__ __forceinline__ int bt_gmax(int n, int h) {
+    const int m = n - 3 < n - 2 - h * B ? n - 3 : n - 2 - h * B;
     return m < 0 ? -1 : m / kBtGroup;
 }
 
-// the first step of the pass starting at hop h0
-template <int B, bool TR>
-__device__ __forceinline__ void bt_step_first(BtStep &s, int n, const i64 *__restrict__ toff, int h0) {
-    s.h0 = h0;
-    s.gA = bt_gmax<B>(n, s.h0);
-    s.gB = bt_gmax<B>(n, s.h0 + 1);
-    s.g = TR ? (s.gB >= 0 ? -1 : 0) : s.gA + 1;
-    s.tg = toff[TR ? s.g + 1 : s.g];
-}
-
-// Next step; false after the last. The offsets follow from the hop counts except
-// at a pass start.
-template <int B, bool TR> __device__ __forceinline__ bool bt_step_next(BtStep &s, int n, const i64 *__restrict__ toff) {
-    if (TR) {
-        if (s.g < s.gA) {
-            ++s.g;
-            s.tg += bt_hops<B>(s.g, n);
-            return true;
-        }
-        s.h0 -= 2;
-        if (s.h0 < 0) return false;
-        s.gA = bt_gmax<B>(n, s.h0);
-        s.gB = bt_gmax<B>(n, s.h0 + 1);
-        s.g = s.gB >= 0 ? -1 : 0;
-        s.tg = toff[s.g + 1];
-        return true;
-    }
-    if (s.g > (s.gB >= 0 ? 0 : 1)) {
-        s.tg -= bt_hops<B>(s.g - 1, n);
-        --s.g;
-        return true;
-    }
-    s.h0 += 2;
-    s.gA = bt_gmax<B>(n, s.h0);
-    if (s.gA < 0) return false;
-    s.gB = bt_gmax<B>(n, s.h0 + 1);
-    s.g = s.gA + 1;
-    s.tg = toff[s.g];
-    return true;
-}
-
-// The two blocks of a step: packed index (il, iu; an absent block, at a pass end,
-// gets the all-zero block nblocks, which leaves its rows unchanged) and the
-// window's first row.
-template <int B, bool TR>
-__device__ __forceinline__ void bt_step_blocks(const BtStep &s, int n, i64 nblocks, i64 &il, i64 &iu, int &top) {
-    if (TR) { // lower (g, h0), upper (g+1, h0+1)
-        il = s.g >= 0 ? s.tg - bt_hops<B>(s.g, n) + s.h0 : nblocks;
-        iu = s.g + 1 <= s.gB ? s.tg + s.h0 + 1 : nblocks;
-        top = s.g * kBtGroup + 1 + s.h0 * B;
-    } else { // lower (g-1, h0), upper (g, h0+1)
-        il = s.g >= 1 ? s.tg - bt_hops<B>(s.g - 1, n) + s.h0 : nblocks;
-        iu = s.g <= s.gB ? s.tg + s.h0 + 1 : nblocks;
-        top = (s.g - 1) * kBtGroup + 1 + s.h0 * B;
-    }
-}
-
-// One half of a block's packed operands: V (half 0) or W (half 1), NP pairs.
-template <typename T, int NP>
-__device__ __forceinline__ void bt_load_half(T (&o)[2 * NP], const T *__restrict__ ops, i64 id, int half, int lane) {
+// Tile j of one half of a block's packed operands, V (half 0) or W (half 1) of NC values.
+template <typename T, int NC>
+__device__ __forceinline__ void bt_load_ops(T (&o)[NC], const T *__restrict__ ops, i64 id, int half, int j, int lane) {
     typedef T T2 __attribute__((ext_vector_type(2)));
-    const T2 *p = reinterpret_cast<const T2 *>(ops + id * (i64)(4 * NP * 64)) + (half * NP) * 64 + lane;
-#pragma unroll
-    for (int c = 0; c < NP; ++c) {
-        const T2 v = p[c * 64];
-        o[2 * c] = v.x;
-        o[2 * c + 1] = v.y;
-    }
+    const T2 *p = reinterpret_cast<const T2 *>(ops + id * (i64)(2 * NC * 64)) + (half * (NC / 2) + 2 * j) * 64 + lane;
+    const T2 v0 = p[0], v1 = p[64];
+    o[4 * j] = v0.x;
+    o[4 * j + 1] = v0.y;
+    o[4 * j + 2] = v1.x;
+    o[4 * j + 3] = v1.y;
 }
 
-// M <- Q_b M (TR: Q_b^T M) for columns [0, ncols), one wave per 16 columns, two
-// blocks per step (see BtStep), over the passes from the one starting at hop h_first
-// to the one starting at hop h_last (in application order; a pass leaves all its
-// rows in M, so a launch may end and the next begin at any pass): the two blocks' products are interleaved, so the
-// MFMA pipe has independent work while either block's chain drains, and a step's
-// fixed costs (LDS round trip, window bookkeeping) are shared by two blocks. The
-// window lives in a ring of 2 NKB + 1 tiles of 16 rows per wave (24 KB at b = 64,
-// so the kernel leaves LDS for the tridiagonal solver's GEMMs running beside it);
-// a step slides it by one tile, storing the tile that leaves and putting the one
-// that enters (loaded a step earlier) into the free slot. The next step's operands
-// are loaded into the registers of the current ones as these die: V after the X
-// products, W after the update.
-template <typename T, int B, bool TR>
-__global__ __launch_bounds__(kBBThreads) void bc_back_pair_kernel(const T *__restrict__ ops,
-                                                                  const i64 *__restrict__ toff,
-                                                                  i64 nblocks, const T *__restrict__ zp,
-                                                                  T *M, i64 ldm, int n, int ncols, int h_first,
-                                                                  int h_last) {
+template <int... PH, typename F> __device__ __forceinline__ void bt_rotations(std::integer_sequence<int, PH...>, F &&f) {
+    (f(std::integral_constant<int, PH>{}), ...);
+}
+
+// M <- Q_b M (TR: M <- Q_b^T M, the blocks in reverse order, each transposed) for columns
+// [0, ncols), over the passes p_first to p_last (in application order; a pass leaves all its rows
+// in M, so a launch may end and the next begin at any pass). One workgroup per 16 NCT columns.
+//
+// Pass p applies the hops p NW + w, wave w one of them. Block (g, h) covers the 16 NKB =
+// b + 16 rows from 16 g + 1 + h b on, and block (g + 1, h + 1) the b + 16 rows after those; of two
+// reflectors whose rows overlap, (s, h + 1) and (s', h) with s' > s, the second goes first. So
+// while wave w is at group g, wave w + 1 may be at group g + 1: the waves' blocks of one step are
+// independent, and their windows make one contiguous window of NW NKB tiles of 16 rows,
+// which moves up by one tile per step (TR: down). Every wave keeps its NKB tiles in registers;
+// at each step the tile at one end of a window goes to the next wave through LDS (at the end of
+// the row: to M), and one enters at the other (at the beginning: from M, its loads issued two
+// steps earlier, behind that step's operand loads, whose waits they would lengthen otherwise).
+// It enters the registers of the tile that left, so the roles of the registers rotate: the step
+// is written out for each rotation (twice, for the two sets of loads from M). A wave without a block in a step (at a
+// pass's ends, or past the last hop) applies the all-zero block, which changes nothing.
+// The next block's operands are loaded into the registers of the current ones as these die, tile
+// by tile. The tile that leaves is updated first, its hand-over hidden behind the other tiles'
+// products; the entering tile is used last in X.
+//
+// Bound: the MFMA pipe (8 NKB NCT products per step and wave: at b = 64 in FP64 2560 NCT cycles of
+// one SIMD) and, where there are fewer of column strips than CUs, their number.
+// Measured in FP64 at b = 64 (direct order, nothing beside it): n = 2500 1.5 ms, 4096 3.8, 8192 23,
+// 16384 175 (2 n^3 flops at 50 TF/s; the products' pipe is busy 80% of the time). With one wave per
+// 16 columns that walked every block, n = 2500 5.7 ms (on 157 of 1024 SIMDs), 4096 14.8, 8192 63,
+// 16384 242; with M's and the operands' loads issued together, one step ahead, 16384 258.
+template <typename T, int B, bool TR, int NCT>
+__global__ __launch_bounds__(64 * bt_waves(TR)) void bc_back_kernel(const T *__restrict__ ops, const i64 *__restrict__ toff,
+                                                             i64 nblocks, const T *__restrict__ zp, T *M, i64 ldm,
+                                                             int n, int ncols, int p_first, int p_last) {
     using MB = MfmaBt<T>;
     using V4 = typename MB::v4;
     constexpr int NKB = B / 16 + 1; // tiles of a block
     constexpr int NC = 4 * NKB;     // 4-row K chunks of a block; values per operand half
-    constexpr int NW = 2 * NKB;     // window tiles
-    constexpr int NS = NW + 1;      // ring slots: the window and the entering tile
-    constexpr int LDW = 17;
-    constexpr int SL = 16 * LDW; // one slot
-    __shared__ T win[(kBBThreads / 64) * NS * SL];
+    constexpr int NW = bt_waves(TR); // hops of a pass
+    constexpr int kSrc = TR ? NW - 1 : 0, kSink = TR ? 0 : NW - 1; // waves next to M
+    constexpr int kIn = TR ? NKB - 1 : 0, kOut = TR ? 0 : NKB - 1; // entering and leaving tile of a window
+    __shared__ T hand[2][NW][NCT][4][64]; // [parity of the step][from wave]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, q = lane >> 4, li = lane & 15;
-    const int wcol = (blockIdx.x * (kBBThreads / 64) + wave) * 16;
-    if (wcol >= ncols) return; // whole wave
-    const int wb = wave * (NS * SL);
-    const int lofs = wb + MB::kidx(0, q) * LDW + li; // a block tile's element of this lane
-    int tb = 0;                                      // ring slot of window tile 0
-    auto slot = [&](int t) { // ring slot of window tile t in [0, NS)
-        const int s = tb + t;
-        return s >= NS ? s - NS : s;
-    };
+    const int wcol = blockIdx.x * (16 * NCT);
 
-// matrix rows [r0, r0+16) of the wave's 16 columns: lane = (row li, columns q + 4i)
-#define BP_LOAD16(r0, v)                                                                           \
-    do {                                                                                           \
-        const int r_ = (r0) + li;                                                                  \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                         \
-            const int col_ = wcol + q + 4 * i_;                                                    \
-            const bool ok_ = r_ >= 0 && r_ < n && col_ < ncols;                                    \
-            (v)[i_] = *(ok_ ? M + r_ + (i64)col_ * ldm : zp);                                      \
-        }                                                                                          \
-    } while (0)
-#define BP_PUT16(s, v)                                                                             \
-    do {                                                                                           \
-        const int o_ = wb + (s) * SL + li * LDW + q;                                               \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) win[o_ + 4 * i_] = (v)[i_];               \
-    } while (0)
-#define BP_STORE16(s, r0)                                                                          \
-    do {                                                                                           \
-        const int r_ = (r0) + li;                                                                  \
-        const int o_ = wb + (s) * SL + li * LDW + q;                                               \
-        T v_[4];                                                                                   \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) v_[i_] = win[o_ + 4 * i_];                \
-        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                         \
-            const int col_ = wcol + q + 4 * i_;                                                    \
-            if (r_ >= 0 && r_ < n && col_ < ncols) M[r_ + (i64)col_ * ldm] = v_[i_];               \
-        }                                                                                          \
-    } while (0)
-
-    BtStep cur;
-    bt_step_first<B, TR>(cur, n, toff, h_first);
-    int top;
-    i64 il, iu;
-    bt_step_blocks<B, TR>(cur, n, nblocks, il, iu, top);
-    T lv[NC], lw[NC], uv[NC], uw[NC];
-    bt_load_half<T, NC / 2>(lv, ops, il, 0, lane);
-    bt_load_half<T, NC / 2>(uv, ops, iu, 0, lane);
-    bt_load_half<T, NC / 2>(lw, ops, il, 1, lane);
-    bt_load_half<T, NC / 2>(uw, ops, iu, 1, lane);
-    for (int t = 0; t < NW; ++t) {
-        T v[4];
-        BP_LOAD16(top + 16 * t, v);
-        BP_PUT16(t, v);
-    }
-    T ent[4];
-    bool putent = false;
-    for (;;) {
-        if (putent) BP_PUT16(slot(TR ? NW - 1 : 0), ent);
-        BtStep nx = cur;
-        const bool more = bt_step_next<B, TR>(nx, n, toff) && (TR ? nx.h0 >= h_last : nx.h0 <= h_last);
-        int ntop = top;
-        i64 nil = il, niu = iu;
-        if (more) bt_step_blocks<B, TR>(nx, n, nblocks, nil, niu, ntop);
-        // the tile entering at the next step, if it is in this pass
-        BP_LOAD16(TR ? top + 16 * NW : top - 16, ent);
-
-        // ---- the two blocks: lower on window tiles [0, NKB), upper on [NKB, NW)
-        T ml[NC], mu[NC];
+    // tile rows [r0, r0 + 16) of the workgroup's columns in accumulator layout
+    auto load_tile = [&](int r0, V4(&v)[NCT]) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int r = MB::kidx(c & 3, 0) * LDW;
-            ml[c] = win[lofs + slot(c >> 2) * SL + r];
-            mu[c] = win[lofs + slot(NKB + (c >> 2)) * SL + r];
-        }
-        // X = V^T M_J, two chains per block
-        V4 xl = {T(0), T(0), T(0), T(0)}, xl1 = xl, xu = xl, xu1 = xl;
-#pragma unroll
-        for (int c = 0; c < NC; c += 2) {
-            xl = MB::mma(lv[c], ml[c], xl);
-            xu = MB::mma(uv[c], mu[c], xu);
-            xl1 = MB::mma(lv[c + 1], ml[c + 1], xl1);
-            xu1 = MB::mma(uv[c + 1], mu[c + 1], xu1);
-        }
-        xl += xl1;
-        xu += xu1;
-        // the next step's V (a repeat of this step's when nothing follows)
-        bt_load_half<T, NC / 2>(lv, ops, nil, 0, lane);
-        bt_load_half<T, NC / 2>(uv, ops, niu, 0, lane);
-        // M_J += W X (W = -V T, or -V T^T). All products are issued before any
-        // store: a store waits for its product, and in-order issue would hold the
-        // remaining products behind it.
-        V4 al[NKB], au[NKB];
-#pragma unroll
-        for (int t = 0; t < NKB; ++t) {
-            al[t] = V4{ml[4 * t], ml[4 * t + 1], ml[4 * t + 2], ml[4 * t + 3]};
-            au[t] = V4{mu[4 * t], mu[4 * t + 1], mu[4 * t + 2], mu[4 * t + 3]};
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int t = 0; t < NKB; ++t) {
-                al[t] = MB::mma(lw[4 * t + r], xl[r], al[t]);
-                au[t] = MB::mma(uw[4 * t + r], xu[r], au[t]);
-            }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = 0; t < NKB; ++t) {
-            const int ol = lofs + slot(t) * SL, ou = lofs + slot(NKB + t) * SL;
+        for (int c = 0; c < NCT; ++c)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                win[ol + MB::kidx(r, 0) * LDW] = al[t][r];
-                win[ou + MB::kidx(r, 0) * LDW] = au[t][r];
+                const int row = r0 + MB::kidx(r, q), col = wcol + 16 * c + li;
+                const bool ok = row >= 0 && row < n && col < ncols;
+                v[c][r] = *(ok ? M + row + (i64)col * ldm : zp);
             }
-        }
+    };
+    auto store_tile = [&](int r0, const V4(&v)[NCT]) {
+#pragma unroll
+        for (int c = 0; c < NCT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = r0 + MB::kidx(r, q), col = wcol + 16 * c + li;
+                if (row >= 0 && row < n && col < ncols) M[row + (i64)col * ldm] = v[c][r];
+            }
+    };
 
-        // ---- window
-        if (!more || nx.h0 != cur.h0) {
-            for (int t = 0; t < NW; ++t) BP_STORE16(slot(t), top + 16 * t);
-            if (!more) break;
-            wave_stores_done(); // the next pass reads these rows back through other lanes
-            tb = 0;
-            for (int t = 0; t < NW; ++t) {
-                T v[4];
-                BP_LOAD16(ntop + 16 * t, v);
-                BP_PUT16(t, v);
-            }
-            putent = false;
-        } else {
-            if (TR) {
-                BP_STORE16(tb, top);
-                tb = tb + 1 == NS ? 0 : tb + 1;
-            } else {
-                BP_STORE16(slot(NW - 1), top + 16 * (NW - 1));
-                tb = tb == 0 ? NS - 1 : tb - 1;
-            }
-            putent = true;
+    for (int p = p_first; TR ? p >= p_last : p <= p_last; p += TR ? -1 : 1) {
+        const int h0 = p * NW, h = h0 + wave, gm = bt_gmax<B>(n, h), gs = bt_gmax<B>(n, h0);
+        const int nst = gs + NW; // steps: wave 0 at the groups gs .. -(NW - 1)
+        int g = (TR ? -(NW - 1) : gs) + wave;
+        int top = g * kBtGroup + 1 + h * B; // first row of this wave's window
+        auto block = [&](int g_) { return g_ >= 0 && g_ <= gm ? toff[g_] + h : nblocks; };
+        T ov[NC], ow[NC];
+        V4 m[NKB][NCT], ent[2][NCT];
+        const i64 id0 = block(g);
+#pragma unroll
+        for (int j = 0; j < NKB; ++j) {
+            bt_load_ops<T, NC>(ov, ops, id0, 0, j, lane);
+            bt_load_ops<T, NC>(ow, ops, id0, 1, j, lane);
         }
-        // the next step's W
-        bt_load_half<T, NC / 2>(lw, ops, nil, 1, lane);
-        bt_load_half<T, NC / 2>(uw, ops, niu, 1, lane);
-        cur = nx;
-        il = nil;
-        iu = niu;
-        top = ntop;
+#pragma unroll
+        for (int j = 0; j < NKB; ++j) load_tile(top + 16 * j, m[j]);
+        if (wave == kSrc) load_tile(TR ? top + 16 * NKB : top - 16, ent[1]);
+
+        // step t in rotation PH, t % (2 NKB): window tile j is m[at(j)]
+        auto step = [&](auto rot, int t) {
+            constexpr int PH = decltype(rot)::value;
+            auto at = [](int j) constexpr { return TR ? (j + PH) % NKB : (j + 2 * NKB - PH) % NKB; };
+            const bool last = t + 1 == nst;
+            if (t > 0) {
+                if (wave == kSrc) {
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c) m[at(kIn)][c] = ent[PH & 1][c];
+                } else {
+                    const int from = TR ? wave + 1 : wave - 1;
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) m[at(kIn)][c][r] = hand[(t - 1) & 1][from][c][r][lane];
+                }
+            }
+            const int ng = TR ? g + 1 : g - 1;
+            const i64 nid = last ? nblocks : block(ng);
+
+            // ---- X = V^T M_J, two chains per 16 columns, the entering tile last
+            V4 x[NCT][2];
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) x[c][0] = x[c][1] = V4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int jj = 1; jj <= NKB; ++jj) {
+                const int j = (kIn + (TR ? NKB - jj : jj)) % NKB;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c)
+                        x[c][r & 1] = MB::mma(ov[4 * j + r], m[at(j)][c][r], x[c][r & 1]);
+                bt_load_ops<T, NC>(ov, ops, nid, 0, j, lane);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) x[c][0] += x[c][1];
+            // ---- M_J += W X (W = -V T, or -V T^T): the leaving tile first; two tiles at a time
+            // where a tile has one chain only
+            constexpr int TW = NCT > 1 ? 1 : 2;
+#pragma unroll
+            for (int j0 = 0; j0 < NKB; j0 += TW) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int jj = j0; jj < j0 + TW && jj < NKB; ++jj) {
+                        const int j = (kOut + jj) % NKB;
+#pragma unroll
+                        for (int c = 0; c < NCT; ++c)
+                            m[at(j)][c] = MB::mma(ow[4 * j + r], x[c][0][r], m[at(j)][c]);
+                    }
+#pragma unroll
+                for (int jj = j0; jj < j0 + TW && jj < NKB; ++jj)
+                    bt_load_ops<T, NC>(ow, ops, nid, 1, (kOut + jj) % NKB, lane);
+                __builtin_amdgcn_sched_barrier(0);
+                if (j0 == (NKB > TW ? TW : 0) && !last && wave != kSink) { // the leaving tile is ready by now
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) hand[t & 1][wave][c][r][lane] = m[at(kOut)][c][r];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (last) {
+#pragma unroll
+                for (int j = 0; j < NKB; ++j) store_tile(top + 16 * j, m[at(j)]);
+            } else if (wave == kSink) {
+                store_tile(top + 16 * kOut, m[at(kOut)]);
+            }
+            if (wave == kSrc && t + 2 < nst) load_tile(TR ? top + 16 * NKB + 16 : top - 32, ent[PH & 1]);
+            __syncthreads();
+            g = ng;
+            top += TR ? 16 : -16;
+        };
+        for (int t = 0; t < nst;) {
+            bool go = true;
+            bt_rotations(std::make_integer_sequence<int, 2 * NKB>{}, [&](auto rot) {
+                if (!go) return;
+                step(rot, t);
+                go = ++t < nst;
+            });
+        }
+        // the next pass reads these rows back through other waves
+        wave_stores_done();
+        __syncthreads();
     }
-#undef BP_LOAD16
-#undef BP_PUT16
-#undef BP_STORE16
+}
+
+// The passes over columns [0, nc) of M, 16 NCT of them per workgroup.
+template <typename T, int B, int NCT>
+int launch_bc_passes(Workspace<T> &ws, hipStream_t s, T *M, i64 ldm, int nc, bool tr, const T *zp) {
+    const int n = ws.n;
+    // Passes in launches of at least kBtSegBlocks blocks each (the last one fewer): the
+    // workgroups of one launch drift apart along the block stream as it goes, and a launch
+    // boundary lines them up again.
+    const int nw = bt_waves(tr), np = (n - 2) / B / nw + 1;
+    std::vector<std::pair<int, int>> segs; // (first, last) pass, in application order
+    i64 acc = 0;
+    for (int k = 0; k < np; ++k) {
+        const int p = tr ? np - 1 - k : k;
+        if (bt_gmax<B>(n, p * nw) < 0) continue;
+        if (acc == 0) segs.emplace_back(p, p);
+        segs.back().second = p;
+        for (int w = 0; w < nw; ++w) acc += bt_gmax<B>(n, p * nw + w) + 1;
+        if (acc >= kBtSegBlocks) acc = 0;
+    }
+    const dim3 grid((unsigned)ceil_div(nc, 16 * NCT));
+    const auto kernel = tr ? bc_back_kernel<T, B, true, NCT> : bc_back_kernel<T, B, false, NCT>;
+    for (const auto &sg : segs) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), 0, s, ws.BtT, ws.bt_off, ws.bt_blocks, zp, M, ldm, n, nc,
+                           sg.first, sg.second);
+        CUEV_LAUNCH_CHECK();
+    }
+    return CUEV_STATUS_SUCCESS;
 }
 
 template <typename T, int B>
@@ -721,70 +412,17 @@ int launch_bc_back(Workspace<T> &ws, hipStream_t s, const T *U, T *M, i64 ldm, b
     // 4 flops per reflector entry per column: sum_s (n-1-s) entries ~ n^2/2
     prof::Scope sc(s, "bt.bc_back", 2.0 * (double)n * n * n);
     const T *zp = U + ws.ldu * (i64)n; // zeros past U's last column
-    // Columns in chunks of one resident round each (one wave per 16 columns, waves
-    // that start together): every wave streams the same block operands, and waves
-    // that start together share them in L2. In one launch of more waves than fit, the
-    // later rounds start as earlier waves finish, spread out along the stream, and
-    // lose that sharing (n = 49152, transposed: 10.6 s in one launch, 6.9 s in three).
-    int per_cu = 0;
-    if constexpr (B == 64)
-        CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bc_back_pair_kernel<T, B, true>,
-                                                              kBBThreads, 0));
-    else
-        CUEV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bc_back_kernel<T, B, true>,
-                                                              kBBThreads, 0));
-    const i64 cols_per_block = 16 * (kBBThreads / 64);
-    const i64 chunk = std::max<i64>(1, (i64)per_cu * device_cu_count()) * cols_per_block;
-    // The paired kernel's passes in launches of at least kBtSegBlocks blocks each (the
-    // last one fewer): the waves of one launch drift apart along the block stream as
-    // it goes, and a launch boundary lines them up again (measured at n = 16384,
-    // 1.3e5 blocks: one launch 252-260 ms, two 245 ms, four 243.6 ms, eight 244.7 ms,
-    // sixteen 245.3 ms; at n = 49152, 1.18e6 blocks per column chunk: one launch
-    // 7.6-12 s, nine 6.6 s).
-    std::vector<std::pair<int, int>> segs; // (first, last) pass start hops, in application order
-    if constexpr (B == 64) {
-        auto gmax = [&](int h) {
-            const int m = std::min(n - 3, n - 2 - h * B);
-            return m < 0 ? -1 : m / kBtGroup;
-        };
-        std::vector<int> passes;
-        if (tr) {
-            for (int h0 = ((n - 2) / B) / 2 * 2; h0 >= 0; h0 -= 2) passes.push_back(h0);
-        } else {
-            for (int h0 = 0; gmax(h0) >= 0; h0 += 2) passes.push_back(h0);
-        }
-        i64 acc = 0;
-        for (size_t q = 0; q < passes.size(); ++q) {
-            if (acc == 0) segs.emplace_back(passes[q], passes[q]);
-            segs.back().second = passes[q];
-            acc += (i64)(gmax(passes[q]) + 1) + (i64)(gmax(passes[q] + 1) + 1);
-            if (acc >= kBtSegBlocks) acc = 0;
-        }
-    }
-    for (i64 c0 = 0; c0 < n; c0 += chunk) {
-        const int nc = (int)std::min<i64>(chunk, n - c0);
-        const dim3 grid((unsigned)ceil_div(nc, cols_per_block));
-        T *Mc = M + c0 * ldm;
-        if constexpr (B == 64) {
-            // two blocks per step (passes of two hops: the default band's window fits)
-            for (const auto &sg : segs) {
-                if (tr)
-                    hipLaunchKernelGGL((bc_back_pair_kernel<T, B, true>), grid, dim3(kBBThreads), 0, s, ws.BtT,
-                                       ws.bt_off, ws.bt_blocks, zp, Mc, ldm, n, nc, sg.first, sg.second);
-                else
-                    hipLaunchKernelGGL((bc_back_pair_kernel<T, B, false>), grid, dim3(kBBThreads), 0, s, ws.BtT,
-                                       ws.bt_off, ws.bt_blocks, zp, Mc, ldm, n, nc, sg.first, sg.second);
-                CUEV_LAUNCH_CHECK();
-            }
-        } else {
-            if (tr)
-                hipLaunchKernelGGL((bc_back_kernel<T, B, true>), grid, dim3(kBBThreads), 0, s, ws.BtT,
-                                   ws.bt_off, zp, Mc, ldm, n, nc);
-            else
-                hipLaunchKernelGGL((bc_back_kernel<T, B, false>), grid, dim3(kBBThreads), 0, s, ws.BtT,
-                                   ws.bt_off, zp, Mc, ldm, n, nc);
-        }
-        CUEV_LAUNCH_CHECK();
+    // Columns in chunks of one workgroup per CU: every workgroup streams the same block operands,
+    // and those that start together share them in L2 (in one launch of more, the later ones
+    // would start as earlier ones finish and lose that). 32 columns per workgroup take 1.5 times as
+    // long as 16 (each operand read serves two products), so 16 where that covers what is left.
+    const i64 ncu = device_cu_count();
+    for (i64 c0 = 0; c0 < n;) {
+        const bool wide = n - c0 > 16 * ncu;
+        const int nc = (int)std::min<i64>(wide ? 32 * ncu : 16 * ncu, n - c0);
+        CUEV_TRY((wide ? launch_bc_passes<T, B, 2>(ws, s, M + c0 * ldm, ldm, nc, tr, zp)
+                       : launch_bc_passes<T, B, 1>(ws, s, M + c0 * ldm, ldm, nc, tr, zp)));
+        c0 += nc;
     }
     return CUEV_STATUS_SUCCESS;
 }
