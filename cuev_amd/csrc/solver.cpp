@@ -66,6 +66,10 @@ int kDcGateFrom(int n) { return std::min(n / 4, 4096); }
 // 6.96 and 18.6 ms in the direct order and 0.84, 1.71, 2.97, 6.10 and 15.0 ms reordered
 // (FP64, b = 32). Below about 64 there is one panel and nothing to hide.
 constexpr int kReorderedFrom = 64;
+// Once every stage fills the GPU by itself, running two side by side only makes them share it, and the
+// reordered order has 4/3 n^3 flops more. FP64 (b = 64): n = 10000 218 ms reordered and 224 direct,
+// 12000 319 and 316, 16384 702 and 634; FP32: 6000 60.8 and 61.7, 8192 98.1 and 97.4, 16384 493 and 430.
+template <typename T> constexpr int kDirectFrom = sizeof(T) == 8 ? 12000 : 8000;
 
 template <typename T>
 int tridi_dc(Context<T> &ctx, T *d, T *e, T *eval, T *evec, i64 ldv, double *dc_ms) {
@@ -122,7 +126,8 @@ int solve_native(Context<T> &ctx, T *A, T *eval, T *evec, cuev_solve_timer *time
     hipStream_t s = ws.stream;
     hipEvent_t *ev = ctx.ev;
     const auto wall0 = clk::now();
-    if (bt_mode == CUEV_BT_AUTO) bt_mode = (n >= kReorderedFrom) ? CUEV_BT_REORDERED : CUEV_BT_DIRECT;
+    if (bt_mode == CUEV_BT_AUTO)
+        bt_mode = (n >= kReorderedFrom && n < kDirectFrom<T>) ? CUEV_BT_REORDERED : CUEV_BT_DIRECT;
     const bool reordered = bt_mode == CUEV_BT_REORDERED;
     if (dc_mode == CUEV_DC_AUTO) dc_mode = (n >= kDeviceDcFrom) ? CUEV_DC_DEVICE : CUEV_DC_HOST;
     const bool dev_dc = dc_mode == CUEV_DC_DEVICE;

@@ -100,7 +100,7 @@ typedef enum cuev_precision_t {
 } cuev_precision_t;
 
 typedef enum cuev_bt_mode_t {
-    CUEV_BT_AUTO = 0,      /* reordered for n >= 64, direct otherwise */
+    CUEV_BT_AUTO = 0,      /* reordered for 64 <= n < 12000 (FP32: 8000), direct otherwise */
     CUEV_BT_DIRECT = 1,    /* evec <- Q_s (Q_b Q_d) after the D&C (reference order) */
     CUEV_BT_REORDERED = 2  /* build Q_b^T Q_s^T on the GPU beside the chase and the D&C, then one GEMM */
 } cuev_bt_mode_t;
