@@ -153,7 +153,9 @@ template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_ker
     __syncthreads();
 
     bool alive = true;
-    for (int c = 0; c <= b; ++c) {
+    // past the last row there is only the Gram column of the last reflector left to form
+    const int steps = min(b, a.rows);
+    for (int c = 0; c <= steps; ++c) {
         const int buf = c & 1;
         const bool has_col = c < b && c < a.rows;
         const int ndot = has_col ? b - c : 0;           // q = 0: ||x||^2, q >= 1: x^T a_{c+q}
@@ -205,7 +207,10 @@ template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_ker
         }
 
         // (2) grid-wide reduction
-        if (!grid_barrier(a.counter, (unsigned)a.G * (unsigned)(c + 1), a.err)) alive = false;
+        if (a.G == 1) { // one workgroup (the last panels): no grid to wait for
+            wave_stores_done();
+            __syncthreads();
+        } else if (!grid_barrier(a.counter, (unsigned)a.G * (unsigned)(c + 1), a.err)) alive = false;
 
         // Sum the G partial vectors: 4 threads per payload entry, each taking every
         // 4th workgroup with its loads issued back to back, then a fixed-order
@@ -243,7 +248,7 @@ template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_ker
         if (ngram)
             for (int i = tid; i < ngram; i += kPQThreads) GT[i + (size_t)(c - 1) * (b + 1)] = sums[b + i];
         if (!has_col) {
-            if (c < b && tid == 0) tauv[c] = 0.0;
+            for (int j = c + tid; j < b; j += kPQThreads) tauv[j] = 0.0;
             __syncthreads();
             continue;
         }
@@ -292,8 +297,8 @@ template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_ker
     }
     (void)alive;
 
-    // (5) T from the Gram matrix: column j overwrites Gram column j
-    for (int j = 0; j < b; ++j) {
+    // (5) T from the Gram matrix: column j overwrites Gram column j (zero past the last row)
+    for (int j = 0; j < steps; ++j) {
         double t = 0.0;
         if (tid < j) {
             for (int q = tid; q < j; ++q) t += GT[tid + (size_t)q * (b + 1)] * GT[q + (size_t)j * (b + 1)];
@@ -849,6 +854,9 @@ __global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
         }
     }
 
+    // with b rows the last column has nothing below its pivot, where LAPACK's H is the identity (tau
+    // = 0) and the one found here only changes the sign of R's last entry: leave it out
+    const bool square = a.rows == B;
     if (g == 0) {
         cq_lu<B>(P, ldp, MC, MC, a.bc, sv, wave, lane);
         if (tid == 0) *a.gate = 0;
@@ -881,8 +889,8 @@ __global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
         // panel rows 0..b-1 of A: R_house = S R on and above the diagonal, L below
         for (int idx = tid; idx < BB; idx += kCQThreads) {
             const int r = idx % B, j = idx / B;
-            const double l = MC[r + j * LD];
-            a.A[(i64)r + (i64)j * a.lda] = (T)((j >= r) ? sv[r] * MA[r + j * LD] : l);
+            const double l = MC[r + j * LD], s = (square && r == B - 1) ? -sv[r] : sv[r];
+            a.A[(i64)r + (i64)j * a.lda] = (T)((j >= r) ? s * MA[r + j * LD] : l);
             if (a.Y) a.Y[(i64)r + (i64)j * a.ldy] = (T)((j < r) ? l : (j == r ? 1.0 : 0.0));
         }
         __syncthreads();
@@ -937,7 +945,7 @@ __global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     const i64 j = 16 * Jt[c] + 4 * u + lk;
-                    if (a.W) a.W[r + j * a.ldw] = (T)w[c][u];
+                    if (a.W) a.W[r + j * a.ldw] = square && j == B - 1 ? T(0) : (T)w[c][u];
                     if (16 * I >= ylo) {
                         a.A[r + j * a.lda] = (T)y[c][u];
                         if (a.Y) a.Y[r + j * a.ldy] = (T)y[c][u];
@@ -953,8 +961,9 @@ __global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int i = 16 * I + 4 * u + lk, j = 16 * J + lr;
-                a.Tm[i + (size_t)j * B] = (T)acc[u];
-                if (i == j) a.tau[j] = (T)acc[u];
+                const T t_ij = square && j == B - 1 ? T(0) : (T)acc[u];
+                a.Tm[i + (size_t)j * B] = t_ij;
+                if (i == j) a.tau[j] = t_ij;
             }
         }
     }
@@ -999,8 +1008,8 @@ size_t panel_qr_scratch_bytes(int n, int b) {
 
 namespace {
 
-// CholQR2 launch if the panel qualifies: b in {16, 32, 64}, at least 2b rows, and
-// rows spread one workgroup per CU with at most kCQMaxCH rows each.
+// CholQR2 launch if the panel qualifies: b in {16, 32, 64}, at least b rows, and rows spread one
+// workgroup per CU with at most kCQMaxCH rows each.
 template <typename T, int B>
 int launch_cholqr(hipStream_t s, T *A, i64 lda, T *Y, i64 ldy, T *W, i64 ldw, T *Tm, T *tau, int rows,
                   void *scratch, size_t scratch_bytes, unsigned *counter, int *err, bool *launched) {
@@ -1059,7 +1068,7 @@ int panel_qr(hipStream_t s, T *A, i64 lda, T *Y, i64 ldy, T *W, i64 ldw, T *Tm, 
     // follows it, the Householder kernel, always launched, the CholQR counter for the
     // next panel), and without a CholQR launch counter[1] is zeroed here.
     bool cq = false;
-    if (rows >= 2 * b) {
+    if (rows >= b) {
         if (b == 64)
             CUEV_TRY((launch_cholqr<T, 64>(s, A, lda, Y, ldy, W, ldw, Tm, tau, rows, scratch, scratch_bytes,
                                            counter, err, &cq)));
