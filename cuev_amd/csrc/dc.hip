@@ -5,7 +5,8 @@
 // tridi.cu:241-418 both follow):
 //  * scale T by its largest entry; tear it recursively into halves, subtracting
 //    |e| at each cut from the two neighbouring diagonal entries (Cuppen 1981);
-//  * leaves (<= leaf size) by implicit QL/QR (host ?steqr, one thread per leaf);
+//  * leaves (<= leaf size) by the small solver's tridiagonal steps, a workgroup each (small.hip);
+//    leaves of more than 64 rows, on request, by implicit QL/QR (host ?steqr, one thread each);
 //  * merge T1 (+) T2 + rho v v^T bottom up. Per merge:
 //      - z = [last row of Q1, first row of Q2]; rho < 0 flips z2; z /= sqrt 2,
 //        rho <- 2|rho| (LAPACK dlaed2's normalisation);
@@ -40,6 +41,7 @@
 
 #include "lapack.hpp"
 #include "profile.hpp"
+#include "small.hpp"
 #include "util.hpp"
 
 namespace cuev {
@@ -68,6 +70,7 @@ struct LeafDesc {
     int off, sz;
     i64 soff; // element offset of the leaf's eigenvectors in the staging block
 };
+static_assert(sizeof(SmallLeaf) <= sizeof(LeafDesc), "either table fits the upload");
 
 template <typename T> struct Eps;
 template <> struct Eps<double> {
@@ -354,9 +357,10 @@ __global__ void dc_scale_kernel(const T *src, T *dst, int n, T s) {
 // host side
 // ---------------------------------------------------------------------------
 
-template <typename F> void parallel_for(int count, F &&f) {
+// f(0) .. f(count - 1), on up to max_threads threads
+template <typename F> void parallel_for(int count, int max_threads, F &&f) {
     const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
-    const int nt = std::min({count, hw, 16});
+    const int nt = std::min({count, hw, 16, max_threads});
     if (nt <= 1) {
         for (int i = 0; i < count; ++i) f(i);
         return;
@@ -585,6 +589,13 @@ template <typename T> void dc_state_destroy(DcState<T> *st) {
     delete st;
 }
 
+// eigenvalues of the leaves are NaN where the solver did not converge
+template <typename T> int check_leaves(int n, const T *val) {
+    for (int i = 0; i < n; ++i)
+        if (val[i] != val[i]) CUEV_FAIL(CUEV_STATUS_LAPACK_ERROR, "dc: QL on the leaf at row %d did not converge", i);
+    return CUEV_STATUS_SUCCESS;
+}
+
 template <typename T>
 int dc_solve(DcState<T> &st, hipStream_t s, int n, const T *d, const T *e, T *Q, i64 ldq, T *eval,
              T *Qc, T *S, T *Qn, Scratch gs, int leaf, hipEvent_t gate, int gate_from) {
@@ -621,54 +632,78 @@ int dc_solve(DcState<T> &st, hipStream_t s, int n, const T *d, const T *e, T *Q,
         ds[m.off + m.n1] -= r;
     }
 
-    // ---- leaves on the host, in parallel
     const UploadLayout &L = st.L;
     char *up = st.h_up;
-    LeafDesc *lv = reinterpret_cast<LeafDesc *>(up + L.leaves);
-    int *leaf_of = reinterpret_cast<int *>(up + L.leaf_of);
-    i64 soff = 0;
-    for (size_t i = 0; i < leaves.size(); ++i) {
-        lv[i] = {leaves[i].first, leaves[i].second, soff};
-        for (int c = 0; c < leaves[i].second; ++c) leaf_of[leaves[i].first + c] = (int)i;
-        soff += (i64)leaves[i].second * leaves[i].second;
-    }
-    const i64 vals_off = soff; // sum of leaf sizes squared <= n^2: fits Qn
-    st.leaf_stage.resize((size_t)(vals_off + n));
-    T *stage = st.leaf_stage.data();
-    std::atomic<int> leaf_info{0};
-    {
+    int max_leaf = 0;
+    for (const auto &lf : leaves) max_leaf = std::max(max_leaf, lf.second);
+    T *hz = st.h_zd, *hval = st.h_zd + n;
+    if (max_leaf <= kSmallTridiMaxN) {
+        // ---- leaves on the GPU, a workgroup each: d and e through d_z and d_tau (free until the merges)
+        SmallLeaf *lv = reinterpret_cast<SmallLeaf *>(up + L.leaves);
+        for (size_t i = 0; i < leaves.size(); ++i) lv[i] = {leaves[i].first, leaves[i].second};
+        for (int i = 0; i < n; ++i) {
+            hz[i] = ds[i];
+            hval[i] = i + 1 < n ? es[i] : T(0);
+        }
         prof::Scope sc(s, "dc.leaves");
-        parallel_for((int)leaves.size(), [&](int i) {
-            const int off = lv[i].off, sz = lv[i].sz;
-            T *z = stage + lv[i].soff;
-            T *dv = stage + vals_off + off;
-            std::vector<T> ee(std::max(sz - 1, 1)), work(std::max(2 * sz - 2, 1));
-            for (int j = 0; j < sz; ++j) dv[j] = ds[off + j];
-            for (int j = 0; j + 1 < sz; ++j) ee[j] = es[off + j];
-            const char compz = 'I';
-            int nn = sz, ldz = sz, info = 0;
-            if constexpr (sizeof(T) == 8)
-                lp->dsteqr(&compz, &nn, (double *)dv, (double *)ee.data(), (double *)z, &ldz,
-                           (double *)work.data(), &info);
-            else
-                lp->ssteqr(&compz, &nn, (float *)dv, (float *)ee.data(), (float *)z, &ldz,
-                           (float *)work.data(), &info);
-            if (info != 0) leaf_info.store(info);
-        });
+        CUEV_HIP(hipMemcpyAsync(st.d_z, hz, sizeof(T) * (size_t)n, hipMemcpyHostToDevice, s));
+        CUEV_HIP(hipMemcpyAsync(st.d_tau, hval, sizeof(T) * (size_t)n, hipMemcpyHostToDevice, s));
+        CUEV_HIP(hipMemcpyAsync(st.d_up + L.leaves, lv, sizeof(SmallLeaf) * leaves.size(), hipMemcpyHostToDevice, s));
+        CUEV_TRY(small_tridi<T>(s, st.d_z, st.d_tau, reinterpret_cast<const SmallLeaf *>(st.d_up + L.leaves),
+                                (int)leaves.size(), max_leaf, st.d_val, Q, ldq));
+        if (merges.empty()) {
+            CUEV_HIP(hipMemcpyAsync(hval, st.d_val, sizeof(T) * n, hipMemcpyDeviceToHost, s));
+            CUEV_HIP(hipStreamSynchronize(s));
+            CUEV_TRY(check_leaves(n, hval));
+        }
+    } else {
+        // ---- larger leaves, asked for by the caller: on the host, in parallel
+        LeafDesc *lv = reinterpret_cast<LeafDesc *>(up + L.leaves);
+        int *leaf_of = reinterpret_cast<int *>(up + L.leaf_of);
+        i64 soff = 0;
+        for (size_t i = 0; i < leaves.size(); ++i) {
+            lv[i] = {leaves[i].first, leaves[i].second, soff};
+            for (int c = 0; c < leaves[i].second; ++c) leaf_of[leaves[i].first + c] = (int)i;
+            soff += (i64)leaves[i].second * leaves[i].second;
+        }
+        const i64 vals_off = soff; // sum of leaf sizes squared <= n^2: fits Qn
+        st.leaf_stage.resize((size_t)(vals_off + n));
+        T *stage = st.leaf_stage.data();
+        std::atomic<int> leaf_info{0};
+        {
+            prof::Scope sc(s, "dc.leaves");
+            parallel_for((int)leaves.size(), 16, [&](int i) {
+                const int off = lv[i].off, sz = lv[i].sz;
+                T *z = stage + lv[i].soff;
+                T *dv = stage + vals_off + off;
+                std::vector<T> ee(std::max(sz - 1, 1)), work(std::max(2 * sz - 2, 1));
+                for (int j = 0; j < sz; ++j) dv[j] = ds[off + j];
+                for (int j = 0; j + 1 < sz; ++j) ee[j] = es[off + j];
+                const char compz = 'I';
+                int nn = sz, ldz = sz, info = 0;
+                if constexpr (sizeof(T) == 8)
+                    lp->dsteqr(&compz, &nn, (double *)dv, (double *)ee.data(), (double *)z, &ldz,
+                               (double *)work.data(), &info);
+                else
+                    lp->ssteqr(&compz, &nn, (float *)dv, (float *)ee.data(), (float *)z, &ldz,
+                               (float *)work.data(), &info);
+                if (info != 0) leaf_info.store(info);
+            });
+        }
+        if (leaf_info.load() != 0)
+            CUEV_FAIL(CUEV_STATUS_LAPACK_ERROR, "dc: ?steqr on a leaf returned %d", leaf_info.load());
+        // leaf eigenvectors through Qn (free until the first merge), eigenvalues through d_z
+        CUEV_HIP(hipMemcpyAsync(Qn, stage, sizeof(T) * (size_t)vals_off, hipMemcpyHostToDevice, s));
+        CUEV_HIP(hipMemcpyAsync(st.d_z, stage + vals_off, sizeof(T) * (size_t)n, hipMemcpyHostToDevice, s));
+        CUEV_HIP(hipMemcpyAsync(st.d_up + L.leaf_of, up + L.leaf_of, sizeof(int) * (size_t)n,
+                                hipMemcpyHostToDevice, s));
+        CUEV_HIP(hipMemcpyAsync(st.d_up + L.leaves, up + L.leaves, sizeof(LeafDesc) * leaves.size(),
+                                hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(dc_leaf_kernel<T>, dim3((unsigned)n), dim3(256), 0, s, Q, ldq, st.d_val, Qn,
+                           st.d_z, reinterpret_cast<const int *>(st.d_up + L.leaf_of),
+                           reinterpret_cast<const LeafDesc *>(st.d_up + L.leaves));
+        CUEV_LAUNCH_CHECK();
     }
-    if (leaf_info.load() != 0)
-        CUEV_FAIL(CUEV_STATUS_LAPACK_ERROR, "dc: ?steqr on a leaf returned %d", leaf_info.load());
-    // leaf eigenvectors through Qn (free until the first merge), eigenvalues through d_z
-    CUEV_HIP(hipMemcpyAsync(Qn, stage, sizeof(T) * (size_t)vals_off, hipMemcpyHostToDevice, s));
-    CUEV_HIP(hipMemcpyAsync(st.d_z, stage + vals_off, sizeof(T) * (size_t)n, hipMemcpyHostToDevice, s));
-    CUEV_HIP(hipMemcpyAsync(st.d_up + L.leaf_of, up + L.leaf_of, sizeof(int) * (size_t)n,
-                            hipMemcpyHostToDevice, s));
-    CUEV_HIP(hipMemcpyAsync(st.d_up + L.leaves, up + L.leaves, sizeof(LeafDesc) * leaves.size(),
-                            hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(dc_leaf_kernel<T>, dim3((unsigned)n), dim3(256), 0, s, Q, ldq, st.d_val, Qn,
-                       st.d_z, reinterpret_cast<const int *>(st.d_up + L.leaf_of),
-                       reinterpret_cast<const LeafDesc *>(st.d_up + L.leaves));
-    CUEV_LAUNCH_CHECK();
 
     // ---- merges, deepest level first
     MergeDesc *md = reinterpret_cast<MergeDesc *>(up + L.md);
@@ -676,7 +711,6 @@ int dc_solve(DcState<T> &st, hipStream_t s, int n, const T *d, const T *e, T *Q,
     const MergeDesc *d_md = reinterpret_cast<const MergeDesc *>(st.d_up + L.md);
     const MergeDesc *d_md0 = reinterpret_cast<const MergeDesc *>(st.d_up + L.md0);
     std::vector<MergeHost<T>> mh;
-    T *hz = st.h_zd, *hval = st.h_zd + n;
     for (int depth = maxdepth; depth >= 0; --depth) {
         std::vector<const Node *> lev;
         for (const Node &m : merges)
@@ -708,9 +742,11 @@ int dc_solve(DcState<T> &st, hipStream_t s, int n, const T *d, const T *e, T *Q,
         CUEV_HIP(hipMemcpyAsync(hz, st.d_z, sizeof(T) * n, hipMemcpyDeviceToHost, s));
         CUEV_HIP(hipMemcpyAsync(hval, st.d_val, sizeof(T) * n, hipMemcpyDeviceToHost, s));
         CUEV_HIP(hipStreamSynchronize(s));
+        if (depth == maxdepth) CUEV_TRY(check_leaves(n, hval));
 
         mh.resize(nm);
-        parallel_for(nm, [&](int i) {
+        // (starting a thread costs about as much as deflating 500 rows)
+        parallel_for(nm, 1 + n / 2048, [&](int i) {
             const Node &m = *lev[i];
             deflate<T>(m.off, m.N, m.n1, es[m.off + m.n1 - 1], hval + m.off, hz + m.off, mh[i]);
         });

@@ -147,10 +147,12 @@ __device__ bool ql_sweep(double *d, double *e, int n, int &l, int &m, int &lo, d
     return true;
 }
 
-// NT threads, orders up to 16 NB
-template <typename T, int NT, int NB>
-__global__ __launch_bounds__(NT) void small_eig_kernel(const T *Ag, int n, T *W, T *V, int il, int iu, int allow_ql,
-                                                       int *dflags, int *hflag) {
+// One matrix per workgroup of NT threads, orders up to 16 NB. TRI: the matrix is tridiagonal, block
+// `leaf` of the rows of (Ag, Eg), and steps 1 and 5 fall away; the eigenvalues go to W and the
+// eigenvectors to the diagonal block of V (ld ldv) at the block's rows; eigenvalues NaN if QL fails.
+template <typename T, int NT, int NB, bool TRI>
+__device__ __forceinline__ void small_eig_body(const T *Ag, const T *Eg, int n, SmallLeaf leaf, T *W, T *V, i64 ldv, int il,
+                                               int iu, int allow_ql, int *dflags, int *hflag) {
     constexpr int NW = NT / 64;
     constexpr int NBW = NB / NW > 1 ? NB / NW : 1; // column blocks of Z per wave in step 4
     constexpr int LPC = NT / (16 * NB);            // lanes per column in step 5
@@ -167,18 +169,39 @@ __global__ __launch_bounds__(NT) void small_eig_kernel(const T *Ag, int n, T *W,
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const i64 mat = (i64)n * n;
-    const T *A = Ag + (i64)blockIdx.x * mat;
+    const T *A = Ag + (TRI ? leaf.off : (i64)blockIdx.x * mat);
     unsigned *wg = reinterpret_cast<unsigned *>(V + (V ? (i64)blockIdx.x * mat : 0)); // packed reflectors, n (n - 1) words
     const int nout = V ? n : iu - il + 1;
-    T *Wo = W + (i64)blockIdx.x * nout;
+    T *Wo = W + (TRI ? leaf.off : (i64)blockIdx.x * nout);
+    bool unconverged = false; // TRI
 
     auto fail = [&](int which) { // host flag only on failure: a good call needs no copy back
-        if (tid == 0) {
+        if (TRI) unconverged = true;
+        else if (tid == 0) {
             atomicAdd(dflags + which, 1);
             __hip_atomic_store(hflag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     };
 
+    int ts;
+    if constexpr (TRI) {
+        double amax = 0.0;
+        for (int i = tid; i < n; i += NT) {
+            sd[i] = (double)A[i];
+            se[i] = i < n - 1 ? (double)Eg[leaf.off + i] : 0.0;
+        }
+        __syncthreads();
+        for (int i = lane; i < n; i += 64) amax = fmax(amax, fmax(fabs(sd[i]), fabs(se[i])));
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) amax = fmax(amax, __shfl_xor(amax, o, 64));
+        ts = amax > 0.0 ? ilogb(amax) + 1 : 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += NT) {
+            sd[i] = ldexp(sd[i], -ts);
+            se[i] = ldexp(se[i], -ts);
+        }
+        __syncthreads();
+    } else {
     // ---- load the lower triangle, scale so that the largest entry is in [1/2, 1)
     double amax = 0.0;
     bool bad = false;
@@ -203,7 +226,7 @@ __global__ __launch_bounds__(NT) void small_eig_kernel(const T *Ag, int n, T *W,
     __syncthreads();
 #pragma unroll
     for (int g = 0; g < NW; ++g) amax = fmax(amax, part[g]);
-    const int ts = amax > 0.0 ? ilogb(amax) + 1 : 0;
+    ts = amax > 0.0 ? ilogb(amax) + 1 : 0;
     for (int j = wave; j < n; j += NW)
         for (int i = j + lane; i < n; i += 64) {
             const double v = ldexp(R[j * ld + i], -ts);
@@ -359,6 +382,8 @@ __global__ __launch_bounds__(NT) void small_eig_kernel(const T *Ag, int n, T *W,
                 }
         }
     }
+
+    } // !TRI
 
     // ---- 2. eigenvalues of T: L lanes each
     double tnorm;
@@ -630,6 +655,16 @@ __global__ __launch_bounds__(NT) void small_eig_kernel(const T *Ag, int n, T *W,
         __syncthreads();
     }
 
+    if constexpr (TRI) {
+        const double bad = __syncthreads_or(unconverged) ? __builtin_nan("") : 0.0;
+        for (int j = wave; j < n; j += NW) {
+            const int pos = rank(j);
+            if (lane == 0) Wo[pos] = (T)(ldexp(slam[j], ts) + bad);
+            for (int i = lane; i < n; i += 64) V[leaf.off + i + (i64)(leaf.off + pos) * ldv] = (T)R[i * ldz + j];
+        }
+        return;
+    }
+
     // ---- 5. V = H_0 ... H_{n-3} Z: LPC neighbouring lanes per column, rows 2 (t LPC + q) + {0, 1}
     const int j = tid / LPC, q = tid % LPC;
     double2 z[RP];
@@ -687,6 +722,17 @@ __global__ __launch_bounds__(NT) void small_eig_kernel(const T *Ag, int n, T *W,
             if (i + 1 < n) vo[i + 1] = (T)z[t].y;
         }
     }
+}
+
+template <typename T, int NT, int NB>
+__global__ __launch_bounds__(NT) void small_eig_kernel(const T *A, int n, T *W, T *V, int il, int iu, int allow_ql,
+                                                       int *dflags, int *hflag) {
+    small_eig_body<T, NT, NB, false>(A, nullptr, n, SmallLeaf{}, W, V, 0, il, iu, allow_ql, dflags, hflag);
+}
+template <typename T, int NT, int NB>
+__global__ __launch_bounds__(NT) void small_tridi_kernel(const T *d, const T *e, const SmallLeaf *leaves, T *W, T *V, i64 ldv) {
+    const SmallLeaf L = leaves[blockIdx.x];
+    small_eig_body<T, NT, NB, true>(d, e, L.sz, L, W, V, ldv, 0, L.sz - 1, 1, nullptr, nullptr);
 }
 
 template <typename T, int NT, int NB>
@@ -815,6 +861,22 @@ int small_eig(hipStream_t s, const T *A, int n, int batch, T *W, T *V, int il, i
     return CUEV_STATUS_SUCCESS;
 }
 
+template <typename T>
+int small_tridi(hipStream_t s, const T *d, const T *e, const SmallLeaf *leaves, int nleaves, int max_sz, T *W, T *V,
+                i64 ldv) {
+    if (max_sz < 1 || max_sz > kSmallTridiMaxN)
+        CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "small_tridi: order %d outside [1, %d]", max_sz, kSmallTridiMaxN);
+    const size_t lds = sizeof(double) * (size_t)small_lds(max_sz, 4).total;
+    CUEV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(small_tridi_kernel<T, 256, 4>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((small_tridi_kernel<T, 256, 4>), dim3((unsigned)nleaves), dim3(256), lds, s, d, e, leaves, W, V, ldv);
+    CUEV_LAUNCH_CHECK();
+    return CUEV_STATUS_SUCCESS;
+}
+
+template int small_tridi<float>(hipStream_t, const float *, const float *, const SmallLeaf *, int, int, float *, float *, i64);
+template int small_tridi<double>(hipStream_t, const double *, const double *, const SmallLeaf *, int, int, double *, double *,
+                                 i64);
 template int small_eig<float>(hipStream_t, const float *, int, int, float *, float *, int, int, int *, int *, int *);
 template int small_eig<double>(hipStream_t, const double *, int, int, double *, double *, int, int, int *, int *,
                                int *);

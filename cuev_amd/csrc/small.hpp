@@ -16,6 +16,18 @@ template <typename T>
 int small_eig(hipStream_t s, const T *A, int n, int batch, T *W, T *V, int il, int iu, int *n_failed,
               int *n_not_finite, int *n_need_ql = nullptr);
 
+// Diagonal blocks of a tridiagonal matrix, of order <= kSmallTridiMaxN each (device array, max_sz the
+// largest): block [off, off + sz) of the diagonal d, with couplings e[off .. off + sz - 2]. Eigenvalues,
+// ascending, to W[off ..], eigenvectors to the diagonal blocks of V (ld ldv; the rest of V is not
+// touched). Not blocking. Eigenvalues are NaN where the QL iteration did not converge.
+constexpr int kSmallTridiMaxN = 64;
+struct SmallLeaf {
+    int off, sz;
+};
+template <typename T>
+int small_tridi(hipStream_t s, const T *d, const T *e, const SmallLeaf *leaves, int nleaves, int max_sz, T *W, T *V,
+                i64 ldv);
+
 // frees the failure counters kept between calls, where no call is using them
 void small_release_all();
 
