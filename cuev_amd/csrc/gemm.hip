@@ -18,7 +18,8 @@
 // unaligned operands take a per-element path with bounds checks into the same LDS
 // layout. In LDS both operands are stored row-major with K contiguous ([m][k] and
 // [n][k]), rows padded by 16 bytes so that the fragment reads of 16 consecutive
-// rows hit distinct banks. A fragment read is one 16-byte ds_read per lane: lane
+// rows hit distinct banks, and the 16-byte chunks of a row are permuted by its 16-row block, so
+// that transposing stores do too. A fragment read is one 16-byte ds_read per lane: lane
 // (i = l%16, j = l/16) reads row i at k = E*j .. E*j+E-1 (E = 2 doubles / 4
 // floats), which feeds E MFMAs at once. Each MFMA then contracts lane group j's
 // k = E*j + e; A and B use the same k assignment, so the sum over the E MFMAs and
@@ -183,13 +184,18 @@ template <typename T, int R, int BK, int NT> struct TileRegs {
             }
         }
     }
-    // into LDS s[row][k] (row stride RS elements)
+    // 16-byte chunk of a row's LDS image that holds its k chunk kc
+    __device__ static __forceinline__ int slot(int row, int kc) { return kc ^ ((row >> 4) & 3); }
+    // into LDS s[row][k] (row stride RS elements), a row's chunks permuted by slot(): a wave
+    // storing an RC tile writes E rows per lane at one k, and rows E apart fall on four (FP32) or
+    // eight (FP64) bank groups only without it. A fragment's 16 rows share one permutation.
+    // (FP32, n = 8192: N N 103 -> 121 TF/s, N T 89 -> 117, T N, with no such stores, 121.)
     template <int RS> __device__ __forceinline__ void store(int lay, T *s, int tid) const {
         if (lay == L_KC) {
 #pragma unroll
             for (int q = 0; q < CH; ++q) {
                 const int c = tid + q * NT;
-                *reinterpret_cast<vec *>(s + (c / KCH) * RS + (c % KCH) * E) = v[q];
+                *reinterpret_cast<vec *>(s + (c / KCH) * RS + slot(c / KCH, c % KCH) * E) = v[q];
             }
         } else {
 #pragma unroll
@@ -197,7 +203,7 @@ template <typename T, int R, int BK, int NT> struct TileRegs {
                 const int c = tid + q * NT;
                 const int kk = c / RCH, r = (c % RCH) * E;
 #pragma unroll
-                for (int e = 0; e < E; ++e) s[(r + e) * RS + kk] = v[q][e];
+                for (int e = 0; e < E; ++e) s[(r + e) * RS + slot(r + e, kk / E) * E + kk % E] = v[q][e];
             }
         }
     }
@@ -320,15 +326,19 @@ __device__ __forceinline__ void gemm_body_regs(const KParams<T> &p) {
         const int cur = kt & 1;
         const bool more = kt + 1 < nkt;
         if (more) load_tiles(kbeg + (i64)(kt + 1) * BK);
-        const T *a_s = sA[cur] + (wm * TM + li) * RS + lj * E;
-        const T *b_s = sB[cur] + (wn * TN + li) * RS + lj * E;
+        const T *a_s = sA[cur] + (wm * TM + li) * RS;
+        const T *b_s = sB[cur] + (wn * TN + li) * RS;
 #pragma unroll
         for (int kg = 0; kg < BK / KG; ++kg) {
             vec af[FM], bf[FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const vec *>(a_s + i * 16 * RS + kg * KG);
+            for (int i = 0; i < FM; ++i)
+                af[i] = *reinterpret_cast<const vec *>(
+                    a_s + i * 16 * RS + TileRegs<T, BM, BK, NT>::slot(wm * TM + i * 16, 4 * kg + lj) * E);
 #pragma unroll
-            for (int j = 0; j < FN; ++j) bf[j] = *reinterpret_cast<const vec *>(b_s + j * 16 * RS + kg * KG);
+            for (int j = 0; j < FN; ++j)
+                bf[j] = *reinterpret_cast<const vec *>(
+                    b_s + j * 16 * RS + TileRegs<T, BN, BK, NT>::slot(wn * TN + j * 16, 4 * kg + lj) * E);
 #pragma unroll
             for (int e = 0; e < E; ++e)
 #pragma unroll
