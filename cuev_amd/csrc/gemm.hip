@@ -843,6 +843,21 @@ int gemm_ex(hipStream_t s, i64 M, i64 N, i64 K, T alpha, const Operand<T> &A,
     }
     const int BMs = cfg_bm(cfg), BNs = cfg_bn(cfg);
     const i64 ntiles = count_tiles(BMs, BNs);
+    // A few tiles more than a whole number of rounds over the CUs cost a whole round. Where they are
+    // at most half of one (and the rounds few, K long), the last tile columns become a product of
+    // their own, split along K over all CUs (n = 3000, 576 tiles on 256 CUs: FP32 0.74 -> 0.61 ms,
+    // FP64 1.18 -> 0.96).
+    if (cfg == C128x128 && !lower && !A.sym && B.split < 0 && K >= 1024 && scratch.bytes > 0) {
+        const i64 tm = ceil_div(M, 128), tn = ceil_div(N, 128), rounds = ntiles / cus;
+        const i64 tn1 = rounds * cus / tm; // tile columns of the whole rounds
+        if (rounds >= 2 && rounds <= 6 && tn1 > 0 && tn1 < tn && tm * (tn - tn1) <= cus / 2 &&
+            scratch.bytes >= (size_t)2 * M * (N - 128 * tn1) * sizeof(T)) {
+            Operand<T> B2 = B;
+            B2.p0 = B.trans ? B.p0 + 128 * tn1 : B.p0 + 128 * tn1 * B.ld0;
+            CUEV_TRY(gemm_ex<T>(s, M, 128 * tn1, K, alpha, A, B, beta, C, ldc, lower, scratch));
+            return gemm_ex<T>(s, M, N - 128 * tn1, K, alpha, A, B2, beta, C + 128 * tn1 * ldc, ldc, lower, scratch);
+        }
+    }
     if (ntiles > 0x7fffffffLL) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "gemm: too many tiles");
     p.tiles_m = (int)ceil_div(M, BMs);
     p.tiles_n = (int)ceil_div(N, BNs);
