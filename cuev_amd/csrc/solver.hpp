@@ -11,10 +11,11 @@ void options_defaults(cuev_options &o);
 // beside it (the gate of dc_solve).
 int kDcGateFrom(int n);
 
-// Order from which the device D&C beats host LAPACK's: at n = 130, 160, 256, 512 and 1000
-// ?stedc takes 0.40, 0.63, 1.5, 5.6 and 19.7 ms in FP64 (0.26, 0.40, 0.9, 3.3 and 11.5 in
-// FP32) and the device form 0.41, 0.45, 0.65, 1.0 and 1.9 (0.38, 0.41, 0.6, 1.0 and 1.7).
-constexpr int kDeviceDcFrom = 160;
+// Order from which the device D&C beats host LAPACK's: whole solves of n = 129, 140 and 159 take 1.20,
+// 1.33 and 1.69 ms with ?stedc in FP64 (0.97, 1.12 and 1.43 in FP32) and 1.08, 1.12 and 1.30 (0.99,
+// 1.05 and 1.27) with the device form; at n = 1000 the stage alone takes 19.7 (11.5) and 1.3
+// (1.0) ms. Up to 128 only solves with stage options get here.
+constexpr int kDeviceDcFrom = 129;
 
 // D&C on device (d, e): eval <- eigenvalues, evec (ld ldv) <- Q_d; host ?stedc
 // or the device-resident form, as ctx.dc_mode says.

@@ -106,7 +106,7 @@ typedef enum cuev_bt_mode_t {
 } cuev_bt_mode_t;
 
 typedef enum cuev_dc_mode_t {
-    CUEV_DC_AUTO = 0,   /* device for n >= 160, host otherwise */
+    CUEV_DC_AUTO = 0,   /* device for n > 128, host otherwise */
     CUEV_DC_HOST = 1,   /* host LAPACK ?stedc, Q_d uploaded (the reference's north-star form) */
     CUEV_DC_DEVICE = 2  /* divide and conquer with Q resident on the GPU: host deflation
                            bookkeeping and leaves, device secular roots, vectors and GEMMs
@@ -128,8 +128,9 @@ typedef struct cuev_options {
 /* The drop-in entry points keep the workspace of the last problem size per
  * device and precision for the next call (the reference allocates and frees it
  * on every call, src/cuda/handle.cu:73 and solver.cu:72). This frees every idle
- * cached workspace now; it must not race with a solve in progress. No reference
- * counterpart. */
+ * cached workspace now, and the buffers that the product, backward and small-order
+ * entry points keep between calls; it must not race with a solve in progress. No
+ * reference counterpart. */
 int cuev_cache_release(void);
 
 /* Fill *opt with the defaults listed above. */

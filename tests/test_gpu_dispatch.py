@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", ["d", "s"])
-@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 159, 160, 161, 255, 256, 257, 700])
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 127, 128, 129, 130, 159, 160, 161, 255, 256, 257, 700])
 def test_auto_options(torch_dev, n, prec):
     torch = torch_dev
     dt = torch.float64 if prec == "d" else torch.float32
