@@ -4,8 +4,8 @@
 Default workload: n = 16384, fp64, A = Q diag(lam) Q^T (Q: Householder-QR factor of
 a seeded Gaussian matrix, lam sorted iid U(-1,1)), bandwidth b = 64, block k = 512,
 all eigenvalues and eigenvectors. One step = one full cuev_dsymm_eig_solve call
-(DBBR -> bulge chasing -> device D&C beside the GPU build of Q_b^T Q_s^T -> final
-GEMM), input already resident in HBM; the copy of A that the solver consumes is
+(DBBR -> bulge chasing -> device D&C -> Q_b -> Q_s in the direct order, which
+"auto" takes at this size), input already resident in HBM; the copy of A that the solver consumes is
 made before each step's timer starts.
 
 --only chase|bcback|copy runs one kernel of interest and nothing else (for hardware
@@ -99,24 +99,6 @@ def cpu_baseline(n_sample, n_full, seed=1):
                       f"to n={n_full}"}
 
 
-def measured_traffic(tag, n, b):
-    """HBM bytes per launch of `tag` from the committed counter summary (FETCH_SIZE and
-    WRITE_SIZE, copy-calibrated), when it was measured for this n and b; else None."""
-    if tag != "bc.chase":
-        return None
-    path = os.path.join(ROOT, "profiles", "bc_chase_q16k_pmc.txt")
-    try:
-        text = open(path).read()
-    except OSError:
-        return None
-    if f"n = {n}, b = {b}" not in text:
-        return None
-    for line in text.splitlines():
-        if line.startswith("# traffic_bytes_per_launch"):
-            return float(line.split()[-1])
-    return None
-
-
 def residual_orth(torch, A0, V, lam, cols=2048):
     from cuev_amd import workloads
     return workloads.residual_orth(A0, V, lam, cols)
@@ -168,7 +150,7 @@ def run_only(which, n, b, k):
             return
     hops = n * n / (2.0 * b)
     print(json.dumps({"only": "chase", "n": n, "b": b, "seconds": dt,
-                      "algorithmic_bytes": hops * 4 * b * b * 8}))
+                      "algorithmic_bytes": hops * 9 * b * 8}))  # messages written and read, U written
 
 
 def run_diff(n, steps, warmup):
@@ -439,11 +421,10 @@ def main():
 def dominant_roofline(prof, n, b):
     """Roofline of the single-launch kernel site with the most GPU time per solve.
 
-    bc_chase (HBM/L2-bound): achieved = the algorithmic bytes of the model this build's
-    library records for it (per hop b columns loaded, b stored, each b x 2b: 4 b^2 S;
-    n^2 / (2b) hops), over its HIP-event duration; "frac_model_5p5bn2S" gives the same
-    duration against the 5.5 b n^2 S L2-traffic model of a kernel that re-reads its
-    window every hop. MFMA-bound kernels: the flops the library records per launch."""
+    bc_chase (latency-bound): achieved = the algorithmic bytes the library records for it (the
+    resident form: two messages of b tagged values written and read and b values of U written
+    per hop, 9 b S; n^2 / (2b) hops) over its HIP-event duration. MFMA-bound kernels: the flops
+    the library records per launch."""
     single = {"bc.chase": "hbm", "bt.bc_back": "mfma", "bt.gemm": "mfma"}
     dom = max((t for t in single if t in prof), key=lambda t: prof[t]["ms"], default=None)
     if not dom:
@@ -453,13 +434,9 @@ def dominant_roofline(prof, n, b):
     if single[dom] == "hbm":
         per_launch = r["bytes"] / r["count"]
         ach = per_launch / dur / 1e9
-        alt = 5.5 * b * n * n * 8 / dur / 1e9
         return {"kernel": dom, "bound": "hbm", "achieved": round(ach, 2), "peak": 8000.0,
                 "unit": "GB/s", "frac": round(ach / 8000.0, 4),
-                "traffic": measured_traffic(dom, n, b),
-                "traffic_source": "committed counter run profiles/bc_chase_q16k_pmc.txt "
-                                  "(FETCH_SIZE + WRITE_SIZE, copy-calibrated), not measured by this run",
-                "frac_model_5p5bn2S": round(alt / 8000.0, 4),
+                "traffic": None,
                 "avg_launch_ms": round(dur * 1e3, 3)}
     per_launch = r["flops"] / r["count"]
     ach = per_launch / dur / 1e12
