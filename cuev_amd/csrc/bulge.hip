@@ -918,16 +918,24 @@ template <typename T, int B, bool RECV> int chase_capacity(i64 *out) {
     return CUEV_STATUS_SUCCESS;
 }
 
+// LDS that the chase asks for on top of its own where it is to have its CUs to itself: what is left
+// (under 20 KB) is less than any product's tile needs. The products that run beside the chase in the
+// reordered order otherwise share the chase's CUs and slow its chain of short steps down.
+constexpr size_t kChasePad = 136 * 1024;
+
 template <typename T, int B, bool RECV>
-int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, int hops) {
+int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, int hops, size_t pad = 0) {
     const int n = ws.n;
     hipStream_t s = ws.stream;
+    if (pad)
+        CUEV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(bc_chase_resident_kernel<T, B, RECV>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)pad));
     const i64 words = (i64)(hops + 1) * 2 * msg_words<T>(B);
     CUEV_TRY(fill_int(s, reinterpret_cast<int *>(ws.chmsg), 2 * words, 0)); // no tag of an earlier chase
     const double nhops = (double)n * n / (2.0 * B);
     // each hop writes and reads two messages of b tagged values and writes b values of U
     prof::Scope sc(s, "bc.chase", nhops * (6.0 * B * B + 16.0 * B * B), nhops * 9.0 * B * sizeof(T));
-    hipLaunchKernelGGL((bc_chase_resident_kernel<T, B, RECV>), dim3((unsigned)hops), dim3(chase_threads(B, RECV)), 0, s,
+    hipLaunchKernelGGL((bc_chase_resident_kernel<T, B, RECV>), dim3((unsigned)hops), dim3(chase_threads(B, RECV)), pad, s,
                        Bp, ws.U, ws.ldu, n, d, e, reinterpret_cast<u64 *>(ws.chmsg), ws.err);
     CUEV_LAUNCH_CHECK();
     return CUEV_STATUS_SUCCESS;
@@ -938,13 +946,19 @@ int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, int hops) {
 // a receiving wave is taken where two such chases fit at once (b = 64 in FP64: n <= 16384;
 // two solves may share the GPU, as with the windowed form), the one without it, which has
 // more room, where one does (n <= 49152; at n = 16384 3.9 us per sweep, windowed 16.4).
+// A chase of at most a quarter of the CUs' number of hops (b = 64: n <= 4096) takes its CUs for itself:
+// four such chases, as many as a process has hardware queues by default, still fit at once. Whole
+// solves: FP64 n = 1024 7.14 -> 7.00 ms, 2500 19.65 -> 19.19, 4096 36.3 -> 34.8 (the chase 14.7 ->
+// 13.3), FP32 4096 29.7 -> 28.8. Up to half of them n = 8192 would gain as well (127.5 -> 120.2), but
+// only two chases would fit.
 template <typename T, int B> int try_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, bool *done) {
     const int hops = (ws.n - 2) / B + 1;
     i64 with = 0, without = 0;
     CUEV_TRY((chase_capacity<T, B, true>(&with)));
     CUEV_TRY((chase_capacity<T, B, false>(&without)));
     *done = true;
-    if (2 * hops <= with) return launch_chase_resident<T, B, true>(ws, Bp, d, e, hops);
+    if (2 * hops <= with)
+        return launch_chase_resident<T, B, true>(ws, Bp, d, e, hops, 4 * hops <= device_cu_count() ? kChasePad : 0);
     if (hops <= without) return launch_chase_resident<T, B, false>(ws, Bp, d, e, hops);
     *done = false;
     return CUEV_STATUS_SUCCESS;
