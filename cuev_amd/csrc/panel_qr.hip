@@ -419,6 +419,13 @@ __device__ __forceinline__ cq_v4 cq_mma(double a, double b, cq_v4 c) {
 // columns at a time, have b + 2.
 __host__ __device__ constexpr int cq_ldp(int CH) { return CH + (50 - CH % 32) % 32; }
 
+// x as a value the compiler knows nothing about: addresses formed with it in a loop, or after an
+// elimination, are formed there and not kept in registers from before.
+__device__ __forceinline__ int cq_fresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 // lower 16 x 16 tile q of a Gram matrix, row by row
 __device__ __forceinline__ void cq_tile(int q, int &I, int &J) {
     I = q >= 6 ? 3 : (q >= 3 ? 2 : (q >= 1 ? 1 : 0));
@@ -584,6 +591,7 @@ __device__ __forceinline__ bool cq_chol(double *P, int ldp, int CH, const double
         }
     __syncthreads();
     if (*s_bad) return false;
+    const int ln = cq_fresh(lane);
 #pragma unroll
     for (int lc = 0; lc < C::LC; ++lc)
 #pragma unroll
@@ -591,7 +599,7 @@ __device__ __forceinline__ bool cq_chol(double *P, int ldp, int CH, const double
             const int j = 4 * (kCQWaves * lc + wave) + u;
 #pragma unroll
             for (int t = 0; t < NSET; ++t) {
-                const int q = 64 * t + lane;
+                const int q = 64 * t + ln;
                 if (j < B && q < B) {
                     if (Rout) Rout[j + q * LD] = q < j ? 0.0 : g[t][4 * lc + u];
                 } else if (j < B && q < B + CH) P[(size_t)j * ldp + q - B] = g[t][4 * lc + u];
@@ -671,6 +679,7 @@ __device__ __forceinline__ void cq_lu(double *P, int ldp, double *LU, double *bu
             for (int u = 0; u < 4; ++u) z[4 * lc + u] -= l[v] * read_lane(z[4 * lc + u], 4 * c + v);
     };
     cq_eliminate<B>(wave, factor, load, apply, rest);
+    lane = cq_fresh(lane);
 #pragma unroll
     for (int lc = 0; lc < C::LC; ++lc)
 #pragma unroll
@@ -700,8 +709,11 @@ template <int B> __device__ __forceinline__ cq_v4 cq_upper_mm(const double *X, c
     return acc;
 }
 
+// Up to 64 rows per workgroup four waves per SIMD (112 VGPRs): a panel's workgroup then fits on a CU beside one of a
+// bulge chase of another solve. Both kinds wait for workgroups of their own to become resident, so
+// where they excluded each other, four solves of n = 8192 at once could block one another.
 template <typename T, int B, int NSET>
-__global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
+__global__ __launch_bounds__(kCQThreads, NSET == 2 ? 4 : 2) void panel_cholqr_kernel(CQArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     constexpr int LD = B + 2, BB = B * B, NTB = B / 16, NT = NTB * (NTB + 1) / 2, NE = 256 * NT;
     constexpr int NP = NTB > 2 ? NTB / 2 : 1; // pairs of column tiles {p, NTB - 1 - p}: equal work for triangular factors
@@ -748,6 +760,7 @@ __global__ __launch_bounds__(kCQThreads) void panel_cholqr_kernel(CQArgs<T> a) {
     unsigned nbar = 0;
 #pragma unroll 1
     for (int pass = 0; pass < 2; ++pass) {
+        const int tid = cq_fresh(threadIdx.x), lane = tid & 63, lr = lane & 15, lk = lane >> 4;
         // ---- Gram matrix of the panel: partials, then fixed-order slice sums
         cq_gram<B>(P, ldp, CH, a.part + (size_t)g * NE, wave, lane);
         if (!grid_barrier_wt(a.counter, (unsigned)a.G * ++nbar, a.err)) return;
