@@ -591,6 +591,8 @@ int run_mixed(Context<float> &cf, MixedBuffers &mb, double *A, int n, double *ev
     hipStream_t bs = cf.bt_stream;
     CUEV_HIP(hipEventRecord(ev[0], s));
     CUEV_TRY((convert2d<double, float>(s, A, n, ws.M, ws.ld, n, n)));
+    PersistentTurn turn;
+    CUEV_TRY(turn.begin(s, n, ws.b));
     CUEV_TRY(dbbr_reduce<float>(ws, ws.M, ws.B));
     CUEV_HIP(hipEventRecord(ev[1], s));
     // 2. M = Q_b^T Q_s^T in FP32 on the back-transform stream: Q_s^T beside the
@@ -600,6 +602,7 @@ int run_mixed(Context<float> &cf, MixedBuffers &mb, double *A, int n, double *ev
     CUEV_TRY(sbr_back_t<float>(ws, bs, ws.Y, ws.W, ws.M, ws.ld));
     CUEV_HIP(hipEventRecord(cf.xev[1], bs));
     CUEV_TRY(bc_chase<float>(ws, ws.B, ws.d, ws.e));
+    CUEV_TRY(turn.end());
     CUEV_HIP(hipEventRecord(ev[2], s));
     CUEV_HIP(hipMemcpyAsync(cf.h_d, ws.d, 4 * (size_t)n, hipMemcpyDeviceToHost, s));
     CUEV_HIP(hipMemcpyAsync(cf.h_e, ws.e, 4 * (size_t)n, hipMemcpyDeviceToHost, s));

@@ -135,10 +135,13 @@ int solve_native(Context<T> &ctx, T *A, T *eval, T *evec, cuev_solve_timer *time
     if (reordered) CUEV_TRY(bt_ensure(ctx));
     hipStream_t bs = ctx.bt_stream;
     CUEV_HIP(hipEventRecord(ev[0], s));
+    PersistentTurn turn;
+    CUEV_TRY(turn.begin(s, n, ws.b));
     CUEV_TRY(dbbr_reduce<T>(ws, A, ws.B));
     CUEV_HIP(hipEventRecord(ev[1], s));
     CUEV_TRY(bc_chase<T>(ws, ws.B, ws.d, ws.e));
     CUEV_HIP(hipEventRecord(ev[2], s));
+    CUEV_TRY(turn.end());
     // (d, e) to the host
     CUEV_HIP(hipMemcpyAsync(ctx.h_d, ws.d, sizeof(T) * n, hipMemcpyDeviceToHost, s));
     CUEV_HIP(hipMemcpyAsync(ctx.h_e, ws.e, sizeof(T) * n, hipMemcpyDeviceToHost, s));
@@ -246,10 +249,13 @@ int solve_values(Context<T> &ctx, T *A, int il, int iu, T *eval, cuev_solve_time
     hipEvent_t *ev = ctx.ev;
     const auto wall0 = clk::now();
     CUEV_HIP(hipEventRecord(ev[0], s));
+    PersistentTurn turn;
+    CUEV_TRY(turn.begin(s, n, ws.b));
     CUEV_TRY(dbbr_reduce<T>(ws, A, ws.B));
     CUEV_HIP(hipEventRecord(ev[1], s));
     CUEV_TRY(bc_chase<T>(ws, ws.B, ws.d, ws.e));
     CUEV_HIP(hipEventRecord(ev[2], s));
+    CUEV_TRY(turn.end());
     {
         prof::Scope sc(s, "tv.multisect");
         CUEV_TRY(tridi_values<T>(s, ws.d, ws.e, n, il, iu, eval));
