@@ -897,6 +897,16 @@ __global__ void bc_extract_kernel(const T *Bp, T *d, T *e, int n, int b) {
     if (i == n - 1) e[i] = T(0);
 }
 
+// the tridiagonal matrix (d, e) as a packed band: what the windowed form leaves in Bp
+template <typename T>
+__global__ __launch_bounds__(256) void bc_band_kernel(T *Bp, const T *d, const T *e, int n, int b) {
+    const i64 ldb = 2 * b, idx = (i64)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= ldb * n) return;
+    const i64 j = idx / ldb;
+    const int r = (int)(idx - j * ldb);
+    Bp[idx] = r == 0 ? d[j] : (r == 1 && j < n - 1) ? e[j] : T(0);
+}
+
 template <typename T> size_t bc_lds_bytes(int b) {
     const size_t nseg = std::max<size_t>(1, kBCThreads / (3 * (size_t)b));
     return sizeof(T) * ((size_t)2 * b * (2 * b + 1) + 2 * b + 3 * b + nseg * 3 * b);
@@ -1013,7 +1023,7 @@ template <typename T, int B> int launch_chase(Workspace<T> &ws, T *Bp) {
     return CUEV_STATUS_SUCCESS;
 }
 
-template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e) {
+template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e, bool write_band) {
     const int n = ws.n;
     hipStream_t s = ws.stream;
     if (n - 2 > 0) {
@@ -1024,7 +1034,14 @@ template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e) {
         case 64: CUEV_TRY((try_chase_resident<T, 64>(ws, Bp, d, e, &done))); break;
         default: CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "bc_chase: unsupported b=%d", ws.b);
         }
-        if (done) return CUEV_STATUS_SUCCESS;
+        if (done) {
+            if (write_band) {
+                hipLaunchKernelGGL(bc_band_kernel<T>, dim3((unsigned)ceil_div((i64)2 * ws.b * n, 256)), dim3(256), 0, s,
+                                   Bp, d, e, n, ws.b);
+                CUEV_LAUNCH_CHECK();
+            }
+            return CUEV_STATUS_SUCCESS;
+        }
         switch (ws.b) {
         case 16: CUEV_TRY((launch_chase<T, 16>(ws, Bp))); break;
         case 32: CUEV_TRY((launch_chase<T, 32>(ws, Bp))); break;
@@ -1038,7 +1055,7 @@ template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e) {
     return CUEV_STATUS_SUCCESS;
 }
 
-template int bc_chase<float>(Workspace<float> &, float *, float *, float *);
-template int bc_chase<double>(Workspace<double> &, double *, double *, double *);
+template int bc_chase<float>(Workspace<float> &, float *, float *, float *, bool);
+template int bc_chase<double>(Workspace<double> &, double *, double *, double *, bool);
 
 } // namespace cuev

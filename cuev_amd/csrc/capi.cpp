@@ -220,7 +220,7 @@ template <typename T> int stage_chase(cuev_handle_t h, T *B, T *d, T *e) {
     detail::clear_error();
     CUEV_CTX(T, h);
     if (!B || !d || !e) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "bc_chase: null pointer");
-    CUEV_TRY(bc_chase<T>(ctx->ws, B, d, e));
+    CUEV_TRY(bc_chase<T>(ctx->ws, B, d, e, true));
     return workspace_check_error(ctx->ws);
 }
 template <typename T> int stage_dc(cuev_handle_t h, T *d, T *e, T *eval, T *evec) {

@@ -257,7 +257,8 @@ int cuev_d_dbbr_panel_qr(cuev_handle_t h, double *A, double *Y, int rows, int b)
    the handle's Y and W; the band is packed into B. */
 int cuev_s_dbbr_reduce(cuev_handle_t h, float *A, float *B);
 int cuev_d_dbbr_reduce(cuev_handle_t h, double *A, double *B);
-/* Band -> tridiagonal. B is overwritten; reflectors go to the handle's U. */
+/* Band -> tridiagonal. B is overwritten by the tridiagonal matrix, packed as the band was (d in
+   row 0, e in row 1, zeros below); reflectors go to the handle's U. */
 int cuev_s_bc_chase(cuev_handle_t h, float *B, float *d, float *e);
 int cuev_d_bc_chase(cuev_handle_t h, double *B, double *d, double *e);
 /* Divide and conquer on device d, e; writes eval (ascending) and the
