@@ -15,8 +15,9 @@ int resolve_blocking(int n, int &b, int &k) {
     // b = 64 halves the band reduction's panels, which are latency-bound, for a sweep lag of
     // the chase of 3.9 instead of 3.2 us. Solves in ms, b = 32 / 64, FP64 (FP32): n = 200
     // 2.5 / 2.5 (2.3 / 2.5), 256 3.0 / 2.8 (2.7 / 2.6), 512 6.1 / 5.3 (5.4 / 4.8), 1024
-    // 15.0 / 11.4 (12.6 / 10.2), 3001 51.7 / 40.9 (45.9 / 37.6).
-    if (b == 0) b = (n >= 256) ? 64 : 32;
+    // 15.0 / 11.4 (12.6 / 10.2), 3001 51.7 / 40.9 (45.9 / 37.6). A caller's block size that only a
+    // bandwidth of 32 divides keeps 32 below 4096.
+    if (b == 0) b = (n >= 4096 || (n >= 256 && k % 64 == 0)) ? 64 : 32;
     if (b != 16 && b != 32 && b != 64)
         CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "bandwidth must be 16, 32 or 64 (got %d)", b);
     if (k == 0) k = 512;

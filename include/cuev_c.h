@@ -114,7 +114,8 @@ typedef enum cuev_dc_mode_t {
 } cuev_dc_mode_t;
 
 typedef struct cuev_options {
-    int bandwidth;       /* b in {16, 32, 64}; 0 selects the default (64 for n >= 256, else 32) */
+    int bandwidth;       /* b in {16, 32, 64}; 0 selects the default: 64 for n >= 256, else 32 (and 32
+                            for n < 4096 if block is set and is no multiple of 64) */
     int block;           /* k, a multiple of b; 0 selects 512 (clamped to n) */
     int precision;       /* cuev_precision_t */
     int refine_sweeps;   /* mixed form: maximum sweeps; 0 selects 3 */
