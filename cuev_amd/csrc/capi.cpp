@@ -90,7 +90,8 @@ int solve_entry(T *A, int n, T *eval, T *evec, hipStream_t s, cuev_solve_timer *
     }
     if (o.precision != CUEV_PRECISION_NATIVE)
         CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "symm_eig_solve: bad precision %d", o.precision);
-    if (n <= kSmallMaxN && !o.bandwidth && !o.block && o.bt_mode == CUEV_BT_AUTO && o.dc_mode == CUEV_DC_AUTO) {
+    if (n <= kSmallMaxN && !o.bandwidth && !o.block && o.bt_mode == CUEV_BT_AUTO && o.dc_mode == CUEV_DC_AUTO &&
+        !o.dc_leaf) {
         bool done = false;
         CUEV_TRY(small_entry<T>(A, n, eval, evec, 0, n - 1, s, timer, &done));
         if (done) return CUEV_STATUS_SUCCESS;
