@@ -44,7 +44,8 @@ template <> Context<double> *ctx_of<double>(cuev_handle_t h) {
 // the staged pipeline's launches and hand-offs (n = 48 and 128 in FP64: 0.50 and 1.67 ms staged,
 // 0.16 and 0.54 in one kernel). An option that names a stage keeps the pipeline, and so do
 // orders above 32 whose eigenvalues are too close for the kernel's fast path (*done = false,
-// A untouched): its QL takes 0.85 ms at n = 48 and 5.2 at 128.
+// A untouched): its QL takes 0.85 ms at n = 48 and 5.2 at 128. Only a matrix too large or too small in
+// scale for the pipeline has its QL here, so that the accepted range does not depend on the gaps.
 template <typename T>
 int small_entry(const T *A, int n, T *eval, T *evec, int il, int iu, hipStream_t s, cuev_solve_timer *timer,
                 bool *done) {

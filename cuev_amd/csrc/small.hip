@@ -50,6 +50,10 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 template <typename T> struct Gap;
 template <> struct Gap<double> { static constexpr double once = 1e-7, min = 1e-10; };
 template <> struct Gap<float> { static constexpr double once = 1e-10, min = 1e-11; }; // of 6e-8
+// Largest exponent, either way, of a matrix that may be left to the staged pipeline, which is not scaled: it
+// squares entries in FP64 (2^300: sums to 2^614; 2^-300: entries below 2^-510 are lost, 2^-210 of
+// the largest) and works in T (FP32 with 26 binary digits of room at either end).
+template <typename T> constexpr int kStagedExp = sizeof(T) == 8 ? 300 : 100;
 
 // LDS in doubles: the n x n region (A, then Z, then the reflectors), then vectors
 struct SmallLds {
@@ -498,7 +502,7 @@ __device__ __forceinline__ void small_eig_body(const T *Ag, const T *Eg, int n, 
             close |= (gap < Gap<T>::once * tnorm ? 1 : 0) | (gap < Gap<T>::min * tnorm ? 2 : 0);
         }
     const bool twice = __syncthreads_or(close & 1), ql = __syncthreads_or(close & 2);
-    if (ql && !allow_ql) {
+    if (ql && !allow_ql && ts >= -kStagedExp<T> && ts <= kStagedExp<T>) {
         fail(2);
         return;
     }

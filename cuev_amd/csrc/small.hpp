@@ -11,7 +11,8 @@ constexpr int kSmallMaxN = 128;
 // the eigenvectors to V; with V == nullptr: eigenvalues il..iu to W (batch x (iu - il + 1)).
 // Blocking. *n_failed: matrices whose QL iteration did not converge; *n_not_finite: matrices
 // with a NaN or infinite entry (their outputs are NaN). n_need_ql: nullptr, or the matrices
-// with eigenvalues too close for the fast path are left unsolved and counted there.
+// with eigenvalues too close for the fast path are left unsolved and counted there, unless their
+// scale is too large or too small for the staged pipeline (kStagedExp in small.hip).
 template <typename T>
 int small_eig(hipStream_t s, const T *A, int n, int batch, T *W, T *V, int il, int iu, int *n_failed,
               int *n_not_finite, int *n_need_ql = nullptr);
