@@ -239,14 +239,15 @@ __global__ __launch_bounds__(64 * bt_waves(TR)) void bc_back_kernel(const T *__r
     const int lane = threadIdx.x & 63, q = lane >> 4, li = lane & 15;
     const int wcol = blockIdx.x * (16 * NCT);
 
-    // tile rows [r0, r0 + 16) of the workgroup's columns in accumulator layout
+    // tile rows [r0, r0 + 16) of the workgroup's columns in accumulator layout; row 0, which no
+    // reflector covers, is not one of M's here: the all-zero block would spread a NaN in it
     auto load_tile = [&](int r0, V4(&v)[NCT]) {
 #pragma unroll
         for (int c = 0; c < NCT; ++c)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = r0 + MB::kidx(r, q), col = wcol + 16 * c + li;
-                const bool ok = row >= 0 && row < n && col < ncols;
+                const bool ok = row > 0 && row < n && col < ncols;
                 v[c][r] = *(ok ? M + row + (i64)col * ldm : zp);
             }
     };
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(64 * bt_waves(TR)) void bc_back_kernel(const T *__r
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = r0 + MB::kidx(r, q), col = wcol + 16 * c + li;
-                if (row >= 0 && row < n && col < ncols) M[row + (i64)col * ldm] = v[c][r];
+                if (row > 0 && row < n && col < ncols) M[row + (i64)col * ldm] = v[c][r];
             }
     };
 
