@@ -952,15 +952,14 @@ int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, int hops, s
 }
 
 // Resident form when its workgroups, one per hop of the first sweep, all fit on the GPU at
-// once (each waits for both neighbours); *done tells whether it was launched. The form with
-// a receiving wave is taken where two such chases fit at once (b = 64 in FP64: n <= 16384;
-// two solves may share the GPU, as with the windowed form), the one without it, which has
-// more room, where one does (n <= 49152; at n = 16384 3.9 us per sweep, windowed 16.4).
-// A chase of at most a quarter of the CUs' number of hops (b = 64: n <= 4096) takes its CUs for itself:
-// four such chases, as many as a process has hardware queues by default, still fit at once. Whole
-// solves: FP64 n = 1024 7.14 -> 7.00 ms, 2500 19.65 -> 19.19, 4096 36.3 -> 34.8 (the chase 14.7 ->
-// 13.3), FP32 4096 29.7 -> 28.8. Up to half of them n = 8192 would gain as well (127.5 -> 120.2), but
-// only two chases would fit.
+// once (each waits for both neighbours); *done tells whether it was launched. The caller holds
+// a CU per workgroup, or the whole GPU (residency.hpp), so other solves need no room here. The form
+// with a receiving wave is taken up to half of what the GPU holds of it (b = 64 in FP64: n <= 16384),
+// the one without it, which has more room, up to all it holds (n <= 49152; at n = 16384 3.9 us
+// per sweep, windowed 16.4). Between n = 16384 and 32768 a chase with it would fit, but has not been measured.
+// A chase of at most a quarter of the CUs' number of hops (b = 64: n <= 4096) takes its CUs for itself.
+// Whole solves: FP64 n = 1024 7.14 -> 7.00 ms, 2500 19.65 -> 19.19, 4096 36.3 -> 34.8 (the chase 14.7 ->
+// 13.3), FP32 4096 29.7 -> 28.8. Above, n = 8192 alone has been measured (127.5 -> 120.2).
 template <typename T, int B> int try_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, bool *done) {
     const int hops = (ws.n - 2) / B + 1;
     i64 with = 0, without = 0;

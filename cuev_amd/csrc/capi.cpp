@@ -208,6 +208,8 @@ template <typename T> int stage_panel_qr(cuev_handle_t h, T *A, T *Y, int rows, 
     if (!A || rows < 1 || b < 1 || b > 64)
         CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "dbbr_panel_qr: rows=%d b=%d", rows, b);
     if (rows > ctx->ws.n) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "dbbr_panel_qr: rows > handle n");
+    CuClaim cus;
+    CUEV_TRY(cus.take(ctx->ws.stream, rows, 64));
     CUEV_TRY(dbbr_panel_qr<T>(ctx->ws, A, Y, nullptr, rows, b));
     return workspace_check_error(ctx->ws);
 }
@@ -215,6 +217,8 @@ template <typename T> int stage_reduce(cuev_handle_t h, T *A, T *B) {
     detail::clear_error();
     CUEV_CTX(T, h);
     if (!A || !B) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "dbbr_reduce: null pointer");
+    CuClaim cus;
+    CUEV_TRY(cus.take(ctx->ws.stream, ctx->ws.n, ctx->ws.b));
     CUEV_TRY(dbbr_reduce<T>(ctx->ws, A, B));
     return workspace_check_error(ctx->ws);
 }
@@ -222,6 +226,8 @@ template <typename T> int stage_chase(cuev_handle_t h, T *B, T *d, T *e) {
     detail::clear_error();
     CUEV_CTX(T, h);
     if (!B || !d || !e) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "bc_chase: null pointer");
+    CuClaim cus;
+    CUEV_TRY(cus.take(ctx->ws.stream, ctx->ws.n, ctx->ws.b));
     CUEV_TRY(bc_chase<T>(ctx->ws, B, d, e, true));
     return workspace_check_error(ctx->ws);
 }

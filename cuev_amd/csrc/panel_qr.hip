@@ -709,9 +709,10 @@ template <int B> __device__ __forceinline__ cq_v4 cq_upper_mm(const double *X, c
     return acc;
 }
 
-// Up to 64 rows per workgroup four waves per SIMD (112 VGPRs): a panel's workgroup then fits on a CU beside one of a
-// bulge chase of another solve. Both kinds wait for workgroups of their own to become resident, so
-// where they excluded each other, four solves of n = 8192 at once could block one another.
+// Up to 64 rows per workgroup four waves per SIMD (112 VGPRs, as fast as 174): the registers leave room for
+// another kernel's waves on the CU, in LDS a panel of 64 columns (141 KB) for an unpadded bulge
+// chase of another solve, not for a padded one or another panel. That every workgroup gets a CU
+// does not depend on it (residency.hpp).
 template <typename T, int B, int NSET>
 __global__ __launch_bounds__(kCQThreads, NSET == 2 ? 4 : 2) void panel_cholqr_kernel(CQArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];

@@ -591,8 +591,8 @@ int run_mixed(Context<float> &cf, MixedBuffers &mb, double *A, int n, double *ev
     hipStream_t bs = cf.bt_stream;
     CUEV_HIP(hipEventRecord(ev[0], s));
     CUEV_TRY((convert2d<double, float>(s, A, n, ws.M, ws.ld, n, n)));
-    PersistentTurn turn;
-    CUEV_TRY(turn.begin(s, n, ws.b));
+    CuClaim cus;
+    CUEV_TRY(cus.take(s, n, ws.b));
     CUEV_TRY(dbbr_reduce<float>(ws, ws.M, ws.B));
     CUEV_HIP(hipEventRecord(ev[1], s));
     // 2. M = Q_b^T Q_s^T in FP32 on the back-transform stream: Q_s^T beside the
@@ -602,7 +602,6 @@ int run_mixed(Context<float> &cf, MixedBuffers &mb, double *A, int n, double *ev
     CUEV_TRY(sbr_back_t<float>(ws, bs, ws.Y, ws.W, ws.M, ws.ld));
     CUEV_HIP(hipEventRecord(cf.xev[1], bs));
     CUEV_TRY(bc_chase<float>(ws, ws.B, ws.d, ws.e));
-    CUEV_TRY(turn.end());
     CUEV_HIP(hipEventRecord(ev[2], s));
     CUEV_HIP(hipMemcpyAsync(cf.h_d, ws.d, 4 * (size_t)n, hipMemcpyDeviceToHost, s));
     CUEV_HIP(hipMemcpyAsync(cf.h_e, ws.e, 4 * (size_t)n, hipMemcpyDeviceToHost, s));
@@ -612,6 +611,7 @@ int run_mixed(Context<float> &cf, MixedBuffers &mb, double *A, int n, double *ev
     CUEV_TRY(bc_back_t<float>(ws, bs, ws.U, ws.M, ws.ld));
     CUEV_HIP(hipEventRecord(cf.xev[3], bs));
     CUEV_HIP(hipEventSynchronize(ev[3]));
+    cus.give(); // (the Rayleigh-Ritz steps solve on their own account)
     for (int i = 0; i < n; ++i) {
         mb.h_d[i] = cf.h_d[i];
         mb.h_e[i] = (i < n - 1) ? cf.h_e[i] : 0.0;

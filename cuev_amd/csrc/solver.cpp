@@ -135,13 +135,12 @@ int solve_native(Context<T> &ctx, T *A, T *eval, T *evec, cuev_solve_timer *time
     if (reordered) CUEV_TRY(bt_ensure(ctx));
     hipStream_t bs = ctx.bt_stream;
     CUEV_HIP(hipEventRecord(ev[0], s));
-    PersistentTurn turn;
-    CUEV_TRY(turn.begin(s, n, ws.b));
+    CuClaim cus;
+    CUEV_TRY(cus.take(s, n, ws.b));
     CUEV_TRY(dbbr_reduce<T>(ws, A, ws.B));
     CUEV_HIP(hipEventRecord(ev[1], s));
     CUEV_TRY(bc_chase<T>(ws, ws.B, ws.d, ws.e));
     CUEV_HIP(hipEventRecord(ev[2], s));
-    CUEV_TRY(turn.end());
     // (d, e) to the host
     CUEV_HIP(hipMemcpyAsync(ctx.h_d, ws.d, sizeof(T) * n, hipMemcpyDeviceToHost, s));
     CUEV_HIP(hipMemcpyAsync(ctx.h_e, ws.e, sizeof(T) * n, hipMemcpyDeviceToHost, s));
@@ -162,6 +161,7 @@ int solve_native(Context<T> &ctx, T *A, T *eval, T *evec, cuev_solve_timer *time
     // wait for (d, e) only; the reordered back-transform keeps running on the GPU.
     // The device error flag is checked once the stream has drained.
     CUEV_HIP(hipEventSynchronize(ev[3]));
+    cus.give();
     for (int i = 0; i < n; ++i)
         if (!std::isfinite((double)ctx.h_d[i]) || (i < n - 1 && !std::isfinite((double)ctx.h_e[i])))
             CUEV_FAIL(CUEV_STATUS_NOT_FINITE,
@@ -249,13 +249,12 @@ int solve_values(Context<T> &ctx, T *A, int il, int iu, T *eval, cuev_solve_time
     hipEvent_t *ev = ctx.ev;
     const auto wall0 = clk::now();
     CUEV_HIP(hipEventRecord(ev[0], s));
-    PersistentTurn turn;
-    CUEV_TRY(turn.begin(s, n, ws.b));
+    CuClaim cus;
+    CUEV_TRY(cus.take(s, n, ws.b));
     CUEV_TRY(dbbr_reduce<T>(ws, A, ws.B));
     CUEV_HIP(hipEventRecord(ev[1], s));
     CUEV_TRY(bc_chase<T>(ws, ws.B, ws.d, ws.e));
     CUEV_HIP(hipEventRecord(ev[2], s));
-    CUEV_TRY(turn.end());
     {
         prof::Scope sc(s, "tv.multisect");
         CUEV_TRY(tridi_values<T>(s, ws.d, ws.e, n, il, iu, eval));
@@ -266,6 +265,7 @@ int solve_values(Context<T> &ctx, T *A, int il, int iu, T *eval, cuev_solve_time
     CUEV_HIP(hipMemcpyAsync(ctx.h_d, ws.d, sizeof(T) * n, hipMemcpyDeviceToHost, s));
     CUEV_HIP(hipMemcpyAsync(ctx.h_e, ws.e, sizeof(T) * n, hipMemcpyDeviceToHost, s));
     CUEV_HIP(hipStreamSynchronize(s));
+    cus.give();
     CUEV_TRY(workspace_check_error(ws));
     for (int i = 0; i < n; ++i)
         if (!std::isfinite((double)ctx.h_d[i]) || (i < n - 1 && !std::isfinite((double)ctx.h_e[i])))

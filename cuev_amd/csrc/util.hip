@@ -1,11 +1,11 @@
 // util.hip — error bookkeeping, device queries and small element-wise kernels.
 #include "util.hpp"
 
-#include <algorithm>
-
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
+
+#include "residency.hpp"
 
 namespace cuev {
 
@@ -168,35 +168,30 @@ template int convert2d<float, double>(hipStream_t, const float *, i64, double *,
 template int convert2d<double, float>(hipStream_t, const double *, i64, float *, i64, i64, i64);
 
 namespace {
-constexpr int kMaxTurnDevices = 64;
-struct Turn {
-    std::mutex mu;
-    hipEvent_t ev = nullptr; // end of the last turn
-};
-Turn g_turn[kMaxTurnDevices];
+constexpr int kMaxDevices = 64;
+CuBudget g_cus[kMaxDevices];
 } // namespace
 
-int PersistentTurn::begin(hipStream_t s, int n, int b) {
-    // workgroups of the panel QR (64 rows each) and of the chase (one per hop of b rows)
-    if (4 * ceil_div(n, std::min(b, 64)) <= device_cu_count()) return CUEV_STATUS_SUCCESS;
+int CuClaim::take(hipStream_t s, i64 n, int b) {
     int dev = 0;
     CUEV_HIP(hipGetDevice(&dev));
-    if (dev < 0 || dev >= kMaxTurnDevices) return CUEV_STATUS_SUCCESS;
-    Turn &t = g_turn[dev];
-    lock_ = std::unique_lock<std::mutex>(t.mu);
-    if (t.ev) CUEV_HIP(hipStreamWaitEvent(s, t.ev, 0));
-    else CUEV_HIP(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+    shares_ = dev >= 0 && dev < kMaxDevices ? cu_shares(n, b, device_cu_count()) : 0;
+    if (shares_ == 0) return CUEV_STATUS_SUCCESS;
+    g_cus[dev].take(shares_);
     dev_ = dev;
     s_ = s;
     return CUEV_STATUS_SUCCESS;
 }
 
-int PersistentTurn::end() {
-    if (dev_ < 0) return CUEV_STATUS_SUCCESS;
-    CUEV_HIP(hipEventRecord(g_turn[dev_].ev, s_));
+void CuClaim::give() {
+    if (dev_ >= 0) g_cus[dev_].give(shares_);
     dev_ = -1;
-    lock_.unlock();
-    return CUEV_STATUS_SUCCESS;
+}
+
+CuClaim::~CuClaim() {
+    if (dev_ < 0) return;
+    (void)hipStreamSynchronize(s_);
+    give();
 }
 
 } // namespace cuev

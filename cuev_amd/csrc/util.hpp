@@ -41,20 +41,20 @@ int convert2d(hipStream_t s, const S *src, i64 lds, D *dst, i64 ldd, i64 m, i64 
 // p[0:n] = v
 int fill_int(hipStream_t s, int *p, i64 n, int v);
 
-// Solves whose band reduction and chase need more than a quarter of the CUs take turns on the GPU for
-// these two stages. Their kernels wait for workgroups of their own to become resident, one per CU:
-// four of up to a quarter each (as many as a process has hardware queues by default) always
-// fit at once, of larger ones each could get a part of the CUs and none all it waits for. begin() makes
-// the stream wait for the turn before (one event per device), end() ends the turn; other threads queue
-// their work once this one's is queued.
-class PersistentTurn {
+// A solve's hold on the CUs of the current device for its band reduction and chase (residency.hpp).
+// give() once they have finished on the GPU; left to the destructor (an error on the way), the
+// stream is waited for first. A thread holds at most one.
+class CuClaim {
   public:
-    int begin(hipStream_t s, int n, int b);
-    int end();
+    CuClaim() = default;
+    CuClaim(const CuClaim &) = delete;
+    CuClaim &operator=(const CuClaim &) = delete;
+    ~CuClaim();
+    int take(hipStream_t s, i64 n, int b);
+    void give();
 
   private:
-    std::unique_lock<std::mutex> lock_;
-    int dev_ = -1;
+    int dev_ = -1, shares_ = 0;
     hipStream_t s_ = nullptr;
 };
 
