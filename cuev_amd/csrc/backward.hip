@@ -29,6 +29,7 @@
 #include <mutex>
 
 #include "gemm.hpp"
+#include "idle_buffers.hpp"
 #include "util.hpp"
 
 namespace cuev {

@@ -9,6 +9,7 @@
 #include "context.hpp"
 #include "dbbr.hpp"
 #include "gemm.hpp"
+#include "idle_buffers.hpp"
 #include "lapack.hpp"
 #include "refine.hpp"
 #include "small.hpp"

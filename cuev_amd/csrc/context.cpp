@@ -2,6 +2,7 @@
 #include "context.hpp"
 
 #include "gemm.hpp"
+#include "idle_buffers.hpp"
 
 #include <cstdlib>
 #include <mutex>
@@ -67,11 +68,8 @@ template <typename T> int dc_ensure(Context<T> &ctx, bool need_q) {
         }
         const size_t sq = sizeof(T) * (size_t)n * n;
         const size_t bytes = (need_q ? 2 : 1) * ((sq + 255) & ~size_t(255));
-        if (hipMalloc(&ctx.dc_pool, bytes) != hipSuccess) {
-            ctx.dc_pool = nullptr;
-            (void)hipGetLastError();
+        if (device_alloc(&ctx.dc_pool, bytes) != hipSuccess)
             CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "dc: hipMalloc(%zu) for the D&C buffers failed", bytes);
-        }
         char *p = static_cast<char *>(ctx.dc_pool);
         ctx.dcQn = reinterpret_cast<T *>(p);
         if (need_q) ctx.dcQ = reinterpret_cast<T *>(p + ((sq + 255) & ~size_t(255)));

@@ -39,6 +39,7 @@
 #include <thread>
 #include <vector>
 
+#include "idle_buffers.hpp"
 #include "lapack.hpp"
 #include "profile.hpp"
 #include "small.hpp"
@@ -552,7 +553,7 @@ template <typename T> int dc_state_create(DcState<T> *&st, int n) {
     st->L = make_layout<T>(n);
     const size_t nn = (size_t)std::max(n, 1);
     size_t dev = st->L.total + sizeof(T) * nn * 6 + sizeof(int) * nn + 4096;
-    if (hipMalloc(&st->pool, dev) != hipSuccess) {
+    if (device_alloc(&st->pool, dev) != hipSuccess) {
         delete st;
         st = nullptr;
         CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "dc: hipMalloc(%zu) failed", dev);

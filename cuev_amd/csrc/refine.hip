@@ -54,6 +54,7 @@
 #include "dbbr.hpp"
 #include "dc.hpp"
 #include "gemm.hpp"
+#include "idle_buffers.hpp"
 #include "lapack.hpp"
 #include "profile.hpp"
 #include "solver.hpp"
@@ -340,8 +341,7 @@ int mixed_alloc(MixedBuffers *&out, int n) {
     const size_t nn = (size_t)n * n;
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     const size_t bytes = 3 * al(nn * 8) + al(n * 8) + al(3 * kRedBlocks * 8) + al(64) + 3 * al(n * 4);
-    if (hipMalloc(&m->pool, bytes) != hipSuccess) {
-        m->pool = nullptr;
+    if (device_alloc(&m->pool, bytes) != hipSuccess) {
         mixed_free(m);
         CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "mixed: hipMalloc(%zu) failed", bytes);
     }

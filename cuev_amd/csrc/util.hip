@@ -37,64 +37,6 @@ int device_cu_count() {
     return cache[dev];
 }
 
-int IdleBuffers::take(Buffer &b, size_t bytes) {
-    int dev = 0;
-    CUEV_HIP(hipGetDevice(&dev));
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        Buffer &slot = idle_[dev & 63];
-        if (slot.p && slot.device == dev && slot.bytes >= bytes) {
-            b = slot;
-            slot = Buffer{};
-            return CUEV_STATUS_SUCCESS;
-        }
-    }
-    b.device = dev;
-    b.bytes = bytes;
-    if (hipMalloc(&b.p, bytes) != hipSuccess) {
-        b.p = nullptr;
-        (void)hipGetLastError();
-        CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "device allocation of %zu bytes failed", bytes);
-    }
-    return CUEV_STATUS_SUCCESS;
-}
-
-void IdleBuffers::give(Buffer &b) {
-    Buffer victim;
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        Buffer &slot = idle_[b.device & 63];
-        if (slot.p && slot.bytes >= b.bytes) {
-            victim = b;
-        } else {
-            victim = slot;
-            slot = b;
-        }
-    }
-    b = Buffer{};
-    if (victim.p) (void)hipFree(victim.p);
-}
-
-void IdleBuffers::release_all() {
-    Buffer victims[64];
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        for (int i = 0; i < 64; ++i) {
-            victims[i] = idle_[i];
-            idle_[i] = Buffer{};
-        }
-    }
-    int cur = 0;
-    (void)hipGetDevice(&cur);
-    for (Buffer &v : victims)
-        if (v.p) {
-            (void)hipSetDevice(v.device);
-            (void)hipDeviceSynchronize();
-            (void)hipFree(v.p);
-        }
-    (void)hipSetDevice(cur);
-}
-
 namespace {
 
 template <typename T>

@@ -1,30 +1,9 @@
 // util.hpp — small element-wise kernels and error bookkeeping.
 #pragma once
 
-#include <mutex>
-
 #include "common.hpp"
 
 namespace cuev {
-
-// One idle device buffer per GPU, kept between blocking calls: take() hands it out if it is
-// large enough and free, else allocates; give() (after the call's work has finished) keeps the
-// larger of the two. Calls that overlap each have a buffer of their own.
-class IdleBuffers {
-  public:
-    struct Buffer {
-        void *p = nullptr;
-        size_t bytes = 0;
-        int device = -1;
-    };
-    int take(Buffer &b, size_t bytes); // on the current device
-    void give(Buffer &b);
-    void release_all();
-
-  private:
-    std::mutex mu_;
-    Buffer idle_[64];
-};
 
 namespace detail {
 const char *last_error();

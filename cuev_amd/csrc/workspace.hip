@@ -5,6 +5,7 @@
 
 #include "bulge.hpp"
 #include "gemm.hpp"
+#include "idle_buffers.hpp"
 #include "panel_qr.hpp"
 #include "util.hpp"
 
@@ -100,9 +101,8 @@ template <typename T> int workspace_alloc(Workspace<T> &ws, int n, int b, int k,
     off += al((bt_off.size() + 1) * sizeof(i64));
     ws.pool_bytes = off;
 
-    hipError_t e = hipMalloc(&ws.pool, ws.pool_bytes);
+    const hipError_t e = device_alloc(&ws.pool, ws.pool_bytes);
     if (e != hipSuccess) {
-        ws.pool = nullptr;
         CUEV_FAIL(CUEV_STATUS_ALLOC_FAILED, "workspace: hipMalloc(%zu bytes) failed: %s",
                   ws.pool_bytes, hipGetErrorString(e));
     }
