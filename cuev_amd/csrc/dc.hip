@@ -605,10 +605,6 @@ int dc_solve(DcState<T> &st, hipStream_t s, int n, const T *d, const T *e, T *Q,
     if (ldq < n) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "dc: ldq < n");
     if (leaf <= 0) leaf = 64;
     leaf = std::max(leaf, 2);
-    const LapackFns *lp = lapack();
-    if (!lp || (sizeof(T) == 8 ? !lp->dsteqr : !lp->ssteqr))
-        CUEV_FAIL(CUEV_STATUS_LAPACK_UNAVAILABLE, "dc: host ?steqr not found");
-
     // scale
     T orgnrm = 0;
     for (int i = 0; i < n; ++i) orgnrm = std::max(orgnrm, (T)std::fabs(d[i]));
@@ -659,6 +655,9 @@ int dc_solve(DcState<T> &st, hipStream_t s, int n, const T *d, const T *e, T *Q,
         }
     } else {
         // ---- larger leaves, asked for by the caller: on the host, in parallel
+        const LapackFns *lp = lapack();
+        if (!lp || (sizeof(T) == 8 ? !lp->dsteqr : !lp->ssteqr))
+            CUEV_FAIL(CUEV_STATUS_LAPACK_UNAVAILABLE, "dc: host ?steqr not found");
         LeafDesc *lv = reinterpret_cast<LeafDesc *>(up + L.leaves);
         int *leaf_of = reinterpret_cast<int *>(up + L.leaf_of);
         i64 soff = 0;
