@@ -117,6 +117,7 @@ def _declare(L):
     L.cuev_handle_destroy.argtypes = [P]
     L.cuev_handle_buffer.argtypes = [P, I, ctypes.POINTER(P), ctypes.POINTER(I64)]
     L.cuev_handle_set_dc.argtypes = [P, I, I]
+    L.cuev_handle_set_chase.argtypes = [P, I]
 
 
 def _check(st):
@@ -353,6 +354,10 @@ class Handle:
         d, _ = self.buffer("D")
         e, _ = self.buffer("E")
         _check(self._f("bc_chase")(self.h, ctypes.c_void_p(B), ctypes.c_void_p(d), ctypes.c_void_p(e)))
+
+    def set_chase(self, windowed=False):
+        """Bulge chase by the windowed form (which large orders take) at any order."""
+        _check(lib().cuev_handle_set_chase(self.h, int(windowed)))
 
     def set_dc(self, mode="host", leaf=0):
         """Tridiagonal stage: host LAPACK ?stedc ("host") or the device-resident D&C."""

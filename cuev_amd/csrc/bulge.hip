@@ -11,7 +11,8 @@
 //
 // Two kernels: the resident form (bc_chase_resident_kernel, described there) wherever its
 // workgroups, one per hop of the first sweep, fit on the GPU at once, and the windowed
-// form below for the larger n (b = 64 in FP64: n > 49152), where it still is the only one.
+// form below for the larger n (b = 64 in FP64: n > 49152), where it still is the only one
+// (and, asked for by cuev_handle_set_chase, at any n).
 //
 // Design of the windowed form (not the reference's):
 //  * Reflector convention: if the vector below the pivot is exactly zero the
@@ -1027,7 +1028,8 @@ template <typename T> int bc_chase(Workspace<T> &ws, T *Bp, T *d, T *e, bool wri
     hipStream_t s = ws.stream;
     if (n - 2 > 0) {
         bool done = false;
-        switch (ws.b) {
+        switch (ws.chase_windowed ? 0 : ws.b) {
+        case 0: break;
         case 16: CUEV_TRY((try_chase_resident<T, 16>(ws, Bp, d, e, &done))); break;
         case 32: CUEV_TRY((try_chase_resident<T, 32>(ws, Bp, d, e, &done))); break;
         case 64: CUEV_TRY((try_chase_resident<T, 64>(ws, Bp, d, e, &done))); break;

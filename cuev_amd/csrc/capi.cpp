@@ -433,6 +433,16 @@ int cuev_handle_set_dc(cuev_handle_t h, int dc_mode, int dc_leaf) {
     return CUEV_STATUS_SUCCESS;
 }
 
+int cuev_handle_set_chase(cuev_handle_t h, int windowed) {
+    detail::clear_error();
+    if (!h) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "handle_set_chase: null handle");
+    if (windowed != 0 && windowed != 1)
+        CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "handle_set_chase: windowed must be 0 or 1 (got %d)", windowed);
+    if (h->f) h->f->ws.chase_windowed = windowed != 0;
+    if (h->d) h->d->ws.chase_windowed = windowed != 0;
+    return CUEV_STATUS_SUCCESS;
+}
+
 int cuev_handle_buffer(cuev_handle_t h, int which, void **ptr, int64_t *ld) {
     detail::clear_error();
     if (!h || !ptr) CUEV_FAIL(CUEV_STATUS_INVALID_ARGUMENT, "handle_buffer: null argument");

@@ -44,6 +44,7 @@ template <typename T> struct Workspace {
     unsigned *counter = nullptr; // panel-QR grid barrier counter
     int *prog = nullptr;         // bc_chase per-sweep progress (n ints)
     void *chmsg = nullptr;       // bc_chase messages between neighbouring workgroups
+    bool chase_windowed = false; // bc_chase by the windowed form also where the resident one fits
     int *err = nullptr;          // device error flag
     // bc_back block reflectors: sweeps grouped kBtGroup at a time; block (g, h) holds
     // the hop-h reflectors of sweeps [16g, 16g+16) as I - V T V^T, its operands packed

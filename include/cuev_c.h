@@ -262,6 +262,10 @@ int cuev_d_dbbr_reduce(cuev_handle_t h, double *A, double *B);
    row 0, e in row 1, zeros below); reflectors go to the handle's U. */
 int cuev_s_bc_chase(cuev_handle_t h, float *B, float *d, float *e);
 int cuev_d_bc_chase(cuev_handle_t h, double *B, double *d, double *e);
+/* The form of the handle's bulge chase (no reference counterpart): 0, the default, keeps the band in
+   the registers of one workgroup per hop where these all fit on the GPU (b = 64 in FP64: n <= 49152)
+   and windows of it in LDS above; 1 takes the windowed form at any n. Same results up to rounding. */
+int cuev_handle_set_chase(cuev_handle_t h, int windowed);
 /* Divide and conquer on device d, e; writes eval (ascending) and the
    tridiagonal eigenvectors Q_d into evec (ld n). Host LAPACK ?stedc by default;
    cuev_handle_set_dc selects the device-resident form. */
