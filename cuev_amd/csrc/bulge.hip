@@ -929,10 +929,23 @@ template <typename T, int B, bool RECV> int chase_capacity(i64 *out) {
     return CUEV_STATUS_SUCCESS;
 }
 
-// LDS that the chase asks for on top of its own where it is to have its CUs to itself: what is left
-// (under 20 KB) is less than any product's tile needs. The products that run beside the chase in the
-// reordered order otherwise share the chase's CUs and slow its chain of short steps down.
-constexpr size_t kChasePad = 136 * 1024;
+// LDS that the chase asks for on top of its own where it is to have its CUs to itself: what is left is
+// less than any product's tiles need (64 x 64 in FP32, 20 KB). The products that run beside the chase
+// in the reordered order otherwise share the chase's CUs and slow its chain of short steps down.
+constexpr size_t kCuLds = 160 * 1024, kSmallestTiles = 20 * 1024;
+template <typename T, int B> constexpr size_t chase_lds() { // the kernel's own
+    return sizeof(T) * (4 * B + 2 * (chase_compute(B) / B) * B + 2) + sizeof(int);
+}
+template <typename T, int B> constexpr size_t chase_pad() {
+    return std::max<size_t>(136 * 1024, kCuLds - kSmallestTiles - chase_lds<T, B>() / 256 * 256);
+}
+template <typename T, int B> constexpr bool chase_alone() {
+    const size_t all = chase_pad<T, B>() + chase_lds<T, B>();
+    return all <= kCuLds && all + kSmallestTiles > kCuLds;
+}
+static_assert(chase_alone<double, 16>() && chase_alone<double, 32>() && chase_alone<double, 64>() &&
+                  chase_alone<float, 16>() && chase_alone<float, 32>() && chase_alone<float, 64>(),
+              "no product beside a padded chase");
 
 template <typename T, int B, bool RECV>
 int launch_chase_resident(Workspace<T> &ws, const T *Bp, T *d, T *e, int hops, size_t pad = 0) {
@@ -968,7 +981,7 @@ template <typename T, int B> int try_chase_resident(Workspace<T> &ws, const T *B
     CUEV_TRY((chase_capacity<T, B, false>(&without)));
     *done = true;
     if (2 * hops <= with)
-        return launch_chase_resident<T, B, true>(ws, Bp, d, e, hops, 4 * hops <= device_cu_count() ? kChasePad : 0);
+        return launch_chase_resident<T, B, true>(ws, Bp, d, e, hops, 4 * hops <= device_cu_count() ? chase_pad<T, B>() : 0);
     if (hops <= without) return launch_chase_resident<T, B, false>(ws, Bp, d, e, hops);
     *done = false;
     return CUEV_STATUS_SUCCESS;
