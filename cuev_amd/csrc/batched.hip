@@ -271,20 +271,20 @@ int eig_batched(hipStream_t s, T *A, int n, int batch, T *W, T *V, int *n_not_co
     const int m = n + (n & 1), np = m / 2;
     const size_t params = (size_t)3 * np * 8 + 4 * 8 + (size_t)2 * np * 4;
     const size_t abytes = (size_t)m * m * sizeof(T);
-    const bool in_lds = abytes <= kLdsMatBytes;
+    // (FP64 matrices of these orders never fit: no such kernel)
+    static_assert((size_t)(kSmallMaxN + 2) * (kSmallMaxN + 2) * 8 > kLdsMatBytes, "the smallest order here");
+    const bool in_lds = sizeof(T) == 4 && abytes <= kLdsMatBytes;
+    const auto kernel = jacobi_batched_kernel<T, false>;
+    const auto lds_kernel = jacobi_batched_kernel<T, sizeof(T) == 4>;
     const size_t lds = (in_lds ? abytes : 0) + params + 16;
     int *dcount = nullptr;
     CUEV_HIP(hipMallocAsync(reinterpret_cast<void **>(&dcount), sizeof(int), s));
     CUEV_HIP(hipMemsetAsync(dcount, 0, sizeof(int), s));
-    if (in_lds && sizeof(T) == 4) { // FP64 matrices of these orders never fit
-        CUEV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(jacobi_batched_kernel<T, true>),
+    if (in_lds)
+        CUEV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(lds_kernel),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((jacobi_batched_kernel<T, true>), dim3((unsigned)batch), dim3(kJThreads), lds, s, A, n,
-                           W, V, dcount);
-    } else {
-        hipLaunchKernelGGL((jacobi_batched_kernel<T, false>), dim3((unsigned)batch), dim3(kJThreads), lds, s, A, n,
-                           W, V, dcount);
-    }
+    hipLaunchKernelGGL((in_lds ? lds_kernel : kernel), dim3((unsigned)batch), dim3(kJThreads), lds, s, A, n, W, V,
+                       dcount);
     const hipError_t le = hipGetLastError();
     int h = 0;
     const hipError_t ce = hipMemcpyAsync(&h, dcount, sizeof(int), hipMemcpyDeviceToHost, s);
