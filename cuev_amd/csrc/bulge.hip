@@ -699,7 +699,7 @@ __global__ __launch_bounds__(chase_threads(B, RECV)) void bc_chase_resident_kern
         for (long long it = 0;; ++it) {
             if (!ok) ok = MsgWord<T>::get(p + lane * NWD, v, tag);
             if (__all(ok)) return true;
-            if (it > kSpinLimit) {
+            if (it > kPollLimit) {
                 if (lane == 0)
                     __hip_atomic_store(err, (int)DEV_WATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return false;

@@ -55,9 +55,13 @@ int device_cu_count();
 enum DeviceError : int { DEV_OK = 0, DEV_WATCHDOG = 1 };
 
 // Bounded-spin budget of persistent kernels, in polls of an agent-scope atomic
-// load plus s_sleep(1) (roughly 0.5-2 us each): a few seconds in total. Healthy
-// waits (one panel column, two bulge hops) end within micro- to milliseconds.
+// load plus s_sleep(1) (roughly 0.5-2 us each): 2 to 8 seconds in total. Healthy
+// waits (one panel column, two bulge hops) end within micro- to milliseconds; waits for a grid's
+// last workgroups, beside another solve's products that keep refilling the CUs, with those products (a
+// merge of the divide and conquer at n = 49152 takes about a second).
 constexpr long long kSpinLimit = 4000000LL;
+// The same for polls without a sleep, one round trip of about 0.4 us each: 8 seconds.
+constexpr long long kPollLimit = 5 * kSpinLimit;
 
 // ---------------------------------------------------------------------------
 // Device helpers
