@@ -220,7 +220,7 @@ template <int... PH, typename F> __device__ __forceinline__ void bt_rotations(st
 // Bound: the MFMA pipe (8 NKB NCT products per step and wave: at b = 64 in FP64 2560 NCT cycles of
 // one SIMD) and, where there are fewer of column strips than CUs, their number.
 // Measured in FP64 at b = 64 (direct order, nothing beside it): n = 2500 1.5 ms, 4096 3.8, 8192 23,
-// 16384 175 (2 n^3 flops at 50 TF/s; the products' pipe is busy 80% of the time). With one wave per
+// 16384 172 (2 n^3 flops at 51 TF/s; the products' pipe is busy 85% of the time). With one wave per
 // 16 columns that walked every block, n = 2500 5.7 ms (on 157 of 1024 SIMDs), 4096 14.8, 8192 63,
 // 16384 242; with M's and the operands' loads issued together, one step ahead, 16384 258.
 template <typename T, int B, bool TR, int NCT>

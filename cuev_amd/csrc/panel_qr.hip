@@ -379,11 +379,13 @@ template <typename T> __global__ __launch_bounds__(kPQThreads) void panel_qr_ker
 // brings it up to date, eliminates its four columns by itself (pivots and multipliers by
 // lane reads) and passes them on through LDS, so there is one barrier for four columns;
 // what the columns further right still miss is made up beside the next group. The products
-// run on the FP64 matrix cores. Measured at b = 64: 150 -> 60 us per panel, of which
-// the first elimination 14, Q_1's 20, both Gram matrices 3.7 and their sums 8, the second pass 3.2
-// and W, Y and the top rows 8 (with a barrier for every column, 4 x 4 blocks per thread, vector
-// products and explicit inverses: elimination and P R_1^-1 41, Q_1 33, Gram 9, second pass 16,
-// W and Y 25); at b = 32 80 -> 28.
+// run on the FP64 matrix cores. Kernel time per panel at b = 64, averaged over a solve: 65 us at n = 333,
+// 66 at 2500, 67 at 4096, 81 at 16384 (62 for its last panels, 114 for the first, where the barriers and
+// sums over 255 workgroups add up); at b = 32 32 us at n = 1024. With a barrier for every column, 4 x 4
+// blocks per thread, vector products and explicit inverses it took 150 (b = 32: 80), and 202 for the first at
+// n = 16384. Of 60 us between stamps in the kernel, the first elimination takes 14, Q_1's 20, both Gram matrices
+// 3.7 and their sums 8, the second pass 3.2 and W, Y and the top rows 8 (before: elimination and
+// P R_1^-1 41, Q_1 33, Gram 9, second pass 16, W and Y 25).
 constexpr int kCQThreads = 512;
 constexpr int kCQWaves = kCQThreads / 64;
 constexpr int kCQMaxCH = 96;

@@ -5,11 +5,11 @@
 // the caller's stream and the call blocking until the results are in place.
 //
 // Two back-transform orders:
-//  * direct (the reference's, backtransform.cu:232-275): after the host D&C,
+//  * direct (the reference's, backtransform.cu:232-275): after the D&C,
 //    evec <- Q_s (Q_b Q_d) with bc_back then sbr_back on Q_d;
-//  * reordered (listed as future work in the reference README:35): while the
-//    host runs dstedc, the GPU builds X = Q_s Q_b (bc_back and sbr_back applied
-//    to the identity); after the D&C only one GEMM evec = X Q_d remains.
+//  * reordered (listed as future work in the reference README:35): X^T = Q_b^T Q_s^T is
+//    built on a second stream, Q_s^T beside the chase and Q_b^T beside the D&C;
+//    after the D&C only one GEMM evec = X Q_d remains.
 #include "solver.hpp"
 
 #include <algorithm>
@@ -52,13 +52,13 @@ float ev_ms(hipEvent_t a, hipEvent_t b) {
 }
 } // namespace
 
-// Smallest merge of the device D&C that waits for the back-transform running beside
-// it: the three top tree levels at n = 16384, which hold nearly all of the D&C's GEMM
-// work (measured there against other levels, no gate, and no overlap at all), and
-// every merge of more than 4096 rows at larger n, so the GEMM-heavy levels never share
-// the GPU with bc_back (merges of up to 4096 rows leave it at its own speed at
-// n = 16384). At n = 49152 one solve took 25.9 s with this gate and 27.8 s with the
-// top three levels only, but bc_back alone varies there from 7.6 to 12 s between runs.
+// Smallest merge of the device D&C that waits for the back-transform running beside it, in the
+// reordered order: the three top tree levels, which hold nearly all of the D&C's GEMM work, and from
+// n = 16384 on every merge of more than 4096 rows. The line is from the earlier back-transform kernel
+// and n = 16384 (which takes this order on request and in the mixed form). Where the automatic choice
+// takes it today, whole solves without a gate are 0.5 to 1.7% faster (FP64: n = 6000 71.4 ms against
+// 72.6, 8192 127.3 and 128.0, 10000 213.8 and 217.2); n / 2 lies in between, n / 8 and waiting for
+// all merges are slower.
 int kDcGateFrom(int n) { return std::min(n / 4, 4096); }
 
 // The reordered order hides Q_s^T behind the chase and Q_b^T behind the D&C, also where
@@ -147,8 +147,8 @@ int solve_native(Context<T> &ctx, T *A, T *eval, T *evec, cuev_solve_timer *time
     CUEV_HIP(hipEventRecord(ev[3], s));
     if (reordered) {
         // X^T = Q_b^T Q_s^T in M on the back-transform stream: Q_s^T needs only the
-        // band reduction and runs beside the bulge chasing (which occupies half the
-        // CUs, LDS-bound); Q_b^T follows the chasing and runs beside the D&C.
+        // band reduction and runs beside the bulge chasing (a workgroup per hop, up to n = 4096 on CUs
+        // of its own); Q_b^T follows the chasing and runs beside the D&C.
         CUEV_HIP(hipStreamWaitEvent(bs, ev[1], 0));
         CUEV_HIP(hipEventRecord(ctx.xev[0], bs));
         CUEV_TRY(sbr_back_t<T>(ws, bs, ws.Y, ws.W, ws.M, ws.ld));

@@ -73,7 +73,7 @@ const char *cuev_lapack_name(void);
 typedef struct cuev_solve_timer {
     float dbbr_ms;       /* full -> band (DBBR) */
     float bc_ms;         /* band -> tridiagonal (bulge chasing, incl. bc_pack) */
-    float dc_ms;         /* host tridiagonal divide and conquer (dstedc), wall time */
+    float dc_ms;         /* tridiagonal divide and conquer, wall time (eigenvalues only: counts) */
     float bt_ms;         /* back-transform work after the D&C returned */
     float total_ms;      /* whole-solve host wall clock */
     float bt_copyin_ms;  /* direct order: M <- Q_d upload; reordered order: Q_d upload */
@@ -82,7 +82,7 @@ typedef struct cuev_solve_timer {
     float bt_copyout_ms; /* reordered order: evec <- (Q_b^T Q_s^T)^T Q_d GEMM; direct: 0 */
     /* additions */
     float refine_ms;     /* mixed form: Ogita-Aishima refinement sweeps */
-    float overlap_ms;    /* GPU back-transform time hidden under the host D&C */
+    float overlap_ms;    /* reordered order: back-transform time beside the chase and the D&C */
     int refine_sweeps;   /* mixed form: sweeps performed */
     int n_cluster_cols;  /* mixed form: eigenvector columns treated as clustered */
     float refine_resid;  /* mixed form: last measured relative residual (FP64; an estimate
@@ -107,10 +107,10 @@ typedef enum cuev_bt_mode_t {
 
 typedef enum cuev_dc_mode_t {
     CUEV_DC_AUTO = 0,   /* device for n > 128, host otherwise */
-    CUEV_DC_HOST = 1,   /* host LAPACK ?stedc, Q_d uploaded (the reference's north-star form) */
+    CUEV_DC_HOST = 1,   /* host LAPACK ?stedc, Q_d uploaded */
     CUEV_DC_DEVICE = 2  /* divide and conquer with Q resident on the GPU: host deflation
-                           bookkeeping and leaves, device secular roots, vectors and GEMMs
-                           (the split of the reference's hybrid, src/cuda/tridi.cu:125-452) */
+                           bookkeeping, device leaves, secular roots, vectors and GEMMs (after the
+                           reference's hybrid, src/cuda/tridi.cu:125-452) */
 } cuev_dc_mode_t;
 
 typedef struct cuev_options {
@@ -121,7 +121,8 @@ typedef struct cuev_options {
     int refine_sweeps;   /* mixed form: maximum sweeps; 0 selects 3 */
     int bt_mode;         /* cuev_bt_mode_t */
     int dc_mode;         /* cuev_dc_mode_t */
-    int dc_leaf;         /* device D&C: largest leaf solved by host ?steqr; 0 selects 64 */
+    int dc_leaf;         /* device D&C: largest leaf, in rows; 0 selects 64. Leaves above 64 rows are
+                            solved by host LAPACK ?steqr */
     double refine_tol;   /* mixed form: stop once the FP64 relative residual
                             ||AV - V diag(lambda)||_F / (n ||A||_F) is below this; 0 selects 2e-14 */
 } cuev_options;
@@ -179,10 +180,11 @@ int cuev_dtridi_values(const double *d, const double *e, int n, int il, int iu, 
 /* Batched small eigenproblems (no reference counterpart: the reference      */
 /* solves one matrix per call, include/cuev.h:31-33). batch matrices of order */
 /* n <= 256, stored one after another (each n x n column-major, ld n; lower   */
-/* triangle read; A may be overwritten); eval receives batch x n eigenvalues      */
-/* (ascending per matrix), evec batch eigenvector matrices (columns). One      */
-/* workgroup per matrix: tridiagonalization up to n = 128, cyclic Jacobi above. Blocking. Returns NOT_CONVERGED if a   */
-/* matrix did not converge (count in *n_not_converged when not NULL).          */
+/* triangle read; A may be overwritten); eval receives batch x n eigenvalues  */
+/* (ascending per matrix), evec batch eigenvector matrices (columns). One     */
+/* workgroup per matrix: tridiagonalization up to n = 128, cyclic Jacobi      */
+/* above. Blocking. Returns NOT_CONVERGED if a matrix did not converge or has */
+/* a non-finite entry (count in *n_not_converged when not NULL).              */
 /* ------------------------------------------------------------------------ */
 int cuev_ssymm_eig_batched(float *A, int n, int batch, float *eval, float *evec, hipStream_t stream,
                            int *n_not_converged);
