@@ -77,6 +77,28 @@ def test_both_forms_agree(torch_dev, n, b, prec):
     assert np.abs(lam[0] - lam[1]).max() <= tol and np.array_equal(lam[0], lam[2])
 
 
+@pytest.mark.parametrize("n,b", [(9000, 16), (17000, 32), (17000, 64)])
+@pytest.mark.parametrize("prec", ["d", "s"])
+def test_resident_without_receiving_wave(torch_dev, n, b, prec):
+    """Orders above half of what the GPU holds of the chase with a receiving wave (256 CUs: n = 8192 at
+    b = 16, 16384 at b = 32 and 64 in FP64) take the form without it: eigenvalues against the windowed form."""
+    torch = torch_dev
+    dt = torch.float64 if prec == "d" else torch.float32
+    Bp = _band(n, b, prec, n)
+    lam = []
+    with cv.Handle(dt, n, b, b) as h:
+        for windowed in (False, True):
+            h.set_chase(windowed=windowed)
+            raw_put(h.buffer("B")[0], Bp, dt)
+            h.bc_chase()
+            torch.cuda.synchronize()
+            d, e = (raw_dev(h.buffer(x)[0], n, dt) for x in "DE")
+            lam.append(cv.tridi_values(torch.from_numpy(d).cuda(), torch.from_numpy(e).cuda()).cpu().numpy())
+    u = 2.0 ** -53 if prec == "d" else 2.0 ** -24
+    # each within n roundings of ||B||
+    assert np.abs(lam[0] - lam[1]).max() <= 2 * n * u * np.abs(lam[0]).max()
+
+
 def test_form_is_checked(torch_dev):
     """A null handle and another value than 0 or 1 are refused."""
     assert cv.lib().cuev_handle_set_chase(None, 1) == 1
