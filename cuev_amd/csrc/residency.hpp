@@ -9,7 +9,7 @@
 namespace cuev {
 
 // The panel QR and the bulge chase wait for workgroups of their own to become resident, and two of
-// their workgroups may not fit on one CU (144 KB of LDS for a panel of 64 columns, 146 KB for a padded
+// their workgroups may not fit on one CU (141 KB of LDS for a panel of 64 columns, 146 KB for a padded
 // chase, of 160). Kernels of several solves that each got a part of the CUs and wait for the rest would
 // block one another until their bounded waits expire. So a solve takes the CUs that its widest such
 // grid needs, one per workgroup, before it queues the band reduction, and gives them back after the
